@@ -57,6 +57,7 @@ struct DlBind {
 struct DlOut {
   int32_t rel[SRD_MAX_DESTS];    // step relation of each destination
   uint32_t n_dest, pipe, grain, direct;
+  uint32_t fixed_grain, pad_;    // slices of exactly `grain` items (set by the caller)
   uint64_t cap_slices, cap_new;
 };
 
@@ -137,7 +138,9 @@ SRD_HD inline void dl_plan_step(DevCtl* c, SrdDyn* d, const uint64_t* work_start
     return;
   }
   const uint64_t tw = work_start[d->n_root];
-  const uint64_t ns = (tw + o.grain - 1) / o.grain;
+  const uint32_t grain = o.fixed_grain ? o.grain : srd_grain(tw, o.grain);
+  const uint64_t ns = (tw + grain - 1) / grain;
+  d->grain = grain;
   d->total_work = tw;
   if (ns > o.cap_slices) {
     dl_raise(c, kOvfSlices, &c->need_slices, ns);

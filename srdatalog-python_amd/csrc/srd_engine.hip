@@ -238,7 +238,7 @@ struct Relation {
   // writes rows instead, turns the set bits into a NEW part; the bitmap is
   // kept (clear) for the next iteration.
   DevBuf<uint32_t> dense_bits;
-  DevBuf<uint32_t> dense_sum;  // a bit per block of the bitmap holding a set bit
+  DevBuf<uint32_t> dense_sum;  // a byte per block of the bitmap: holds a set bit
   uint64_t dense_words = 0;
   uint32_t dense_shift = 0;
   uint32_t dense_bound = 0;
@@ -933,6 +933,7 @@ static void pr_root(srd_engine& e, PipeRun& R) {
 static void pr_slices(srd_engine& e, PipeRun& R) {
   const SrdPipelineDesc* d = R.d;
   R.a.total_work = R.host[0];
+  if (!e.grain_override) R.a.grain = srd_grain(R.a.total_work, d->default_grain);
   R.a.n_slices = (R.a.total_work + R.a.grain - 1) / R.a.grain;
   const bool direct = d->direct_ok && !d->count_only && !e.two_pass && !e.no_direct;
   R.weigh_items = 0;
@@ -1339,7 +1340,7 @@ static void pr_dense(srd_engine& e, std::vector<PipeRun*>& runs) {
       if (R->d->mark && R->d->n_dest == 1 && rel_id(e, R->d->dest[0].rel) == kv.first) {
         R->dense = true;
         R->a.mark_bits = r.dense_bits.p;
-        R->a.mark_sum = r.dense_sum.p;
+        R->a.mark_sum = reinterpret_cast<uint8_t*>(r.dense_sum.p);
         R->a.mark_shift = r.dense_shift;
       }
   }
@@ -2030,6 +2031,7 @@ static void devloop_alloc(srd_engine& e, const Step& st, DevLoop& L, const DevCa
     P.out.n_dest = d->n_dest;
     P.out.pipe = uint32_t(pi);
     P.out.grain = P.a.grain;
+    P.out.fixed_grain = e.grain_override ? 1u : 0u;
     P.out.direct = P.direct ? 1u : 0u;
     P.out.cap_slices = L.cap_slices;
     P.out.cap_new = cn;

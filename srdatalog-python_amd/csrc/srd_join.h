@@ -71,6 +71,16 @@ __device__ __forceinline__ uint64_t next_slice(const SrdLaunchArgs& A, uint64_t 
   return n;
 }
 
+// Mark mode: note that the key's block of 2^18 keys holds a set bit.  A byte
+// per block, stored plainly: the bytes of a whole bitmap fill a few lines,
+// and a bit set with an atomic per newly marked key serialised every wave of
+// the launch on those lines (the load of 260,000 R-MAT pairs: 254 us with
+// 64 waves in flight and 1,744 us with 4,096; 70 us with stores).
+__device__ __forceinline__ void mark_block(const SrdLaunchArgs& A, uint64_t key) {
+  __hip_atomic_store(A.mark_sum + (key >> 18), uint8_t(1), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // Fused mode: open a staging segment of SRD_SEG rows for the wave (all lanes
 // take part; lane 0's bump is broadcast with v_readlane).  Returns ~0 when
 // staging is exhausted (the overflow flag is raised; the slice keeps

@@ -335,7 +335,7 @@ __device__ __forceinline__ void dense_load(const uint32_t* bits, uint64_t w0, ui
 }
 
 __device__ __forceinline__ bool dense_marked(const uint32_t* sum, uint32_t b) {
-  return (sum[b >> 5] >> (b & 31u)) & 1u;
+  return reinterpret_cast<const uint8_t*>(sum)[b] != 0;
 }
 
 __global__ __launch_bounds__(kBlock) void dense_count_kernel(const uint32_t* __restrict__ bits,

@@ -312,10 +312,10 @@ void exclusive_scan_u64(const uint64_t* in, uint64_t* out, uint64_t n, Workspace
 // Dense-bitmap NEW (the joins' mark mode): bit `key` of the bitmap holds
 // tuple (v_0 .. v_k-1) with key = sum(v_c << shift*(k-1-c)).  words must be
 // a multiple of kDenseBlockWords (the allocation is rounded up to it and the
-// tail stays clear); summary bit b (of words / kDenseBlockWords, in
-// dense_sum_words u32) is set when block b (2^18 keys) holds a set bit.
+// tail stays clear); summary byte b (of words / kDenseBlockWords, in
+// dense_sum_words u32) is 1 when block b (2^18 keys) holds a set bit.
 constexpr uint64_t kDenseBlockWords = 8192;
-inline uint64_t dense_sum_words(uint64_t words) { return (words / kDenseBlockWords + 31) / 32; }
+inline uint64_t dense_sum_words(uint64_t words) { return (words / kDenseBlockWords + 3) / 4; }
 // The tuples of the set bits, in key order (the index order: sorted and
 // duplicate-free), written to `out` (allocated here, column c at
 // out.p + c * stride, stride returned); only blocks marked in the summary

@@ -178,7 +178,7 @@ class PipelineGen:
     counts the searches only (probe runs), 6 sets the tuple's bit in the
     destination's dense bitmap (a plain load first: most derivations of a
     deduplicating join are repeats, whose bit is already set), and, for a
-    bit it sets, its block's bit in the summary the extraction reads."""
+    bit it sets, its block's byte in the summary the extraction reads."""
     lines = [f"{ind}{{",
              f"{ind}  const uint64_t m_ = srd::ballot({cond});",
              f"{ind}  const uint32_t c_ = __popcll(m_);",
@@ -240,9 +240,7 @@ class PipelineGen:
                 f"{ind}    const uint32_t b_ = 1u << uint32_t(key_ & 31u);",
                 f"{ind}    if (!(*w_ & b_)) {{",
                 f"{ind}      atomicOr(w_, b_);",
-                f"{ind}      uint32_t* s_ = A.mark_sum + (key_ >> 23);",
-                f"{ind}      const uint32_t sb_ = 1u << uint32_t((key_ >> 18) & 31u);",
-                f"{ind}      if (!(*s_ & sb_)) atomicOr(s_, sb_);",
+                f"{ind}      srdj::mark_block(A, key_);",
                 f"{ind}    }}",
                 f"{ind}  }}"]
     lines += [f"{ind}  opos += c_;",
@@ -633,7 +631,8 @@ class PipelineGen:
          "  const uint32_t drv_ = DYN ? A.dyn->drv_view : A.drv_view;",
          "  (void)drv_;",
          "  const uint64_t tw_ = DYN ? A.dyn->total_work : A.total_work;",
-         "  const uint64_t ns_ = DYN ? A.dyn->n_slices : A.n_slices;"]
+         "  const uint64_t ns_ = DYN ? A.dyn->n_slices : A.n_slices;",
+         "  const uint32_t gr_ = DYN ? A.dyn->grain : A.grain;"]
     for di in range(len(self.dests)):
       o.append(f"  const uint64_t ob{di}_ = DYN ? A.dyn->out_base[{di}] : A.out[{di}].base;")
     o += ["  const uint32_t lane = srd::lane_id();"]
@@ -687,9 +686,9 @@ class PipelineGen:
           "  for (;;) {",
           "    const uint64_t slice = srdj::next_slice(A, ns_);  // wave-uniform",
           "    if (slice >= ns_) break;",
-          "    const uint64_t it0 = A.slice_start ? A.slice_start[slice] : slice * A.grain;",
+          "    const uint64_t it0 = A.slice_start ? A.slice_start[slice] : slice * gr_;",
           "    const uint64_t it1 = A.slice_start ? A.slice_start[slice + 1]"
-          " : min(it0 + A.grain, tw_);",
+          " : min(it0 + gr_, tw_);",
           "    uint64_t opos = MODE == 1 ? A.offsets[slice] : 0;",
           "    uint32_t cnt = 0;",
           "    uint32_t seg_used = 0, seg_local = 0;",

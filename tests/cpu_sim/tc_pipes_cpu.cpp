@@ -152,6 +152,7 @@ void dyn_launch(const SrdLaunchArgs* a, hipStream_t s) {
   b.n_root = d.n_root;
   b.drv_view = d.drv_view;
   b.total_work = d.total_work;
+  b.grain = d.grain;
   b.n_slices = d.n_slices;
   for (int k = 0; k < SRD_MAX_DESTS; ++k) b.out[k].base = d.out_base[k];
   b.dyn = nullptr;
