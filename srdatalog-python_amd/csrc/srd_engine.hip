@@ -264,6 +264,7 @@ struct srd_engine {
   std::map<std::string, int> rel_by_name;
   std::vector<srd::Step> steps;
   std::map<std::string, const SrdPipelineDesc*> pipes;
+  std::map<std::string, const SrdPipelineExt*> exts;
   hipStream_t s = nullptr;
   srd::Workspace ws;
   std::string err;
@@ -320,6 +321,9 @@ struct srd_engine {
   // eighth of the device's memory.
   uint64_t dense_max_bits = uint64_t(1) << 36;
   uint64_t dense_bytes = 0;        // bitmaps allocated so far
+  // SRDATALOG_MARK_PRODUCTS=0: the mark mode sets the bits of a product one
+  // tuple at a time
+  bool mark_products = true;
   uint64_t mark_chunk_slices = 0;  // SRDATALOG_MARK_CHUNK_SLICES (0: one launch per traversal)
   uint32_t weigh_ranges = SRD_XCDS;  // SRDATALOG_WEIGH_RANGES: of the weigh launch
   // column-1 bitmaps of heavy keys for views nested levels search
@@ -965,6 +969,29 @@ static void pr_weighed(srd_engine& e, PipeRun& R) {
   // fewer than the uniform slicing had, never more than one per item
   // and at least e.min_slices_per_wave per wave, so that a mid-sized join
   // whose cost / weigh_target is below the wave count still spreads
+  if (R.dense && R.a.mark_prod == 2) {
+    // products priced in row steps, cut at equal costs wherever the cut
+    // falls: enough slices to even out the waves, none below a few steps
+    const uint64_t S = std::max<uint64_t>(
+        std::min<uint64_t>(std::max<uint64_t>(w / e.weigh_target, e.min_slices_per_wave * SRD_GRID_WAVES),
+                           w / 1024), 1);
+    x.slice_start.reserve(S + 1, R.s);
+    cost_items(x.item_pref.p, n, w, S, x.slice_start.p, R.s);
+    R.a.slice_start = x.slice_start.p;
+    R.a.item_pref = x.item_pref.p;
+    R.a.n_items = n;
+    R.a.cost_q = w / S;
+    R.a.cost_rem = w % S;
+    R.a.n_slices = S;
+    R.a.item_cost = nullptr;
+    R.a.n_ranges = e.xcd_ranges;
+    if (e.trace) {
+      std::fprintf(stderr, "[srd]   %s: %llu items, cost %llu cut into %llu slices\n", R.d->rule,
+                   (unsigned long long)n, (unsigned long long)w, (unsigned long long)S);
+      std::fflush(stderr);
+    }
+    return;
+  }
   const uint64_t cap = std::max<uint64_t>(R.a.n_slices, e.slices_per_wave * 4 * 2048);
   const uint64_t floor_s = e.min_slices_per_wave * 4 * 2048;
   uint64_t S = std::min<uint64_t>(
@@ -1342,6 +1369,11 @@ static void pr_dense(srd_engine& e, std::vector<PipeRun*>& runs) {
         R->a.mark_bits = r.dense_bits.p;
         R->a.mark_sum = reinterpret_cast<uint8_t*>(r.dense_sum.p);
         R->a.mark_shift = r.dense_shift;
+        // rows of whole 64-bit words (a probe run walks the same items in
+        // another mode, which counts tuples)
+        const auto x = e.exts.find(R->d->rule);
+        R->a.mark_prod = x != e.exts.end() && e.mark_products && !e.count_probes && r.dense_shift >= 6
+                             ? x->second->mark_prod : 0u;
       }
   }
 }
@@ -2929,6 +2961,11 @@ static int eguard(srd_engine* e, int code_on_error, F&& f) {
 extern "C" {
 
 srd_engine* srd_engine_create(const char* text, const SrdPipelineDesc* pipes, uint32_t n) {
+  return srd_engine_create_ext(text, pipes, n, nullptr, 0);
+}
+
+srd_engine* srd_engine_create_ext(const char* text, const SrdPipelineDesc* pipes, uint32_t n,
+                                  const SrdPipelineExt* exts, uint32_t n_exts) {
   auto* e = new srd_engine();
   try {
     pool_init(0);
@@ -2948,6 +2985,8 @@ srd_engine* srd_engine_create(const char* text, const SrdPipelineDesc* pipes, ui
       e->xcd_ranges = std::min<uint32_t>(std::max<uint32_t>(uint32_t(std::atoi(c)), 1), SRD_XCDS);
     if (const char* c = std::getenv("SRDATALOG_MARK_CHUNK_SLICES"))
       e->mark_chunk_slices = std::strtoull(c, nullptr, 10);
+    if (const char* c = std::getenv("SRDATALOG_MARK_PRODUCTS"))
+      e->mark_products = !(*c == '0' && c[1] == 0);
     if (const char* c = std::getenv("SRDATALOG_DENSE_MAX_BITS"))
       e->dense_max_bits = std::strtoull(c, nullptr, 10);
     if (const char* c = std::getenv("SRDATALOG_WINDOW_MIN"))
@@ -2990,6 +3029,7 @@ srd_engine* srd_engine_create(const char* text, const SrdPipelineDesc* pipes, ui
       e->no_direct = std::string(m) == "fused";
     }
     for (uint32_t i = 0; i < n; ++i) e->pipes[pipes[i].rule] = &pipes[i];
+    for (uint32_t i = 0; i < n_exts; ++i) e->exts[exts[i].rule] = &exts[i];
     parse_program(*e, text);
   } catch (const std::exception& ex) {
     std::cerr << "srdatalog_init: " << ex.what() << std::endl;

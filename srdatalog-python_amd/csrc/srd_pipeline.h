@@ -120,12 +120,28 @@ struct SrdLaunchArgs {
   uint32_t* mark_bits;
   uint8_t* mark_sum;
   uint32_t mark_shift;
-  uint32_t mark_pad_;
+  // rules whose last level is a product marked row by row (srdj::prod_mark):
+  // 1 = the root launch and the weigh mode price large products in row
+  // steps, and the mark mode walks them so
+  uint32_t mark_prod;
+  // weighed mark launches of such rules: slice s covers the cost range
+  // [srd_cost_cut(s), srd_cost_cut(s+1)) of the items' cost prefix (nullptr:
+  // whole items), slice_start[s] being the item that holds its first unit; a
+  // large product is split by rows where a cut falls inside it
+  const uint64_t* item_pref;
+  uint64_t n_items;
+  uint64_t cost_q, cost_rem;
   // device-sized launches (the *_dyn entry points) only: views, key and
   // slice counts and output bases are read from this device struct, which
   // kernels of the same iteration fill in, instead of the fields above
   const SrdDyn* dyn;
 };
+
+// Cost at which slice s of a launch of S slices over w cost units starts
+// (q = w / S, rem = w % S).
+__host__ __device__ inline uint64_t srd_cost_cut(uint64_t s, uint64_t q, uint64_t rem) {
+  return s * q + (s < rem ? s : rem);
+}
 
 // Device-resident part of a device-sized launch.  skip != 0 turns every
 // launch reading it into a no-op (an iteration after convergence, or one
@@ -150,6 +166,9 @@ struct SrdDyn {
 #define SRD_CTR_STRIDE 32u     // one 128-byte line per counter: atomics on one line serialise
 
 #define SRD_ITEM_COST 4u       // level-1 cost of an item, in level-2 candidates
+// A product is marked row by row when it has at least this many tuples and
+// its row steps, 64 lanes each, are no more than its tuples.
+#define SRD_PROD_MIN 256u
 // Two-source cartesian products at a nested last level with at least this
 // many tuples, and a source of at least SRD_CART_TILE_DIM rows, are walked in
 // register tiles (one 64-row tile per lane register, the other broadcast a
@@ -220,6 +239,15 @@ struct SrdPipelineDesc {
   SrdLaunchFn mark;
 };
 
+// What a rule's mark mode can do beyond marking tuple by tuple, by rule name.
+struct SrdPipelineExt {
+  const char* rule;
+  // large products of the rule's last level are walked row by row: 1 = the
+  // product is the level under the root (its keys are the items), 2 = the
+  // second level, whose items are weighed, 3 = a deeper one, 0 = no such level
+  uint32_t mark_prod;
+};
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -231,6 +259,10 @@ struct srd_engine;
 // reference's S-expression form.
 struct srd_engine* srd_engine_create(const char* program_text, const SrdPipelineDesc* pipelines,
                                      uint32_t n_pipelines);
+// The same with the rules' mark-mode extensions.
+struct srd_engine* srd_engine_create_ext(const char* program_text, const SrdPipelineDesc* pipelines,
+                                         uint32_t n_pipelines, const SrdPipelineExt* exts,
+                                         uint32_t n_exts);
 void srd_engine_destroy(struct srd_engine* e);
 const char* srd_engine_last_error(struct srd_engine* e);
 

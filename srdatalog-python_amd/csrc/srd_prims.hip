@@ -531,6 +531,31 @@ __global__ __launch_bounds__(kBlock) void slice_bounds_kernel(const uint64_t* __
   out[s] = lo;
 }
 
+// out[s] = the item that holds cost unit srd_cost_cut(s): the last i < n with
+// pref[i] <= cut (out[S] = n - 1, the last item).
+__global__ __launch_bounds__(kBlock) void cost_items_kernel(const uint64_t* __restrict__ pref,
+                                                            uint64_t n, uint64_t q, uint64_t rem,
+                                                            uint64_t S, uint64_t* __restrict__ out) {
+  const uint64_t s = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (s > S) return;
+  const uint64_t target = srd_cost_cut(s, q, rem);
+  uint64_t lo = 0, hi = n;  // answer in [lo, hi)
+  while (hi - lo > 1) {
+    const uint64_t mid = (lo + hi) >> 1;
+    if (pref[mid] <= target) lo = mid;
+    else hi = mid;
+  }
+  out[s] = lo;
+}
+
+void cost_items(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
+                hipStream_t s) {
+  if (S == 0 || n == 0) fail("cost_items: no slices");
+  cost_items_kernel<<<uint32_t((S + 1 + kBlock - 1) / kBlock), kBlock, 0, s>>>(pref, n, w / S, w % S,
+                                                                             S, out);
+  SRD_CHECK(hipGetLastError());
+}
+
 void slice_bounds(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
                   hipStream_t s) {
   if (S == 0) fail("slice_bounds: no slices");

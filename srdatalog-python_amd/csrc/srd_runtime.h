@@ -377,6 +377,12 @@ void build_root_pos(const Index& x, uint64_t max_entries, hipStream_t s);
 void slice_bounds(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
                   hipStream_t s);
 
+// Cost-cut slices: out[s] (s = 0..S) = the item holding the cost unit at which
+// slice s starts (srd_cost_cut over w units; pref as for slice_bounds), the
+// last item for s = S.
+void cost_items(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
+                hipStream_t s);
+
 // Synthetic columns (k fields of one 64-bit key per row, low k-1 fields
 // fbits wide): key = mul*i + off when range == 0 (ascending, distinct for
 // mul > 0), else a hash of i+off reduced mod range.

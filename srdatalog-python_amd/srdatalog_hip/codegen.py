@@ -248,6 +248,38 @@ class PipelineGen:
               f"{ind}}}"]
     return "\n".join(lines)
 
+  def prod_level(self, lv) -> dict | None:
+    """How the mark mode walks the product of last level `lv` row by row
+    (srdj::prod_mark), or None: two sources of one variable each, no check
+    left to apply, and a destination index whose last column is one of the
+    two variables (`m`, from source `jm`) and one other column the other one
+    (`r`, from `jr`, at index column `cr`); the remaining columns are
+    bound."""
+    if not self.mark_ok() or not isinstance(lv, M.CartesianJoin) or lv is not self.levels[-1]:
+      return None
+    if isinstance(self.root, M.Scan):
+      return None
+    if len(lv.sources) != 2 or not all(len(vs) == 1 for vs in lv.var_from_source or ()):
+      return None
+    cart = [vs[0] for vs in lv.var_from_source]
+    for f in self.filters:
+      if any(v in cart for v in (f.prefix if isinstance(f, M.Negation) else f.vars)):
+        return None
+    d = self.dests[0]
+    row = [d.terms[c] for c in d.index]
+    if cart[0] == cart[1] or row[-1] not in cart or any(row.count(v) != 1 for v in cart):
+      return None
+    jm = cart.index(row[-1])
+    return {"jm": jm, "jr": 1 - jm, "cr": row.index(cart[1 - jm]),
+            "bound": [(c, v) for c, v in enumerate(row) if v not in cart], "k": len(row)}
+
+  def prod_base(self, p: dict, get) -> str:
+    """Bit of the product's tuple with zero row and last column: the bound
+    variables at their index columns."""
+    parts = [f"(uint64_t({get(self.var(v))}) << (A.mark_shift * {p['k'] - 1 - c}u))"
+             for c, v in p["bound"]]
+    return " + ".join(parts) or "uint64_t(0)"
+
   def mark_ok(self) -> bool:
     """Mode 6 applies: one destination whose terms are all variables (every
     value then comes from a source column, so the engine can bound the key
@@ -394,6 +426,15 @@ class PipelineGen:
         body.append("    work = 1;")
         for r in rngs:
           body.append(f"    work *= uint64_t({self.size_expr(r, True)});")
+        p = self.prod_level(lv)
+        if p:
+          # mark launches: a large product counts as its row steps
+          rm, rr = rngs[p["jm"]], rngs[p["jr"]]
+          body += ["    if (A.mark_prod && work >= SRD_PROD_MIN) {",
+                   f"      const uint64_t st = 64u * srdj::prod_steps({self.col_expr(rm.view, rm.depth)}, "
+                   f"{rm.b}, {rm.e}, {rr.e} - {rr.b});",
+                   "      if (st <= work) { work = st; drv = 1; }",
+                   "    }"]
     out += body
     out.append("  }")
     # probe runs: root_find of every slot but the driver's, and the range
@@ -636,13 +677,16 @@ class PipelineGen:
     for di in range(len(self.dests)):
       o.append(f"  const uint64_t ob{di}_ = DYN ? A.dyn->out_base[{di}] : A.out[{di}].base;")
     o += ["  const uint32_t lane = srd::lane_id();"]
+    # the product the mark mode walks row by row, at the level under the root
+    prod0 = (self.prod_level(self.levels[0])
+             if self.levels else None)
     # levels walked by the wave from LDS frames: every level below the
     # first (the first is one item per lane), or, under a scan root (whose
     # rows are the items), every level
     scan_root = isinstance(self.root, M.Scan)
     deep = len(self.levels) >= 2 or (scan_root and len(self.levels) >= 1)
     self._lds = []
-    if deep or self.ring:
+    if deep or self.ring or prod0:
       o += ["  const uint32_t wv = threadIdx.x / 64u;"]
     lds_at = len(o)
     ring_cols = sum(len(d.index) for d in self.dests)
@@ -677,6 +721,19 @@ class PipelineGen:
             "  };"]
     slots = self.root_slots()
     ns = len(slots)
+    if any(self.prod_level(lv) for lv in self.levels[-1:]):
+      o += ["  // mark mode: the (word, mask) pairs of the product being walked",
+            "  uint32_t* lw_ = nullptr;",
+            "  uint64_t* lm_ = nullptr;",
+            "  if constexpr (MODE == 6) {",
+            "    __shared__ uint32_t prod_w[4][128];",
+            "    __shared__ uint64_t prod_m[4][128];",
+            "    lw_ = prod_w[wv];",
+            "    lm_ = prod_m[wv];",
+            "    lm_[lane] = lm_[64 + lane] = 0;",
+            "    __builtin_amdgcn_wave_barrier();",
+            "    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, \"wavefront\");",
+            "  }"]
     o += ["  // fused mode: the wave's open staging segment, kept across slices (a",
           "  // slice's rows in it are one record; the next slice goes on behind them)",
           "  uint32_t probes_ = 0;  // MODE 5: searches, map lookups and bitmap tests of this lane",
@@ -687,18 +744,28 @@ class PipelineGen:
           "    const uint64_t slice = srdj::next_slice(A, ns_);  // wave-uniform",
           "    if (slice >= ns_) break;",
           "    const uint64_t it0 = A.slice_start ? A.slice_start[slice] : slice * gr_;",
-          "    const uint64_t it1 = A.slice_start ? A.slice_start[slice + 1]"
+          "    uint64_t it1 = A.slice_start ? A.slice_start[slice + 1]"
           " : min(it0 + gr_, tw_);",
+          *(["    // cost-cut launches: the slice's cost range, and its last item, which the",
+             "    // next slice shares",
+             "    uint64_t c0_ = 0, c1_ = ~uint64_t(0);",
+             "    if (MODE == 6 && A.item_pref) {",
+             "      c0_ = srd_cost_cut(slice, A.cost_q, A.cost_rem);",
+             "      c1_ = srd_cost_cut(slice + 1, A.cost_q, A.cost_rem);",
+             "      it1 = min(it1 + 1, A.n_items);",
+             "    }"] if len(self.levels) == 2 and self.prod_level(self.levels[-1]) else []),
           "    uint64_t opos = MODE == 1 ? A.offsets[slice] : 0;",
           "    uint32_t cnt = 0;",
           "    uint32_t seg_used = 0, seg_local = 0;",
           "    uint32_t kc = ~0u;  // key of the previous batch's last item",
-          "    for (uint64_t base = it0; base < it1; base += 64) {",
+          "    uint64_t step_ = 64;",
+          "    for (uint64_t base = it0; base < it1; base += step_) {",
           "      const uint64_t item = base + lane;",
-          "      const bool act = item < it1;",
+          f"      {'' if prod0 else 'const '}bool act = item < it1;",
           "      const uint64_t last_item = min(base + 63, it1 - 1);",
           "      const uint32_t klo = kc == ~0u ? srdj::find_slot(A.work_start, nroot_, base)",
           "                                     : srdj::find_slot_from(A.work_start, kc, nroot_, base);",
+          *(self.gen_prod_root(prod0, slots) if prod0 else []),
           "      const uint32_t khi = srdj::find_slot_from(A.work_start, klo, nroot_, last_item) + 1;",
           "      kc = khi - 1;",
           "      uint32_t k = klo;",
@@ -708,6 +775,14 @@ class PipelineGen:
           " if (A.work_start[mid] <= item) lo = mid; else hi = mid; }",
           "        k = lo;",
           "      }",
+          *(["      if (MODE == 6 && A.mark_prod) {  // a large product ends the batch before it",
+             "        const uint64_t bg_ = srd::ballot(act && A.key_aux[k] != 0);",
+             "        if (bg_) {",
+             "          step_ = uint64_t(__builtin_ctzll(bg_));",
+             "          act = act && lane < step_;",
+             "          kc = klo;",
+             "        }",
+             "      }"] if prod0 else []),
           "      const uint64_t li = act ? item - A.work_start[k] : 0;"]
     ind = "      "
     bound: set[str] = set()
@@ -791,6 +866,35 @@ class PipelineGen:
     o[lds_at:lds_at] = self._lds
     return "\n".join(o)
 
+  def gen_prod_root(self, p: dict, slots: list) -> list[str]:
+    """Mark mode, product under the root: a key whose product is large
+    (key_aux set by the root kernel) is walked row by row, the slice's part
+    of its cost giving its part of the rows."""
+    lv = self.levels[0]
+    ns = len(slots)
+    at = {}
+    for j in (p["jm"], p["jr"]):
+      s_ = lv.sources[j]
+      at[j] = (slots.index((self.vid(s_), tuple(s_.prefix))), self.col_expr(self.vid(s_), len(s_.prefix)))
+    (sm, cm), (sr, cr) = at[p["jm"]], at[p["jr"]]
+    return ["      if (MODE == 6 && A.mark_prod) {",
+            "        step_ = 64;",
+            "        if (A.key_aux[klo]) {",
+            "          const uint64_t ks_ = A.work_start[klo], kw_ = A.work_start[klo + 1] - ks_;",
+            "          const uint64_t hi_ = min(it1, ks_ + kw_);",
+            f"          const uint32_t* kr_ = A.key_rng + uint64_t(klo) * {2 * ns};",
+            f"          const uint32_t {self.var(self.root.var)} = V.v[drv_].root_vals[klo];",
+            f"          (void){self.var(self.root.var)};",
+            f"          const uint32_t rb_ = kr_[{2 * sr}], nr_ = kr_[{2 * sr + 1}] - rb_;",
+            f"          srdj::prod_mark(A, {self.prod_base(p, lambda v: v)}, "
+            f"A.mark_shift * {p['k'] - 1 - p['cr']}u, {cm}, kr_[{2 * sm}], kr_[{2 * sm + 1}], {cr}, "
+            "rb_ + srdj::prod_cut(nr_, base - ks_, kw_), rb_ + srdj::prod_cut(nr_, hi_ - ks_, kw_), lw_, lm_);",
+            "          kc = klo;",
+            "          step_ = hi_ - base;",
+            "          continue;",
+            "        }",
+            "      }"]
+
   def needed_after(self, li: int) -> set[str]:
     """Variables read from level li on: source prefixes, checks, heads."""
     need: set[str] = set()
@@ -861,11 +965,27 @@ class PipelineGen:
     if (isinstance(lv, M.ColumnJoin) and len(rngs) > 1 and not self.coop_search
         and not any(r.full0 for r in rngs)):
       self.gen_window(rngs, per_lane, frame, t, hvar, o, ind)
+    p = self.prod_level(lv) if li >= 1 else None
+    if p:
+      rm, rr = rngs[p["jm"]], rngs[p["jr"]]
+      mb, me = (rm.b, rm.e) if not rm.full0 else ("0u", f"V.v[{rm.view}].n")
+      rb, re_ = (rr.b, rr.e) if not rr.full0 else ("0u", f"V.v[{rr.view}].n")
+      o.append(f"{ind}uint64_t pc{t} = 0;  // cost of the item's product walked row by row (0: it is not)")
+      o.append(f"{ind}if constexpr (MODE == 4 || MODE == 6) {{")
+      o.append(f"{ind}  if (A.mark_prod && {hvar} && sz{t} >= SRD_PROD_MIN) {{")
+      o.append(f"{ind}    pc{t} = 64u * srdj::prod_steps({self.col_expr(rm.view, rm.depth)}, {mb}, {me}, "
+               f"{re_} - {rb});")
+      o.append(f"{ind}    if (pc{t} > sz{t}) pc{t} = 0;")
+      o.append(f"{ind}  }}")
+      o.append(f"{ind}}}")
     if li == 1:
+      cost = f"(pc{t} ? pc{t} : sz{t})" if p else f"sz{t}"
       o.append(f"{ind}if constexpr (MODE == 4) {{  // weigh: the item's level-2 candidates")
-      o.append(f"{ind}  if (act) A.item_cost[item] = sz{t} + SRD_ITEM_COST;")
+      o.append(f"{ind}  if (act) A.item_cost[item] = {cost} + SRD_ITEM_COST;")
       o.append(f"{ind}  continue;")
       o.append(f"{ind}}}")
+    if p:
+      o += self.gen_prod_nested(p, t, rm, mb, me, rr, rb, re_, li, hvar, ind)
     tiled = (self.cart_tiles and isinstance(lv, M.CartesianJoin) and li == len(self.levels) - 1
              and len(rngs) == 2 and all(len(vs) == 1 for vs in lv.var_from_source))
     if tiled:
@@ -873,7 +993,8 @@ class PipelineGen:
       # below (its weigh cost above still counts it)
       sizes = [self.size_expr(r, True) for r in rngs]
       o.append(f"{ind}const bool big{t} = {hvar} && sz{t} >= SRD_CART_TILE_MIN && "
-               f"max(uint32_t({sizes[0]}), uint32_t({sizes[1]})) >= SRD_CART_TILE_DIM;")
+               f"max(uint32_t({sizes[0]}), uint32_t({sizes[1]})) >= SRD_CART_TILE_DIM"
+               + (" && !(MODE == 6 && A.mark_prod)" if p else "") + ";")
       o.append(f"{ind}if (big{t}) sz{t} = 0;")
     o += bm_code
     o.append(f"{ind}const uint64_t inc{t} = srd::wave_incl_scan<uint64_t>(sz{t});")
@@ -954,6 +1075,37 @@ class PipelineGen:
     o.append(f"{ind}}}")
     if tiled:
       self.gen_cart_tiles(lv, li, rngs, per_lane, keep, done, o, ind)
+
+  def gen_prod_nested(self, p: dict, t: str, rm: Rg, mb: str, me: str, rr: Rg, rb: str, re_: str,
+                      li: int, hvar: str, ind: str) -> list[str]:
+    """Mark mode, product at a nested last level: the owners of large products
+    are walked one at a time, row by row; under a cost-cut launch the
+    slice takes its part of the item's rows, and of the other items those
+    that start inside its cost range."""
+    i1, i2 = ind + "  ", ind + "    "
+    rl = lambda v: f"__builtin_amdgcn_readlane({v}, ow_)"
+    code = [f"{ind}if constexpr (MODE == 6) {{",
+            f"{i1}uint32_t p0_ = 0, p1_ = pc{t} ? {re_} - {rb} : 0u;  // this slice's rows of the product"]
+    if len(self.levels) == 2:
+      code += [f"{i1}if (A.item_pref && {hvar}) {{",
+               f"{i2}const uint64_t s_ = A.item_pref[item], e_ = A.item_pref[item + 1];",
+               f"{i2}if (pc{t}) {{",
+               f"{i2}  if (c0_ > s_) p0_ = srdj::prod_cut({re_} - {rb}, min(c0_, e_) - s_, e_ - s_);",
+               f"{i2}  if (c1_ < e_) p1_ = srdj::prod_cut({re_} - {rb}, max(c1_, s_) - s_, e_ - s_);",
+               f"{i2}}} else if (s_ < c0_ || s_ >= c1_) {{",
+               f"{i2}  sz{t} = 0;",
+               f"{i2}}}",
+               f"{i1}}}"]
+    code += [f"{i1}if (pc{t}) sz{t} = 0;",
+             f"{i1}for (uint64_t bp_ = srd::ballot(p1_ > p0_); bp_; bp_ &= bp_ - 1) {{",
+             f"{i2}const uint32_t ow_ = uint32_t(__builtin_ctzll(bp_));",
+             f"{i2}const uint32_t rb_ = {rl(f'uint32_t({rb})')};",
+             f"{i2}srdj::prod_mark(A, {self.prod_base(p, rl)}, A.mark_shift * {p['k'] - 1 - p['cr']}u, "
+             f"{self.col_expr(rm.view, rm.depth)}, {rl(f'uint32_t({mb})')}, {rl(f'uint32_t({me})')}, "
+             f"{self.col_expr(rr.view, rr.depth)}, rb_ + {rl('p0_')}, rb_ + {rl('p1_')}, lw_, lm_);",
+             f"{i1}}}",
+             f"{ind}}}"]
+    return code
 
   def gen_window(self, rngs: list[Rg], per_lane: list, frame: list, t: str, hvar: str,
                  o: list[str], ind: str) -> None:
@@ -1109,6 +1261,16 @@ class PipelineGen:
            f"}}  // namespace {self.ns}", ""]
     return "\n".join(out)
 
+  def prod_kind(self) -> int:
+    """SrdPipelineExt.mark_prod: where the mark mode's row-by-row product is
+    (cost-cut launches need it at the second level, whose items are weighed)."""
+    if not self.levels or not self.prod_level(self.levels[-1]):
+      return 0
+    return min(len(self.levels), 3)
+
+  def gen_ext(self) -> str:
+    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}}}"
+
   def gen_desc(self) -> str:
     views = []
     bmv = self.bm_views()
@@ -1167,7 +1329,8 @@ SHIM = r"""
 static srd_engine* g_eng = nullptr;
 
 static bool ensure_engine() {
-  if (!g_eng) g_eng = srd_engine_create(k_program, k_pipes, sizeof(k_pipes) / sizeof(k_pipes[0]));
+  if (!g_eng) g_eng = srd_engine_create_ext(k_program, k_pipes, sizeof(k_pipes) / sizeof(k_pipes[0]),
+                                 k_exts, sizeof(k_exts) / sizeof(k_exts[0]));
   return g_eng && srd_engine_ok(g_eng);
 }
 
@@ -1272,7 +1435,8 @@ int srdatalog_export_instances(const char* rel_name, uint32_t* out, uint64_t cap
 // ---- engine handles: resumable runs for iteration-granular serving ----
 void* srdatalog_engine_new(void) {
   try {
-    srd_engine* e = srd_engine_create(k_program, k_pipes, sizeof(k_pipes) / sizeof(k_pipes[0]));
+    srd_engine* e = srd_engine_create_ext(k_program, k_pipes, sizeof(k_pipes) / sizeof(k_pipes[0]),
+                                 k_exts, sizeof(k_exts) / sizeof(k_exts[0]));
     if (e && !srd_engine_ok(e)) {
       srd_engine_destroy(e);
       return nullptr;
@@ -1370,6 +1534,9 @@ def generate_program_source(name: str, decls: list[RelDecl], prog: M.Program) ->
     out.append(g.gen_kernels())
   out.append("static const SrdPipelineDesc k_pipes[] = {")
   out.append(",\n".join(g.gen_desc() for g in gens) if gens else "")
+  out.append("};")
+  out.append("static const SrdPipelineExt k_exts[] = {")
+  out.append(",\n".join(g.gen_ext() for g in gens) if gens else "")
   out.append("};")
   out.append(f'static const char* k_program = R"SRDMIR({text})SRDMIR";')
   out.append(SHIM)

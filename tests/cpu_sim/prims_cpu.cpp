@@ -188,6 +188,15 @@ void export_rows(const Index& x, uint32_t* host_out, const uint32_t* bounds, uin
   }
 }
 
+void cost_items(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
+                hipStream_t) {
+  if (S == 0 || n == 0) fail("cost_items: no slices");
+  for (uint64_t s = 0; s <= S; ++s) {
+    const uint64_t t = srd_cost_cut(s, w / S, w % S);
+    out[s] = uint64_t(std::upper_bound(pref, pref + n, t) - pref) - 1;
+  }
+}
+
 void slice_bounds(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
                   hipStream_t) {
   const uint64_t q = w / S, rem = w % S;
