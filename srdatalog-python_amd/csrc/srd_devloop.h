@@ -210,6 +210,81 @@ SRD_HD inline void dl_iter_end_step(DevCtl* c, const DlEnd& e) {
   if (sum == 0) c->done = 1;
 }
 
+// ---------------------------------------------------- dense iterations ----
+// A step whose relations' key spaces fit bitmaps keeps FULL and NEW as
+// bitmaps in HBM and runs an iteration in six launches: the rules' root
+// launch, one scan-and-plan block, the mark traversal, then per relation a
+// count of NEW & ~FULL by block of 2^18 keys, one bookkeeping block that
+// scans the counts and decides, and the emission of DELTA (rows and root
+// arrays, in key order) that also ORs NEW into FULL and clears it.  Nothing
+// is sorted, subtracted or merged.  The column-0 values of a block are its
+// own: shift * (k - 1) <= 18 bits per column-0 value.
+struct DenseRel {
+  uint64_t* nw;          // NEW bitmap, FULL bitmap and their block bytes
+  uint64_t* fl;
+  uint8_t* nsum;
+  uint8_t* fsum;
+  uint64_t* blk;         // per block: NEW rows | column-0 values << kDenseRowBits, scanned in place
+                         // (no column-0 values counted for k == 1: every row is one)
+  uint32_t* delta;       // k columns of `stride` rows, root arrays
+  uint32_t* root_v;
+  uint32_t* root_o;
+  uint64_t* rec;         // |DELTA| of every iteration
+  uint64_t stride;
+  uint32_t nblocks, k, shift, pad_;
+};
+
+// What the host polls (pinned memory): `tick` counts the bookkeeping blocks
+// that ran an iteration or found an overflow.
+struct DenseSeen {
+  uint64_t tick, iter, need;
+  uint32_t done, overflow;
+};
+
+struct DenseCtl {
+  uint32_t skip, emit, done, overflow;
+  uint64_t iter, max_iter, iter_cap, tick;
+  uint64_t full_n[kDevRels], delta_n[kDevRels], delta_r[kDevRels];
+  uint64_t keys[kDevPipes];
+};
+
+struct DensePipe {
+  DlBind bind;
+  SrdDyn* dyn;
+};
+
+struct DenseBook {
+  DenseCtl* ctl;
+  DenseSeen* seen;
+  DenseRel rel[kDevRels];
+  DensePipe pipe[kDevPipes];
+  uint32_t nrels, npipes;
+};
+
+constexpr uint32_t kDenseRowBits = 40;
+constexpr uint64_t kDenseRowMask = (uint64_t(1) << kDenseRowBits) - 1;
+constexpr uint64_t kDensePlanKeys = 65536;  // most keys the one-block scan takes
+
+// FULL bitmap := the rows of an index (bits and block bytes set).
+void dense_set_rows(const uint32_t* cols, uint64_t stride, uint64_t n, uint32_t k, uint32_t shift,
+                    uint64_t* bits, uint8_t* sum, hipStream_t s);
+// Scan of a pipeline's per-key work, its total, grain and slice count, and
+// its slice counters cleared.
+void dense_plan(DenseCtl* c, SrdDyn* d, uint32_t pipe, const uint64_t* key_work, uint64_t* work_start,
+                uint64_t cap_keys, uint64_t* scan_tmp, uint32_t* work_ctr, uint32_t grain,
+                bool fixed_grain, hipStream_t s);
+void dense_count(const DenseCtl* c, const DenseRel& r, hipStream_t s);
+void dense_book(const DenseBook& b, hipStream_t s);
+void dense_emit(const DenseCtl* c, const DenseRel& r, hipStream_t s);
+// Row c->iter - 1 of out: the instances' DELTA rows of the iteration just emitted.
+void dense_inst(const DenseCtl* c, uint32_t rel, const uint32_t* col0, const uint32_t* bounds,
+                uint32_t n_inst, uint64_t* out, hipStream_t s);
+// Index of a bitmap's set bits, counted first (the packed total in
+// blk[nblocks]), then written (r.delta, r.root_v, r.root_o): r.nw and r.nsum
+// are the bits and block bytes, r.fl is null; nothing is cleared.
+void dense_index_count(const DenseRel& r, hipStream_t s);
+void dense_index_emit(const DenseRel& r, hipStream_t s);
+
 // Enqueue the steps (one thread each) on stream s.
 void dl_iter_begin(DevCtl* c, uint32_t nrels, hipStream_t s);
 void dl_bind(DevCtl* c, SrdDyn* d, const DlBind& b, hipStream_t s);

@@ -128,6 +128,9 @@ struct SrdLaunchArgs {
   // [srd_cost_cut(s), srd_cost_cut(s+1)) of the items' cost prefix (nullptr:
   // whole items), slice_start[s] being the item that holds its first unit; a
   // large product is split by rows where a cut falls inside it
+  // device-sized mark launches: tuples derived, summed into SRD_ROW_CTRS
+  // counters SRD_ROW_CTR_STRIDE words apart (nullptr: not counted)
+  unsigned long long* mark_rows;
   const uint64_t* item_pref;
   uint64_t n_items;
   uint64_t cost_q, cost_rem;
@@ -164,6 +167,9 @@ struct SrdDyn {
 // slices of the other ranges once their own is done.
 #define SRD_XCDS 8u
 #define SRD_CTR_STRIDE 32u     // one 128-byte line per counter: atomics on one line serialise
+
+#define SRD_ROW_CTRS 64u
+#define SRD_ROW_CTR_STRIDE 16u // u64 words: a 128-byte line per counter
 
 #define SRD_ITEM_COST 4u       // level-1 cost of an item, in level-2 candidates
 // A product is marked row by row when it has at least this many tuples and
@@ -246,6 +252,7 @@ struct SrdPipelineExt {
   // product is the level under the root (its keys are the items), 2 = the
   // second level, whose items are weighed, 3 = a deeper one, 0 = no such level
   uint32_t mark_prod;
+  SrdLaunchFn mark_dyn;   // device-sized mark mode; nullptr outside recursive steps
 };
 
 #ifdef __cplusplus

@@ -3099,4 +3099,399 @@ void dl_inst(const DevCtl* c, uint32_t r, const uint32_t* col0, const uint32_t* 
   SRD_CHECK(hipGetLastError());
 }
 
+
+// ================================================== dense iterations ====
+// A block of 2^18 keys is 4096 words of 64 keys: 64 chunks of one word per
+// lane, four chunks for each of a workgroup's 16 waves.  A word's keys go out
+// one per lane, and the rows of a word are one coalesced store per column.
+constexpr int kDenseWg = 1024;
+constexpr int kDenseWgWaves = kDenseWg / kWave;
+constexpr int kDenseChunks = 64;
+constexpr int kDenseWaveChunks = kDenseChunks / kDenseWgWaves;
+static_assert(kDenseBlockWords == 2ull * kDenseChunks * kWave, "64 chunks of 64 words of 64 keys");
+
+struct DenseScan {
+  uint64_t x[kDenseWaveChunks];     // this lane's words of NEW & ~FULL
+  uint64_t first[kDenseWaveChunks]; // words that open a column-0 value, by chunk
+  uint32_t cnt, roots;              // of the whole block
+  uint32_t cbase[kDenseWaveChunks], rbase[kDenseWaveChunks];  // before each chunk, in the block
+};
+
+// The block's new words, which of them hold the first rows of a column-0
+// value, and the rows and values before each of the wave's chunks.  s_*: LDS
+// of the workgroup.  rs = bits of a column-0 value's keys (k == 1: 0).
+__device__ __forceinline__ void dense_scan_block(const uint64_t* nw, const uint64_t* fl, uint64_t b,
+                                                 uint32_t rs, uint32_t* s_cnt, uint32_t* s_root,
+                                                 DenseScan& d) {
+  const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  const uint64_t w0 = b * (kDenseBlockWords / 2);
+  uint32_t pc[kDenseWaveChunks];
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave + l;
+    uint64_t x = nw[at];
+    if (fl) x &= ~fl[at];
+    d.x[i] = x;
+    pc[i] = wave_sum<uint32_t>(__popcll(x));
+    if (l == 0) s_cnt[w * kDenseWaveChunks + i] = pc[i];
+  }
+  __syncthreads();
+  const uint32_t mine = s_cnt[l];  // lane l: rows of chunk l
+  const uint64_t chunks = ballot(mine != 0);
+  const uint32_t cincl = wave_incl_scan<uint32_t>(mine);
+  uint32_t rc[kDenseWaveChunks];
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint32_t ch = w * kDenseWaveChunks + i;
+    const uint64_t nz = ballot(d.x[i] != 0);
+    if (rs == 0) {
+      d.first[i] = nz;
+      rc[i] = pc[i];
+    } else {
+      // words of the lane's column-0 value before it: in the chunk, and, for
+      // values wider than a chunk, in the chunks before it
+      const uint32_t wb = rs - 6;  // log2 words of a value
+      const uint32_t g = wb >= 6 ? 0u : (l >> wb) << wb;
+      const uint64_t below = (uint64_t(1) << l) - 1, from = ~((uint64_t(1) << g) - 1);
+      bool first = d.x[i] != 0 && (nz & below & from) == 0;
+      if (wb > 6) {
+        const uint32_t c0 = (ch >> (wb - 6)) << (wb - 6);
+        const uint64_t cb = (uint64_t(1) << ch) - 1, cf = ~((uint64_t(1) << c0) - 1);
+        first = first && (chunks & cb & cf) == 0;
+      }
+      d.first[i] = ballot(first);
+      rc[i] = __popcll(d.first[i]);
+    }
+    if (l == 0) s_root[ch] = rc[i];
+  }
+  __syncthreads();
+  const uint32_t rmine = s_root[l];
+  const uint32_t rincl = wave_incl_scan<uint32_t>(rmine);
+  d.cnt = __builtin_amdgcn_readlane(cincl, kWave - 1);
+  d.roots = __builtin_amdgcn_readlane(rincl, kWave - 1);
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint32_t ch = w * kDenseWaveChunks + i;
+    d.cbase[i] = __shfl(cincl - mine, int(ch), kWave);
+    d.rbase[i] = __shfl(rincl - rmine, int(ch), kWave);
+  }
+}
+
+__device__ __forceinline__ uint32_t dense_root_shift(const DenseRel& r) {
+  return r.shift * (r.k - 1);
+}
+
+__global__ __launch_bounds__(kDenseWg) void dense_count_blocks_kernel(const DenseCtl* c, DenseRel r,
+                                                                      bool index) {
+  __shared__ uint32_t s_cnt[kDenseChunks], s_root[kDenseChunks];
+  if (!index && c->skip) return;
+  const uint64_t b = blockIdx.x;
+  if (!r.nsum[b]) {
+    if (threadIdx.x == 0) r.blk[b] = 0;
+    return;
+  }
+  DenseScan d;
+  dense_scan_block(r.nw, r.fl, b, dense_root_shift(r), s_cnt, s_root, d);
+  if (threadIdx.x == 0) r.blk[b] = uint64_t(d.cnt) | (r.k > 1 ? uint64_t(d.roots) << kDenseRowBits : 0);
+}
+
+// DELTA rows and root arrays of the block (its counts scanned in r.blk);
+// NEW joins FULL and is cleared, unless only an index is written.
+__global__ __launch_bounds__(kDenseWg) void dense_emit_blocks_kernel(const DenseCtl* c, DenseRel r,
+                                                                     bool index) {
+  __shared__ uint32_t s_cnt[kDenseChunks], s_root[kDenseChunks];
+  if (!index && !c->emit) return;
+  const uint64_t b = blockIdx.x;
+  if (!r.nsum[b]) return;
+  const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  const uint64_t w0 = b * (kDenseBlockWords / 2);
+  DenseScan d;
+  dense_scan_block(r.nw, r.fl, b, dense_root_shift(r), s_cnt, s_root, d);
+  const uint64_t off = r.blk[b];
+  const uint32_t row0 = uint32_t(off & kDenseRowMask), root0 = uint32_t(off >> kDenseRowBits);
+  const uint64_t mask = (uint64_t(1) << r.shift) - 1;
+  const uint32_t rs = dense_root_shift(r);
+  const uint64_t lt = (uint64_t(1) << l) - 1;
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave;
+    const uint64_t x = d.x[i];
+    const uint32_t p = __popcll(x);
+    const uint32_t base = row0 + d.cbase[i] + wave_incl_scan<uint32_t>(p) - p;
+    for (uint64_t nz = ballot(x != 0); nz; nz &= nz - 1) {
+      const int j = __builtin_ctzll(nz);
+      const uint64_t xj = read_lane_u64(x, j);
+      const uint32_t bj = __builtin_amdgcn_readlane(base, j);
+      const uint64_t key = ((at + uint64_t(j)) << 6) | l;
+      if ((xj >> l) & 1u) {
+        const uint32_t pos = bj + uint32_t(__popcll(xj & lt));
+        if (r.k == 2) {
+          r.delta[pos] = uint32_t(key >> r.shift);
+          r.delta[r.stride + pos] = uint32_t(key & mask);
+        } else {
+          for (uint32_t col = 0; col < r.k; ++col)
+            r.delta[uint64_t(col) * r.stride + pos] =
+                uint32_t((key >> (r.shift * (r.k - 1 - col))) & mask);
+        }
+        if (r.k == 1) {
+          r.root_v[pos] = uint32_t(key);
+          r.root_o[pos] = pos;
+        }
+      }
+      if (r.k > 1 && ((d.first[i] >> j) & 1u) && l == 0) {
+        const uint32_t g = root0 + d.rbase[i] + uint32_t(__popcll(d.first[i] & ((uint64_t(1) << j) - 1)));
+        r.root_v[g] = uint32_t(key >> rs);
+        r.root_o[g] = bj;
+      }
+    }
+    if (!index) {
+      if (x) r.fl[at + l] |= x;
+      if (r.nw[at + l]) r.nw[at + l] = 0;
+    }
+  }
+  if (!index) {
+    // every wave has read the byte; r.nw and r.fl are this block's own
+    if (threadIdx.x == 0) {
+      r.nsum[b] = 0;
+      r.fsum[b] = 1;
+    }
+  }
+}
+
+// Exclusive scan of n u64 in place by one workgroup; returns the total.
+__device__ __forceinline__ uint64_t scan_u64_wg(const uint64_t* in, uint64_t* out, uint64_t n,
+                                                uint64_t* s_w) {
+  constexpr int V = 8;
+  const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  uint64_t carry = 0;
+  for (uint64_t t0 = 0; t0 < n; t0 += uint64_t(V) * kDenseWg) {
+    // lane l of wave w: items t0 + (w*V + i)*64 + l
+    uint64_t v[V], run = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const uint64_t at = t0 + uint64_t(w * V + i) * kWave + l;
+      v[i] = at < n ? in[at] : 0;
+      run += v[i];
+    }
+    run = wave_sum<uint64_t>(run);
+    __syncthreads();  // s_w of the tile before is read
+    if (l == 0) s_w[w] = run;
+    __syncthreads();
+    uint64_t off = carry;
+    for (int j = 0; j < kDenseWgWaves; ++j) {
+      const uint64_t x = s_w[j];
+      if (uint32_t(j) < w) off += x;
+      carry += x;
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const uint64_t inc = wave_incl_scan<uint64_t>(v[i]);
+      const uint64_t at = t0 + uint64_t(w * V + i) * kWave + l;
+      if (at < n) out[at] = off + inc - v[i];
+      off += read_lane_u64(inc, kWave - 1);
+    }
+  }
+  return carry;
+}
+
+__global__ __launch_bounds__(kDenseWg) void dense_book_kernel(DenseBook B) {
+  __shared__ uint64_t s_w[kDenseWgWaves];
+  DenseCtl* c = B.ctl;
+  if (c->skip) {
+    __syncthreads();
+    if (threadIdx.x == 0) c->emit = 0;
+    return;
+  }
+  uint64_t tot[kDevRels] = {};
+#pragma unroll
+  for (int r = 0; r < kDevRels; ++r)
+    if (uint32_t(r) < B.nrels)
+      tot[r] = scan_u64_wg(B.rel[r].blk, B.rel[r].blk, B.rel[r].nblocks, s_w);
+  if (threadIdx.x != 0) return;
+  uint64_t need = 0, sum = 0;
+#pragma unroll
+  for (int r = 0; r < kDevRels; ++r)
+    if (uint32_t(r) < B.nrels) {
+      const uint64_t n = tot[r] & kDenseRowMask;
+      if (n > B.rel[r].stride && n > need) need = n;
+      sum += n;
+    }
+  uint32_t ovf = need ? uint32_t(kOvfNew) : 0u;
+  if (c->iter >= c->iter_cap) ovf |= uint32_t(kOvfIters);
+  if (ovf) {
+    c->overflow = ovf;
+    c->skip = 1;
+    c->emit = 0;
+    for (uint32_t p = 0; p < B.npipes; ++p) B.pipe[p].dyn->skip = 1;
+  } else {
+#pragma unroll
+    for (int r = 0; r < kDevRels; ++r)
+      if (uint32_t(r) < B.nrels) {
+        const uint64_t n = tot[r] & kDenseRowMask;
+        const uint64_t g = B.rel[r].k > 1 ? tot[r] >> kDenseRowBits : n;
+        B.rel[r].rec[c->iter] = n;
+        c->delta_n[r] = n;
+        c->delta_r[r] = g;
+        c->full_n[r] += n;
+        if (n) B.rel[r].root_o[g] = uint32_t(n);
+      }
+    c->iter += 1;
+    c->done = sum == 0 ? 1u : 0u;
+    c->emit = 1;
+    c->skip = c->done || c->iter >= c->max_iter ? 1u : 0u;
+    for (uint32_t p = 0; p < B.npipes; ++p) {
+      SrdDyn* d = B.pipe[p].dyn;
+      const DlBind& bd = B.pipe[p].bind;
+      for (uint32_t v = 0; v < bd.n_views; ++v) {
+        const int r = bd.vrel[v];
+        if (r < 0) continue;
+        IndexView& iv = d->views.v[v];
+        iv.cols = B.rel[r].delta;
+        iv.root_vals = B.rel[r].root_v;
+        iv.root_offs = B.rel[r].root_o;
+        iv.stride = B.rel[r].stride;
+        iv.n = uint32_t(c->delta_n[r]);
+        iv.r = uint32_t(c->delta_r[r]);
+      }
+      uint32_t drv = bd.root_view[0], nr;
+      if (bd.root_kind == SRD_ROOT_JOIN) {
+        for (uint32_t i = 0; i < bd.n_root_src; ++i)
+          if (d->views.v[bd.root_view[i]].r < d->views.v[drv].r) drv = bd.root_view[i];
+        nr = d->views.v[drv].r;
+      } else {
+        nr = d->views.v[drv].n ? 1u : 0u;
+      }
+      d->skip = c->skip;
+      d->drv_view = drv;
+      d->n_root = nr;
+      c->keys[p] = nr;
+    }
+  }
+  c->tick += 1;
+  DenseSeen* h = B.seen;
+  __hip_atomic_store(&h->iter, c->iter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&h->need, need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&h->done, c->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&h->overflow, ovf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&h->tick, c->tick, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ void dense_plan_finish(SrdDyn* d, uint64_t tw, uint32_t* work_ctr,
+                                                  uint32_t grain, bool fixed_grain) {
+  for (uint32_t i = threadIdx.x; i < SRD_XCDS * SRD_CTR_STRIDE; i += blockDim.x) work_ctr[i] = 0;
+  if (threadIdx.x == 0) {
+    const uint32_t g = fixed_grain ? grain : srd_grain(tw, grain);
+    d->total_work = tw;
+    d->grain = g;
+    d->n_slices = (tw + g - 1) / g;
+  }
+}
+
+__global__ __launch_bounds__(kDenseWg) void dense_plan_kernel(SrdDyn* d, const uint64_t* key_work,
+                                                              uint64_t* work_start,
+                                                              uint32_t* work_ctr, uint32_t grain,
+                                                              bool fixed_grain) {
+  __shared__ uint64_t s_w[kDenseWgWaves];
+  if (d->skip) return;
+  const uint64_t n = d->n_root;
+  const uint64_t tw = scan_u64_wg(key_work, work_start, n, s_w);
+  if (threadIdx.x == 0) work_start[n] = tw;
+  dense_plan_finish(d, tw, work_ctr, grain, fixed_grain);
+}
+
+// After a multi-launch scan.
+__global__ __launch_bounds__(kBlock) void dense_plan_tail_kernel(SrdDyn* d, const uint64_t* work_start,
+                                                                 uint32_t* work_ctr, uint32_t grain,
+                                                                 bool fixed_grain) {
+  if (d->skip) return;
+  dense_plan_finish(d, work_start[d->n_root], work_ctr, grain, fixed_grain);
+}
+
+void dense_plan(DenseCtl* c, SrdDyn* d, uint32_t pipe, const uint64_t* key_work, uint64_t* work_start,
+                uint64_t cap_keys, uint64_t* scan_tmp, uint32_t* work_ctr, uint32_t grain,
+                bool fixed_grain, hipStream_t s) {
+  if (cap_keys <= kDensePlanKeys) {
+    dense_plan_kernel<<<1, kDenseWg, 0, s>>>(d, key_work, work_start, work_ctr, grain, fixed_grain);
+  } else {
+    exclusive_scan_u64_dev(key_work, work_start, cap_keys, &c->keys[pipe], scan_tmp, s);
+    dense_plan_tail_kernel<<<1, kBlock, 0, s>>>(d, work_start, work_ctr, grain, fixed_grain);
+  }
+  SRD_CHECK(hipGetLastError());
+}
+
+__global__ __launch_bounds__(kBlock) void dense_set_rows_kernel(const uint32_t* __restrict__ cols,
+                                                                uint64_t stride, uint64_t n, uint32_t k,
+                                                                uint32_t shift,
+                                                                unsigned long long* __restrict__ bits,
+                                                                uint8_t* __restrict__ sum) {
+  for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n;
+       i += uint64_t(gridDim.x) * kBlock) {
+    uint64_t key = 0;
+    for (uint32_t c = 0; c < k; ++c) key = (key << shift) | cols[uint64_t(c) * stride + i];
+    atomicOr(bits + (key >> 6), 1ull << (key & 63u));
+    __hip_atomic_store(sum + (key >> 18), uint8_t(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+}
+
+void dense_set_rows(const uint32_t* cols, uint64_t stride, uint64_t n, uint32_t k, uint32_t shift,
+                    uint64_t* bits, uint8_t* sum, hipStream_t s) {
+  if (n == 0) return;
+  dense_set_rows_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(
+      cols, stride, n, k, shift, reinterpret_cast<unsigned long long*>(bits), sum);
+  SRD_CHECK(hipGetLastError());
+}
+
+void dense_count(const DenseCtl* c, const DenseRel& r, hipStream_t s) {
+  dense_count_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(c, r, false);
+  SRD_CHECK(hipGetLastError());
+}
+
+void dense_book(const DenseBook& b, hipStream_t s) {
+  dense_book_kernel<<<1, kDenseWg, 0, s>>>(b);
+  SRD_CHECK(hipGetLastError());
+}
+
+void dense_emit(const DenseCtl* c, const DenseRel& r, hipStream_t s) {
+  dense_emit_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(c, r, false);
+  SRD_CHECK(hipGetLastError());
+}
+
+__global__ __launch_bounds__(kDenseWg) void dense_index_scan_kernel(uint64_t* blk, uint32_t n) {
+  __shared__ uint64_t s_w[kDenseWgWaves];
+  const uint64_t t = scan_u64_wg(blk, blk, n, s_w);
+  if (threadIdx.x == 0) blk[n] = t;
+}
+
+void dense_index_count(const DenseRel& r, hipStream_t s) {
+  dense_count_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(nullptr, r, true);
+  SRD_CHECK(hipGetLastError());
+  dense_index_scan_kernel<<<1, kDenseWg, 0, s>>>(r.blk, r.nblocks);
+  SRD_CHECK(hipGetLastError());
+}
+
+void dense_index_emit(const DenseRel& r, hipStream_t s) {
+  dense_emit_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(nullptr, r, true);
+  SRD_CHECK(hipGetLastError());
+}
+
+__global__ __launch_bounds__(kBlock) void dense_inst_kernel(const DenseCtl* c, uint32_t r,
+                                                            const uint32_t* __restrict__ col0,
+                                                            const uint32_t* __restrict__ bounds,
+                                                            uint32_t n_inst, uint64_t* __restrict__ out) {
+  if (!c->emit) return;
+  const uint32_t g = blockIdx.x * kBlock + threadIdx.x;
+  if (g >= n_inst) return;
+  const uint32_t n = uint32_t(c->delta_n[r]);
+  const uint32_t lo = n ? lower_bound(col0, 0, n, bounds[g]) : 0;
+  const uint32_t hi = n ? lower_bound(col0, lo, n, bounds[g + 1]) : 0;
+  out[(c->iter - 1) * n_inst + g] = hi - lo;
+}
+
+void dense_inst(const DenseCtl* c, uint32_t rel, const uint32_t* col0, const uint32_t* bounds,
+                uint32_t n_inst, uint64_t* out, hipStream_t s) {
+  if (n_inst == 0) return;
+  dense_inst_kernel<<<(n_inst + kBlock - 1) / kBlock, kBlock, 0, s>>>(c, rel, col0, bounds, n_inst, out);
+  SRD_CHECK(hipGetLastError());
+}
+
 }  // namespace srd

@@ -673,7 +673,9 @@ class PipelineGen:
          "  (void)drv_;",
          "  const uint64_t tw_ = DYN ? A.dyn->total_work : A.total_work;",
          "  const uint64_t ns_ = DYN ? A.dyn->n_slices : A.n_slices;",
-         "  const uint32_t gr_ = DYN ? A.dyn->grain : A.grain;"]
+         "  const uint32_t gr_ = DYN ? A.dyn->grain : A.grain;",
+         "  // a block beyond the slices would only find every counter exhausted",
+         "  if (A.slice_lo + blockIdx.x * 4ull >= ns_) return;"]
     for di in range(len(self.dests)):
       o.append(f"  const uint64_t ob{di}_ = DYN ? A.dyn->out_base[{di}] : A.out[{di}].base;")
     o += ["  const uint32_t lane = srd::lane_id();"]
@@ -734,6 +736,8 @@ class PipelineGen:
             "    __builtin_amdgcn_wave_barrier();",
             "    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, \"wavefront\");",
             "  }"]
+    if self.mark_ok():
+      o += ["  uint64_t rows_ = 0;  // MODE 6: tuples this wave derived"]
     o += ["  // fused mode: the wave's open staging segment, kept across slices (a",
           "  // slice's rows in it are one record; the next slice goes on behind them)",
           "  uint32_t probes_ = 0;  // MODE 5: searches, map lookups and bitmap tests of this lane",
@@ -835,7 +839,14 @@ class PipelineGen:
           "      if (seg_start != ~uint64_t(0)) { seg_start += seg_used; seg_room -= seg_used; }",
           "    }",
           "    if ((MODE == 0 || MODE == 2) && lane == 0) A.counts[slice] = cnt;",
+          *(["    if (MODE == 6) rows_ += cnt;"] if self.mark_ok() else []),
           "  }"]
+    if self.mark_ok():
+      o += ["  if constexpr (MODE == 6) {",
+            "    if (A.mark_rows && lane == 0 && rows_)",
+            "      atomicAdd(A.mark_rows + ((blockIdx.x * 4u + threadIdx.x / 64u) % SRD_ROW_CTRS) * "
+            "SRD_ROW_CTR_STRIDE, (unsigned long long)rows_);",
+            "  }"]
     if self.ring:
       o += ["  if (MODE == 2 && seg_start != ~uint64_t(0)) ring_out(seg_start, false);"]
     o += ["  if constexpr (MODE == 5) {",
@@ -886,9 +897,12 @@ class PipelineGen:
             f"          const uint32_t {self.var(self.root.var)} = V.v[drv_].root_vals[klo];",
             f"          (void){self.var(self.root.var)};",
             f"          const uint32_t rb_ = kr_[{2 * sr}], nr_ = kr_[{2 * sr + 1}] - rb_;",
+            "          const uint32_t p0_ = srdj::prod_cut(nr_, base - ks_, kw_);",
+            "          const uint32_t p1_ = srdj::prod_cut(nr_, hi_ - ks_, kw_);",
             f"          srdj::prod_mark(A, {self.prod_base(p, lambda v: v)}, "
             f"A.mark_shift * {p['k'] - 1 - p['cr']}u, {cm}, kr_[{2 * sm}], kr_[{2 * sm + 1}], {cr}, "
-            "rb_ + srdj::prod_cut(nr_, base - ks_, kw_), rb_ + srdj::prod_cut(nr_, hi_ - ks_, kw_), lw_, lm_);",
+            "rb_ + p0_, rb_ + p1_, lw_, lm_);",
+            f"          rows_ += uint64_t(p1_ - p0_) * (kr_[{2 * sm + 1}] - kr_[{2 * sm}]);",
             "          kc = klo;",
             "          step_ = hi_ - base;",
             "          continue;",
@@ -1103,6 +1117,7 @@ class PipelineGen:
              f"{i2}srdj::prod_mark(A, {self.prod_base(p, rl)}, A.mark_shift * {p['k'] - 1 - p['cr']}u, "
              f"{self.col_expr(rm.view, rm.depth)}, {rl(f'uint32_t({mb})')}, {rl(f'uint32_t({me})')}, "
              f"{self.col_expr(rr.view, rr.depth)}, rb_ + {rl('p0_')}, rb_ + {rl('p1_')}, lw_, lm_);",
+             f"{i2}rows_ += uint64_t({rl('p1_')} - {rl('p0_')}) * ({rl(f'uint32_t({me})')} - {rl(f'uint32_t({mb})')});",
              f"{i1}}}",
              f"{ind}}}"]
     return code
@@ -1257,7 +1272,10 @@ class PipelineGen:
            "}"] + ([
            "void launch_direct_dyn(const SrdLaunchArgs* a, hipStream_t s) {",
            "  run_k<3, true><<<a->grid_blocks, 256, 0, s>>>(*a);",
-           "}"] if self.direct_ok() else []) if self.dyn else []) + [
+           "}"] if self.direct_ok() else []) + ([
+           "void launch_mark_dyn(const SrdLaunchArgs* a, hipStream_t s) {",
+           "  run_k<6, true><<<a->grid_blocks, 256, 0, s>>>(*a);",
+           "}"] if self.mark_ok() else []) if self.dyn else []) + [
            f"}}  // namespace {self.ns}", ""]
     return "\n".join(out)
 
@@ -1269,7 +1287,8 @@ class PipelineGen:
     return min(len(self.levels), 3)
 
   def gen_ext(self) -> str:
-    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}}}"
+    dyn = f"&{self.ns}::launch_mark_dyn" if self.dyn and self.mark_ok() else "nullptr"
+    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}, {dyn}}}"
 
   def gen_desc(self) -> str:
     views = []

@@ -18,7 +18,7 @@ typedef int hipError_t;
 typedef void* hipStream_t;
 typedef void* hipEvent_t;
 typedef void* hipMemPool_t;
-enum { hipSuccess = 0 };
+enum { hipSuccess = 0, hipErrorNotReady = 600 };
 enum hipMemcpyKind { hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipMemcpyDeviceToDevice,
                      hipMemcpyHostToHost };
 enum { hipStreamNonBlocking = 1, hipHostMallocDefault = 0 };
@@ -29,6 +29,7 @@ inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (void*)1; return 0; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 // Everything runs in program order on the host: events and waits do nothing
 // but report to sim_stream_event (op 0: a record on s, 1: s waits), which

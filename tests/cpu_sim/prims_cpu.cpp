@@ -188,6 +188,25 @@ void export_rows(const Index& x, uint32_t* host_out, const uint32_t* bounds, uin
   }
 }
 
+// Dense iterations need rules with device-sized mark launches, which the
+// host-only pipelines do not have.
+void dense_set_rows(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uint64_t*, uint8_t*,
+                    hipStream_t) {
+  fail("dense_set_rows: not in the host-only build");
+}
+void dense_plan(DenseCtl*, SrdDyn*, uint32_t, const uint64_t*, uint64_t*, uint64_t, uint64_t*, uint32_t*,
+                uint32_t, bool, hipStream_t) {
+  fail("dense_plan: not in the host-only build");
+}
+void dense_count(const DenseCtl*, const DenseRel&, hipStream_t) { fail("dense_count: not in the host-only build"); }
+void dense_book(const DenseBook&, hipStream_t) { fail("dense_book: not in the host-only build"); }
+void dense_emit(const DenseCtl*, const DenseRel&, hipStream_t) { fail("dense_emit: not in the host-only build"); }
+void dense_inst(const DenseCtl*, uint32_t, const uint32_t*, const uint32_t*, uint32_t, uint64_t*, hipStream_t) {
+  fail("dense_inst: not in the host-only build");
+}
+void dense_index_count(const DenseRel&, hipStream_t) { fail("dense_index_count: not in the host-only build"); }
+void dense_index_emit(const DenseRel&, hipStream_t) { fail("dense_index_emit: not in the host-only build"); }
+
 void cost_items(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
                 hipStream_t) {
   if (S == 0 || n == 0) fail("cost_items: no slices");
