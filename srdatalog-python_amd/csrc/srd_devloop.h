@@ -224,6 +224,8 @@ struct DenseRel {
   uint64_t* fl;
   uint8_t* nsum;
   uint8_t* fsum;
+  uint8_t* live;         // blocks to emit: their bytes of nsum when they were counted
+  uint64_t* chunk;       // per 4096 keys: rows and column-0 values before it in its block
   uint64_t* blk;         // per block: NEW rows | column-0 values << kDenseRowBits, scanned in place
                          // (no column-0 values counted for k == 1: every row is one)
   uint32_t* delta;       // k columns of `stride` rows, root arrays
@@ -268,11 +270,12 @@ constexpr uint64_t kDensePlanKeys = 65536;  // most keys the one-block scan take
 // FULL bitmap := the rows of an index (bits and block bytes set).
 void dense_set_rows(const uint32_t* cols, uint64_t stride, uint64_t n, uint32_t k, uint32_t shift,
                     uint64_t* bits, uint8_t* sum, hipStream_t s);
-// Scan of a pipeline's per-key work, its total, grain and slice count, and
-// its slice counters cleared.
+// Scan of a pipeline's per-key work, its total, grain (srd_grain from `grain`
+// and `least`; exactly `grain` when least is 0) and slice count, and its slice
+// counters cleared.
 void dense_plan(DenseCtl* c, SrdDyn* d, uint32_t pipe, const uint64_t* key_work, uint64_t* work_start,
                 uint64_t cap_keys, uint64_t* scan_tmp, uint32_t* work_ctr, uint32_t grain,
-                bool fixed_grain, hipStream_t s);
+                uint32_t least, hipStream_t s);
 void dense_count(const DenseCtl* c, const DenseRel& r, hipStream_t s);
 void dense_book(const DenseBook& b, hipStream_t s);
 void dense_emit(const DenseCtl* c, const DenseRel& r, hipStream_t s);

@@ -943,7 +943,8 @@ static void pr_root(srd_engine& e, PipeRun& R) {
 static void pr_slices(srd_engine& e, PipeRun& R) {
   const SrdPipelineDesc* d = R.d;
   R.a.total_work = R.host[0];
-  if (!e.grain_override) R.a.grain = srd_grain(R.a.total_work, d->default_grain);
+  if (!e.grain_override)
+    R.a.grain = srd_grain(R.a.total_work, d->default_grain, R.a.mark_prod == 1 ? SRD_PROD_GRAIN : 64u);
   R.a.n_slices = (R.a.total_work + R.a.grain - 1) / R.a.grain;
   const bool direct = d->direct_ok && !d->count_only && !e.two_pass && !e.no_direct;
   R.weigh_items = 0;
@@ -2602,8 +2603,8 @@ struct DenseRelState {
   int rel = -1;
   DenseRel d;
   const Index* full0 = nullptr;
-  DevBuf<uint32_t> fl, fsum, delta, root_v, root_o;
-  DevBuf<uint64_t> blk, rec, inst;
+  DevBuf<uint32_t> fl, fsum, live, delta, root_v, root_o;
+  DevBuf<uint64_t> blk, chunk, rec, inst;
 };
 
 struct DensePipeState {
@@ -2713,7 +2714,11 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
     fill_u32(R.fl.p, 0, words, s);
     R.fsum.alloc(sum_words, s);
     fill_u32(R.fsum.p, 0, sum_words, s);
+    R.live.alloc(sum_words, s);
     R.blk.alloc(uint64_t(R.d.nblocks) + 1, s);
+    R.chunk.alloc(uint64_t(R.d.nblocks) * 64, s);
+    R.d.live = reinterpret_cast<uint8_t*>(R.live.p);
+    R.d.chunk = R.chunk.p;
     R.rec.alloc(h.iter_cap, s);
     if (e.n_inst) R.inst.alloc(h.iter_cap * e.n_inst, s);
     R.d.nw = reinterpret_cast<uint64_t*>(r.dense_bits.p);
@@ -2819,7 +2824,8 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
       P.d->root_dyn(&a, s);
       SRD_CHECK(hipGetLastError());
       dense_plan(ctl, const_cast<SrdDyn*>(P.a.dyn), uint32_t(p), P.key_work.p, P.work_start.p, P.cap_keys,
-                 P.scan.p, P.work_ctr.p, P.grain, e.grain_override != 0, s);
+                 P.scan.p, P.work_ctr.p, P.grain,
+                 e.grain_override ? 0u : (P.a.mark_prod == 1 ? SRD_PROD_GRAIN : 64u), s);
       P.x->mark_dyn(&P.a, s);
       SRD_CHECK(hipGetLastError());
     }

@@ -195,16 +195,21 @@ struct SrdDyn {
 // each wave, in whole 64-item batches.  A wave walks its slice serially, a
 // dozen dependent loads per batch, so with 4096 items a slice the 5,000 rows
 // of a small relation ran on two waves: 83 us against 31 us for the load of
-// 5,000 pairs, 254 us against 70 us for 260,000 pairs, and 133 us against
+// 5,000 pairs, 254 us against 70 us for 260,000 pairs (21 and 22 us since waves
+// own their first slices), and 133 us against
 // 95 us (mean over the iterations) for the recursive join of the closure of
 // 5,000 pairs over 1,000 vertices.
 #define SRD_GRID_WAVES 8192u
-__host__ __device__ inline uint32_t srd_grain(uint64_t total, uint32_t dflt) {
-  if (dflt <= 64u) return dflt;
+// A launch whose products are marked row by row counts 64 units a step and
+// folds a product's values anew in every slice that holds some of its rows:
+// its slices hold at least SRD_PROD_GRAIN units.
+#define SRD_PROD_GRAIN 1024u
+__host__ __device__ inline uint32_t srd_grain(uint64_t total, uint32_t dflt, uint32_t least = 64u) {
+  if (dflt <= least) return dflt;
   const uint64_t share = (total + SRD_GRID_WAVES - 1) / SRD_GRID_WAVES;
   if (share >= dflt) return dflt;
   const uint32_t g = (uint32_t(share) + 63u) & ~63u;
-  return g < 64u ? 64u : (g < dflt ? g : dflt);
+  return g < least ? least : (g < dflt ? g : dflt);
 }
 
 typedef void (*SrdLaunchFn)(const SrdLaunchArgs* args, hipStream_t stream);

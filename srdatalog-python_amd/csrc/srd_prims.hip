@@ -3110,114 +3110,101 @@ constexpr int kDenseChunks = 64;
 constexpr int kDenseWaveChunks = kDenseChunks / kDenseWgWaves;
 static_assert(kDenseBlockWords == 2ull * kDenseChunks * kWave, "64 chunks of 64 words of 64 keys");
 
-struct DenseScan {
-  uint64_t x[kDenseWaveChunks];     // this lane's words of NEW & ~FULL
-  uint64_t first[kDenseWaveChunks]; // words that open a column-0 value, by chunk
-  uint32_t cnt, roots;              // of the whole block
-  uint32_t cbase[kDenseWaveChunks], rbase[kDenseWaveChunks];  // before each chunk, in the block
-};
-
-// The block's new words, which of them hold the first rows of a column-0
-// value, and the rows and values before each of the wave's chunks.  s_*: LDS
-// of the workgroup.  rs = bits of a column-0 value's keys (k == 1: 0).
-__device__ __forceinline__ void dense_scan_block(const uint64_t* nw, const uint64_t* fl, uint64_t b,
-                                                 uint32_t rs, uint32_t* s_cnt, uint32_t* s_root,
-                                                 DenseScan& d) {
-  const uint32_t w = threadIdx.x / kWave, l = lane_id();
-  const uint64_t w0 = b * (kDenseBlockWords / 2);
-  uint32_t pc[kDenseWaveChunks];
-#pragma unroll
-  for (int i = 0; i < kDenseWaveChunks; ++i) {
-    const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave + l;
-    uint64_t x = nw[at];
-    if (fl) x &= ~fl[at];
-    d.x[i] = x;
-    pc[i] = wave_sum<uint32_t>(__popcll(x));
-    if (l == 0) s_cnt[w * kDenseWaveChunks + i] = pc[i];
-  }
-  __syncthreads();
-  const uint32_t mine = s_cnt[l];  // lane l: rows of chunk l
-  const uint64_t chunks = ballot(mine != 0);
-  const uint32_t cincl = wave_incl_scan<uint32_t>(mine);
-  uint32_t rc[kDenseWaveChunks];
-#pragma unroll
-  for (int i = 0; i < kDenseWaveChunks; ++i) {
-    const uint32_t ch = w * kDenseWaveChunks + i;
-    const uint64_t nz = ballot(d.x[i] != 0);
-    if (rs == 0) {
-      d.first[i] = nz;
-      rc[i] = pc[i];
-    } else {
-      // words of the lane's column-0 value before it: in the chunk, and, for
-      // values wider than a chunk, in the chunks before it
-      const uint32_t wb = rs - 6;  // log2 words of a value
-      const uint32_t g = wb >= 6 ? 0u : (l >> wb) << wb;
-      const uint64_t below = (uint64_t(1) << l) - 1, from = ~((uint64_t(1) << g) - 1);
-      bool first = d.x[i] != 0 && (nz & below & from) == 0;
-      if (wb > 6) {
-        const uint32_t c0 = (ch >> (wb - 6)) << (wb - 6);
-        const uint64_t cb = (uint64_t(1) << ch) - 1, cf = ~((uint64_t(1) << c0) - 1);
-        first = first && (chunks & cb & cf) == 0;
-      }
-      d.first[i] = ballot(first);
-      rc[i] = __popcll(d.first[i]);
-    }
-    if (l == 0) s_root[ch] = rc[i];
-  }
-  __syncthreads();
-  const uint32_t rmine = s_root[l];
-  const uint32_t rincl = wave_incl_scan<uint32_t>(rmine);
-  d.cnt = __builtin_amdgcn_readlane(cincl, kWave - 1);
-  d.roots = __builtin_amdgcn_readlane(rincl, kWave - 1);
-#pragma unroll
-  for (int i = 0; i < kDenseWaveChunks; ++i) {
-    const uint32_t ch = w * kDenseWaveChunks + i;
-    d.cbase[i] = __shfl(cincl - mine, int(ch), kWave);
-    d.rbase[i] = __shfl(rincl - rmine, int(ch), kWave);
-  }
+// Rows, column-0 values before a chunk in its block (18 bits each), and
+// whether the chunk's first column-0 value has rows in an earlier chunk.
+__device__ __forceinline__ uint64_t chunk_pack(uint32_t rows, uint32_t roots, bool cont) {
+  return uint64_t(rows) | (uint64_t(roots) << 20) | (cont ? uint64_t(1) << 63 : 0);
 }
 
 __device__ __forceinline__ uint32_t dense_root_shift(const DenseRel& r) {
   return r.shift * (r.k - 1);
 }
 
+// Which of a chunk's words (x: this lane's) hold the first row of a column-0
+// value of 2^rs keys; cont: the chunk's first value began in an earlier chunk.
+__device__ __forceinline__ uint64_t chunk_firsts(uint64_t x, uint32_t rs, bool cont) {
+  const uint32_t l = lane_id();
+  const uint64_t nz = ballot(x != 0);
+  if (rs == 0) return nz;
+  const uint32_t wb = rs - 6;  // log2 words of a value
+  const uint32_t g = wb >= 6 ? 0u : (l >> wb) << wb;
+  const uint64_t below = (uint64_t(1) << l) - 1, from = ~((uint64_t(1) << g) - 1);
+  return ballot(x != 0 && (nz & below & from) == 0 && !(wb > 6 && cont));
+}
+
+// Rows and column-0 values of the block's new words: the totals to blk, what
+// precedes each chunk to chunk.
 __global__ __launch_bounds__(kDenseWg) void dense_count_blocks_kernel(const DenseCtl* c, DenseRel r,
                                                                       bool index) {
   __shared__ uint32_t s_cnt[kDenseChunks], s_root[kDenseChunks];
   if (!index && c->skip) return;
   const uint64_t b = blockIdx.x;
-  if (!r.nsum[b]) {
+  const bool on = r.nsum[b] != 0;
+  if (!index && threadIdx.x == 0) r.live[b] = on ? 1 : 0;
+  if (!on) {
     if (threadIdx.x == 0) r.blk[b] = 0;
     return;
   }
-  DenseScan d;
-  dense_scan_block(r.nw, r.fl, b, dense_root_shift(r), s_cnt, s_root, d);
-  if (threadIdx.x == 0) r.blk[b] = uint64_t(d.cnt) | (r.k > 1 ? uint64_t(d.roots) << kDenseRowBits : 0);
+  const uint32_t w = threadIdx.x / kWave, l = lane_id(), rs = dense_root_shift(r);
+  const uint64_t w0 = b * (kDenseBlockWords / 2);
+  uint64_t x[kDenseWaveChunks];
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave + l;
+    x[i] = r.nw[at];
+    if (r.fl) x[i] &= ~r.fl[at];
+    const uint32_t pc = wave_sum<uint32_t>(__popcll(x[i]));
+    if (l == 0) s_cnt[w * kDenseWaveChunks + i] = pc;
+  }
+  __syncthreads();
+  const uint32_t mine = s_cnt[l];  // lane l: rows of chunk l
+  const uint64_t chunks = ballot(mine != 0);
+  const uint32_t wb = rs >= 6 ? rs - 6 : 0;
+  // lane l: chunk l's value began in an earlier chunk that holds rows of it
+  const uint32_t c0 = wb > 6 ? (l >> (wb - 6)) << (wb - 6) : l;
+  const bool cont = (chunks & ((uint64_t(1) << l) - 1) & ~((uint64_t(1) << c0) - 1)) != 0;
+  const uint64_t conts = ballot(cont);
+#pragma unroll
+  for (int i = 0; i < kDenseWaveChunks; ++i) {
+    const uint32_t ch = w * kDenseWaveChunks + i;
+    const uint64_t f = chunk_firsts(x[i], rs, (conts >> ch) & 1u);
+    if (l == 0) s_root[ch] = __popcll(f);
+  }
+  __syncthreads();
+  if (w != 0) return;
+  const uint32_t rmine = r.k > 1 ? s_root[l] : 0u;
+  const uint32_t cincl = wave_incl_scan<uint32_t>(mine), rincl = wave_incl_scan<uint32_t>(rmine);
+  r.chunk[b * kDenseChunks + l] = chunk_pack(cincl - mine, rincl - rmine, cont);
+  if (l == kWave - 1) r.blk[b] = uint64_t(cincl) | (uint64_t(rincl) << kDenseRowBits);
 }
 
-// DELTA rows and root arrays of the block (its counts scanned in r.blk);
-// NEW joins FULL and is cleared, unless only an index is written.
-__global__ __launch_bounds__(kDenseWg) void dense_emit_blocks_kernel(const DenseCtl* c, DenseRel r,
-                                                                     bool index) {
-  __shared__ uint32_t s_cnt[kDenseChunks], s_root[kDenseChunks];
+// DELTA rows and root arrays of the block's chunks (counted in r.chunk, the
+// blocks before in r.blk); NEW joins FULL and is cleared, unless only an index
+// is written.  gridDim.y workgroups share a block's chunks: a bitmap of few
+// blocks is written by more CUs than it has blocks (390,000 rows in the four
+// blocks of 2^20 keys: 67 us with a workgroup per block, 18 us with 16).
+__global__ __launch_bounds__(kBlock) void dense_emit_blocks_kernel(const DenseCtl* c, DenseRel r,
+                                                                   bool index) {
   if (!index && !c->emit) return;
   const uint64_t b = blockIdx.x;
-  if (!r.nsum[b]) return;
-  const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  if (!(index ? r.nsum[b] : r.live[b])) return;
+  const uint32_t l = lane_id(), rs = dense_root_shift(r);
   const uint64_t w0 = b * (kDenseBlockWords / 2);
-  DenseScan d;
-  dense_scan_block(r.nw, r.fl, b, dense_root_shift(r), s_cnt, s_root, d);
   const uint64_t off = r.blk[b];
   const uint32_t row0 = uint32_t(off & kDenseRowMask), root0 = uint32_t(off >> kDenseRowBits);
   const uint64_t mask = (uint64_t(1) << r.shift) - 1;
-  const uint32_t rs = dense_root_shift(r);
   const uint64_t lt = (uint64_t(1) << l) - 1;
-#pragma unroll
-  for (int i = 0; i < kDenseWaveChunks; ++i) {
-    const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave;
-    const uint64_t x = d.x[i];
+  for (uint32_t ch = blockIdx.y * kWavesPerBlock + threadIdx.x / kWave; ch < uint32_t(kDenseChunks);
+       ch += gridDim.y * kWavesPerBlock) {
+    const uint64_t at = w0 + uint64_t(ch) * kWave;
+    const uint64_t n = r.nw[at + l];
+    const uint64_t f = r.fl ? r.fl[at + l] : 0;
+    const uint64_t x = n & ~f;
+    const uint64_t ck = r.chunk[b * kDenseChunks + ch];
+    const uint64_t first = chunk_firsts(x, rs, ck >> 63);
     const uint32_t p = __popcll(x);
-    const uint32_t base = row0 + d.cbase[i] + wave_incl_scan<uint32_t>(p) - p;
+    const uint32_t base = row0 + uint32_t(ck & 0xFFFFFu) + wave_incl_scan<uint32_t>(p) - p;
+    const uint32_t groot = root0 + uint32_t((ck >> 20) & 0xFFFFFu);
     for (uint64_t nz = ballot(x != 0); nz; nz &= nz - 1) {
       const int j = __builtin_ctzll(nz);
       const uint64_t xj = read_lane_u64(x, j);
@@ -3238,24 +3225,24 @@ __global__ __launch_bounds__(kDenseWg) void dense_emit_blocks_kernel(const Dense
           r.root_o[pos] = pos;
         }
       }
-      if (r.k > 1 && ((d.first[i] >> j) & 1u) && l == 0) {
-        const uint32_t g = root0 + d.rbase[i] + uint32_t(__popcll(d.first[i] & ((uint64_t(1) << j) - 1)));
+      if (r.k > 1 && ((first >> j) & 1u) && l == 0) {
+        const uint32_t g = groot + uint32_t(__popcll(first & ((uint64_t(1) << j) - 1)));
         r.root_v[g] = uint32_t(key >> rs);
         r.root_o[g] = bj;
       }
     }
     if (!index) {
-      if (x) r.fl[at + l] |= x;
-      if (r.nw[at + l]) r.nw[at + l] = 0;
+      if (x) r.fl[at + l] = f | x;
+      if (n) r.nw[at + l] = 0;
     }
   }
-  if (!index) {
-    // every wave has read the byte; r.nw and r.fl are this block's own
-    if (threadIdx.x == 0) {
-      r.nsum[b] = 0;
-      r.fsum[b] = 1;
-    }
-  }
+  if (!index && threadIdx.x == 0 && blockIdx.y == 0) r.fsum[b] = 1;
+}
+
+// Workgroups per block: all 64 chunks at once for small bitmaps, down to one
+// workgroup for those whose mostly unmarked blocks already fill the chip.
+static uint32_t dense_emit_parts(const DenseRel& r) {
+  return r.nblocks <= 256 ? 16u : (r.nblocks <= 2048 ? 4u : 1u);
 }
 
 // Exclusive scan of n u64 in place by one workgroup; returns the total.
@@ -3307,6 +3294,20 @@ __global__ __launch_bounds__(kDenseWg) void dense_book_kernel(DenseBook B) {
   for (int r = 0; r < kDevRels; ++r)
     if (uint32_t(r) < B.nrels)
       tot[r] = scan_u64_wg(B.rel[r].blk, B.rel[r].blk, B.rel[r].nblocks, s_w);
+  __syncthreads();
+  bool fits = c->iter < c->iter_cap;
+#pragma unroll
+  for (int r = 0; r < kDevRels; ++r)
+    if (uint32_t(r) < B.nrels) fits = fits && (tot[r] & kDenseRowMask) <= B.rel[r].stride;
+  if (fits) {
+    // the marked blocks are noted in `live`: the next iteration marks anew
+#pragma unroll
+    for (int r = 0; r < kDevRels; ++r)
+      if (uint32_t(r) < B.nrels)
+        for (uint32_t i = threadIdx.x; i < (B.rel[r].nblocks + 3) / 4; i += kDenseWg)
+          reinterpret_cast<uint32_t*>(B.rel[r].nsum)[i] = 0;
+  }
+  __syncthreads();  // c->iter is read
   if (threadIdx.x != 0) return;
   uint64_t need = 0, sum = 0;
 #pragma unroll
@@ -3377,10 +3378,10 @@ __global__ __launch_bounds__(kDenseWg) void dense_book_kernel(DenseBook B) {
 }
 
 __device__ __forceinline__ void dense_plan_finish(SrdDyn* d, uint64_t tw, uint32_t* work_ctr,
-                                                  uint32_t grain, bool fixed_grain) {
+                                                  uint32_t grain, uint32_t least) {
   for (uint32_t i = threadIdx.x; i < SRD_XCDS * SRD_CTR_STRIDE; i += blockDim.x) work_ctr[i] = 0;
   if (threadIdx.x == 0) {
-    const uint32_t g = fixed_grain ? grain : srd_grain(tw, grain);
+    const uint32_t g = least ? srd_grain(tw, grain, least) : grain;
     d->total_work = tw;
     d->grain = g;
     d->n_slices = (tw + g - 1) / g;
@@ -3390,31 +3391,31 @@ __device__ __forceinline__ void dense_plan_finish(SrdDyn* d, uint64_t tw, uint32
 __global__ __launch_bounds__(kDenseWg) void dense_plan_kernel(SrdDyn* d, const uint64_t* key_work,
                                                               uint64_t* work_start,
                                                               uint32_t* work_ctr, uint32_t grain,
-                                                              bool fixed_grain) {
+                                                              uint32_t least) {
   __shared__ uint64_t s_w[kDenseWgWaves];
   if (d->skip) return;
   const uint64_t n = d->n_root;
   const uint64_t tw = scan_u64_wg(key_work, work_start, n, s_w);
   if (threadIdx.x == 0) work_start[n] = tw;
-  dense_plan_finish(d, tw, work_ctr, grain, fixed_grain);
+  dense_plan_finish(d, tw, work_ctr, grain, least);
 }
 
 // After a multi-launch scan.
 __global__ __launch_bounds__(kBlock) void dense_plan_tail_kernel(SrdDyn* d, const uint64_t* work_start,
                                                                  uint32_t* work_ctr, uint32_t grain,
-                                                                 bool fixed_grain) {
+                                                                 uint32_t least) {
   if (d->skip) return;
-  dense_plan_finish(d, work_start[d->n_root], work_ctr, grain, fixed_grain);
+  dense_plan_finish(d, work_start[d->n_root], work_ctr, grain, least);
 }
 
 void dense_plan(DenseCtl* c, SrdDyn* d, uint32_t pipe, const uint64_t* key_work, uint64_t* work_start,
                 uint64_t cap_keys, uint64_t* scan_tmp, uint32_t* work_ctr, uint32_t grain,
-                bool fixed_grain, hipStream_t s) {
+                uint32_t least, hipStream_t s) {
   if (cap_keys <= kDensePlanKeys) {
-    dense_plan_kernel<<<1, kDenseWg, 0, s>>>(d, key_work, work_start, work_ctr, grain, fixed_grain);
+    dense_plan_kernel<<<1, kDenseWg, 0, s>>>(d, key_work, work_start, work_ctr, grain, least);
   } else {
     exclusive_scan_u64_dev(key_work, work_start, cap_keys, &c->keys[pipe], scan_tmp, s);
-    dense_plan_tail_kernel<<<1, kBlock, 0, s>>>(d, work_start, work_ctr, grain, fixed_grain);
+    dense_plan_tail_kernel<<<1, kBlock, 0, s>>>(d, work_start, work_ctr, grain, least);
   }
   SRD_CHECK(hipGetLastError());
 }
@@ -3452,7 +3453,7 @@ void dense_book(const DenseBook& b, hipStream_t s) {
 }
 
 void dense_emit(const DenseCtl* c, const DenseRel& r, hipStream_t s) {
-  dense_emit_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(c, r, false);
+  dense_emit_blocks_kernel<<<dim3(r.nblocks, dense_emit_parts(r)), kBlock, 0, s>>>(c, r, false);
   SRD_CHECK(hipGetLastError());
 }
 
@@ -3470,7 +3471,7 @@ void dense_index_count(const DenseRel& r, hipStream_t s) {
 }
 
 void dense_index_emit(const DenseRel& r, hipStream_t s) {
-  dense_emit_blocks_kernel<<<r.nblocks, kDenseWg, 0, s>>>(nullptr, r, true);
+  dense_emit_blocks_kernel<<<dim3(r.nblocks, dense_emit_parts(r)), kBlock, 0, s>>>(nullptr, r, true);
   SRD_CHECK(hipGetLastError());
 }
 

@@ -673,9 +673,7 @@ class PipelineGen:
          "  (void)drv_;",
          "  const uint64_t tw_ = DYN ? A.dyn->total_work : A.total_work;",
          "  const uint64_t ns_ = DYN ? A.dyn->n_slices : A.n_slices;",
-         "  const uint32_t gr_ = DYN ? A.dyn->grain : A.grain;",
-         "  // a block beyond the slices would only find every counter exhausted",
-         "  if (A.slice_lo + blockIdx.x * 4ull >= ns_) return;"]
+         "  const uint32_t gr_ = DYN ? A.dyn->grain : A.grain;"]
     for di in range(len(self.dests)):
       o.append(f"  const uint64_t ob{di}_ = DYN ? A.dyn->out_base[{di}] : A.out[{di}].base;")
     o += ["  const uint32_t lane = srd::lane_id();"]
@@ -744,8 +742,8 @@ class PipelineGen:
           "  uint64_t seg_start = ~uint64_t(0);",
           "  uint32_t seg_room = 0;",
           "  bool seg_dead = false;  // staging exhausted: count only (host re-runs the write pass)",
-          "  for (;;) {",
-          "    const uint64_t slice = srdj::next_slice(A, ns_);  // wave-uniform",
+          "  for (bool first_ = true;; first_ = false) {",
+          "    const uint64_t slice = srdj::next_slice(A, ns_, first_);  // wave-uniform",
           "    if (slice >= ns_) break;",
           "    const uint64_t it0 = A.slice_start ? A.slice_start[slice] : slice * gr_;",
           "    uint64_t it1 = A.slice_start ? A.slice_start[slice + 1]"

@@ -195,7 +195,7 @@ void dense_set_rows(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uin
   fail("dense_set_rows: not in the host-only build");
 }
 void dense_plan(DenseCtl*, SrdDyn*, uint32_t, const uint64_t*, uint64_t*, uint64_t, uint64_t*, uint32_t*,
-                uint32_t, bool, hipStream_t) {
+                uint32_t, uint32_t, hipStream_t) {
   fail("dense_plan: not in the host-only build");
 }
 void dense_count(const DenseCtl*, const DenseRel&, hipStream_t) { fail("dense_count: not in the host-only build"); }
