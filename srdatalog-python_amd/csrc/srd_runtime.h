@@ -191,6 +191,7 @@ struct Workspace {
   DevBuf<uint64_t> tile_scan;    // per-tile offsets
   DevBuf<uint8_t> flags;
   DevBuf<uint32_t> hostbuf_dev;  // staging for values read back
+  DevBuf<uint64_t> small_out;    // counts and maxima of a one-launch sort
   uint32_t epoch = 0;            // lookback epoch (avoids per-pass clears)
   DevBuf<uint64_t> mp_lb;        // merge-path set-difference inter-tile state
   DevBuf<uint64_t> mp_split;     // merge-path tile split points
