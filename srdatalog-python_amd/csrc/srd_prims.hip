@@ -29,6 +29,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -789,6 +790,126 @@ static void copy_out(uint8_t* dst, const uint8_t* src, uint64_t bytes, Workspace
   }
   SRD_CHECK(hipEventDestroy(ev[0]));
   SRD_CHECK(hipEventDestroy(ev[1]));
+}
+
+// Columns and maxima of row-major rows: each thread reads whole rows.
+template <int K>
+__global__ __launch_bounds__(kBlock) void deinterleave_kernel(const uint32_t* __restrict__ rows,
+                                                              uint64_t n, uint32_t k,
+                                                              uint32_t* __restrict__ cols,
+                                                              uint64_t stride,
+                                                              uint32_t* __restrict__ maxima) {
+  constexpr int KM = K ? K : 8;
+  const uint32_t kk = K ? uint32_t(K) : k;
+  uint32_t m[KM] = {};
+  for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n;
+       i += uint64_t(gridDim.x) * kBlock) {
+    if (K == 2) {
+      const uint2 v = reinterpret_cast<const uint2*>(rows)[i];
+      cols[i] = v.x;
+      cols[stride + i] = v.y;
+      m[0] = max(m[0], v.x);
+      m[KM > 1 ? 1 : 0] = max(m[KM > 1 ? 1 : 0], v.y);
+    } else {
+#pragma unroll
+      for (uint32_t c = 0; c < uint32_t(KM); ++c)
+        if (c < kk) {
+          const uint32_t v = rows[i * kk + c];
+          cols[uint64_t(c) * stride + i] = v;
+          m[c] = max(m[c], v);
+        }
+    }
+  }
+  __shared__ uint32_t s_m[kWavesPerBlock][KM];
+#pragma unroll
+  for (int c = 0; c < KM; ++c) {
+    const uint32_t v = wave_max(m[c]);
+    if (lane_id() == 0) s_m[threadIdx.x / kWave][c] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < kk) {
+    uint32_t v = 0;
+    for (int j = 0; j < kWavesPerBlock; ++j) v = max(v, s_m[j][threadIdx.x]);
+    atomicMax(&maxima[threadIdx.x], v);
+  }
+}
+
+// Pageable host memory to the device.  Up to eight threads each copy pieces
+// of 4 MiB into two pinned slots of their own and issue their DMA, so the
+// host copies run side by side and under the transfers; one pageable copy of
+// 126 MB took 20 ms, these 4 ms.
+static void copy_in(uint8_t* dst, const uint8_t* src, uint64_t bytes, Workspace& ws, hipStream_t s) {
+  constexpr uint64_t kPiece = uint64_t(4) << 20, kStage = uint64_t(128) << 20;
+  constexpr unsigned kMaxThreads = unsigned(kStage / (2 * kPiece)) / 2;
+  if (bytes <= kPiece) {
+    SRD_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+    SRD_CHECK(hipStreamSynchronize(s));
+    return;
+  }
+  if (!ws.stage_host)
+    ws.stage_host = static_cast<uint8_t*>(pinned_acquire(kStage, &ws.stage_host_bytes));
+  const uint64_t pieces = (bytes + kPiece - 1) / kPiece;
+  const unsigned hw = std::thread::hardware_concurrency();
+  const unsigned nt = unsigned(std::min<uint64_t>(
+      std::max(1u, std::min(kMaxThreads, hw ? hw / 2 : 4u)), pieces));
+  std::atomic<uint64_t> next{0};
+  std::atomic<int> bad{int(hipSuccess)};
+  int dev = 0;
+  SRD_CHECK(hipGetDevice(&dev));
+  auto work = [&](unsigned t) {
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    auto ok = [&](hipError_t e) {
+      if (e != hipSuccess) bad = int(e);
+      return e == hipSuccess;
+    };
+    uint8_t* slot = ws.stage_host + uint64_t(t) * 2 * kPiece;
+    if (ok(hipSetDevice(dev)) && ok(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming)) &&
+        ok(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming))) {
+      uint64_t used = 0;
+      for (uint64_t p; bad == int(hipSuccess) && (p = next++) < pieces; ++used) {
+        const uint64_t off = p * kPiece, len = std::min(kPiece, bytes - off);
+        uint8_t* q = slot + (used & 1) * kPiece;
+        if (used >= 2 && !ok(hipEventSynchronize(ev[used & 1]))) break;
+        std::memcpy(q, src + off, len);
+        if (!ok(hipMemcpyAsync(dst + off, q, len, hipMemcpyHostToDevice, s)) ||
+            !ok(hipEventRecord(ev[used & 1], s)))
+          break;
+      }
+    }
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+  };
+  std::vector<std::thread> th;
+  th.reserve(nt);
+  try {
+    for (unsigned t = 1; t < nt; ++t) th.emplace_back(work, t);
+  } catch (const std::system_error&) {
+    // fewer threads than asked for: those there are take all pieces
+  }
+  work(0);
+  for (auto& x : th) x.join();
+  const hipError_t done = hipStreamSynchronize(s);  // the slots are free again
+  SRD_CHECK(hipError_t(bad.load()));
+  SRD_CHECK(done);
+}
+
+void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>& out, uint64_t stride,
+                 std::vector<uint32_t>& maxima, Workspace& ws, hipStream_t s) {
+  if (k == 0 || k > 8) fail("upload_rows: arity must be in [1, 8]");
+  maxima.assign(k, 0);
+  if (n == 0) return;
+  out.alloc(stride * k, s);
+  DevBuf<uint32_t> raw(n * k, s), mx(8, s);
+  fill_u32(mx.p, 0, 8, s);
+  copy_in(reinterpret_cast<uint8_t*>(raw.p), reinterpret_cast<const uint8_t*>(rows), n * k * 4, ws, s);
+  const uint32_t g = grid_for(n, kBlock * 4, 4096);
+  if (k == 2) deinterleave_kernel<2><<<g, kBlock, 0, s>>>(raw.p, n, k, out.p, stride, mx.p);
+  else deinterleave_kernel<0><<<g, kBlock, 0, s>>>(raw.p, n, k, out.p, stride, mx.p);
+  SRD_CHECK(hipGetLastError());
+  uint32_t* h = pinned_words(ws, 8);
+  SRD_CHECK(hipMemcpyAsync(h, mx.p, 8 * 4, hipMemcpyDeviceToHost, s));
+  SRD_CHECK(hipStreamSynchronize(s));
+  for (uint32_t c = 0; c < k; ++c) maxima[c] = h[c];
 }
 
 void export_rows(const Index& x, uint32_t* host_out, const uint32_t* dev_bounds,

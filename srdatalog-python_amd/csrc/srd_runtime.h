@@ -352,6 +352,11 @@ void calib_copy(uint64_t bytes, int reps, hipStream_t s, double* ms_per_rep);
 void export_rows(const Index& x, uint32_t* host_out, const uint32_t* dev_bounds,
                  uint32_t n_bounds, Workspace& ws, hipStream_t s);
 
+// Row-major host rows to device columns (column c at out.p + c * stride) and
+// their maxima.  Returns once the rows are consumed.
+void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>& out, uint64_t stride,
+                 std::vector<uint32_t>& maxima, Workspace& ws, hipStream_t s);
+
 // out[g] = rows of the column-0-sorted column col0 (n rows) with value in
 // [bounds[g], bounds[g+1]), g < n_inst (bounds has n_inst+1 entries).
 void instance_counts(const uint32_t* col0, uint64_t n, const uint32_t* bounds, uint32_t n_inst,

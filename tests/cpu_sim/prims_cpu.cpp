@@ -188,6 +188,18 @@ void export_rows(const Index& x, uint32_t* host_out, const uint32_t* bounds, uin
   }
 }
 
+void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>& out, uint64_t stride,
+                 std::vector<uint32_t>& maxima, Workspace&, hipStream_t s) {
+  maxima.assign(k, 0);
+  if (n == 0) return;
+  out.alloc(stride * k, s);
+  for (uint64_t i = 0; i < n; ++i)
+    for (uint32_t c = 0; c < k; ++c) {
+      out.p[c * stride + i] = rows[i * k + c];
+      maxima[c] = std::max(maxima[c], rows[i * k + c]);
+    }
+}
+
 // Dense iterations need rules with device-sized mark launches, which the
 // host-only pipelines do not have.
 void dense_set_rows(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uint64_t*, uint8_t*,
