@@ -255,6 +255,7 @@ struct PipeScratch {
   DevBuf<uint64_t> recs, stage_ctr;
   DevBuf<uint64_t> item_cost, item_pref, slice_start;
   DevBuf<uint64_t> probe_buf;
+  DevBuf<uint32_t> uni_bits, uni_sum;  // unions of the rule's root keys (clear between runs)
 };
 
 }  // namespace srd
@@ -325,6 +326,9 @@ struct srd_engine {
   // SRDATALOG_MARK_PRODUCTS=0: the mark mode sets the bits of a product one
   // tuple at a time
   bool mark_products = true;
+  // SRDATALOG_MARK_UNION=0: products are walked per level-1 value, never per
+  // root key over the union of its values
+  bool mark_union = true;
   uint64_t mark_chunk_slices = 0;  // SRDATALOG_MARK_CHUNK_SLICES (0: one launch per traversal)
   uint32_t weigh_ranges = SRD_XCDS;  // SRDATALOG_WEIGH_RANGES: of the weigh launch
   // column-1 bitmaps of heavy keys for views nested levels search
@@ -801,6 +805,8 @@ static uint32_t stage_cols(const SrdPipelineDesc* d) {
 // runtime/generalized_datalog/gpu/runtime/stream_pool.h:18-89).
 struct PipeRun {
   const SrdPipelineDesc* d = nullptr;
+  const SrdPipelineDesc* t = nullptr;  // pipeline traversed: d, or its union pipeline
+  UnionProducts uni;                   // with a union pipeline: its products
   PipeScratch* x = nullptr;
   hipStream_t s = nullptr;
   SrdLaunchArgs a;
@@ -854,7 +860,8 @@ static bool stage_ready(srd_engine& e, PipeRun& R) {
 // wherever the rule reads DELTA), build the bitmaps and root maps they ask
 // for, pick the driver.
 static void pr_views(srd_engine& e, PipeRun& R, uint64_t iteration) {
-  const SrdPipelineDesc* d = R.d;
+  if (!R.t) R.t = R.d;
+  const SrdPipelineDesc* d = R.t;
   std::memset(&R.a, 0, sizeof(R.a));
   for (uint32_t v = 0; v < d->n_views; ++v) {
     const SrdViewSpec& vs = d->views[v];
@@ -920,7 +927,7 @@ static void pr_launch(srd_engine& e, PipeRun& R, SrdLaunchFn fn, const char* pha
 // Phase 2 (run stream): the root launch and the scan of the per-key work;
 // the work total is fetched.
 static void pr_root(srd_engine& e, PipeRun& R) {
-  const SrdPipelineDesc* d = R.d;
+  const SrdPipelineDesc* d = R.t;
   PipeScratch& x = *R.x;
   const uint64_t nk = R.a.n_root;
   x.key_rng.reserve(nk * 2 * SRD_MAX_VIEWS, R.s);
@@ -953,7 +960,7 @@ static void pr_root(srd_engine& e, PipeRun& R) {
 // nested levels the weigh launch -- every level-1 item's level-2 candidates
 // + SRD_ITEM_COST, prefix-summed -- whose total is fetched.
 static void pr_slices(srd_engine& e, PipeRun& R) {
-  const SrdPipelineDesc* d = R.d;
+  const SrdPipelineDesc* d = R.t;
   R.a.total_work = R.host[0];
   if (!e.grain_override)
     R.a.grain = srd_grain(R.a.total_work, d->default_grain, R.a.mark_prod == 1 ? SRD_PROD_GRAIN : 64u);
@@ -1033,7 +1040,7 @@ static void pr_weighed(srd_engine& e, PipeRun& R) {
 // the direct mode (one row per item), the count launch, or the fused launch
 // into staging -- with its total (and the staging overflow flag) fetched.
 static void pr_traverse(srd_engine& e, PipeRun& R) {
-  const SrdPipelineDesc* d = R.d;
+  const SrdPipelineDesc* d = R.t;
   PipeScratch& x = *R.x;
   if (e.trace) {
     std::fprintf(stderr, "[srd]   %s: keys %u drv %u work %llu slices %llu\n", d->rule, R.a.n_root,
@@ -1053,6 +1060,7 @@ static void pr_traverse(srd_engine& e, PipeRun& R) {
     const uint64_t step = e.mark_chunk_slices;
     if (!step || R.slices <= step) {
       pr_launch(e, R, d->mark, "mark");
+      if (R.t != R.d) union_products(R.uni, R.s);
       return;
     }
     for (uint64_t s0 = 0; s0 < R.slices; s0 += step) {
@@ -1069,6 +1077,7 @@ static void pr_traverse(srd_engine& e, PipeRun& R) {
     }
     R.a.slice_lo = 0;
     R.a.n_slices = R.slices;
+    if (R.t != R.d) union_products(R.uni, R.s);
     return;
   }
   x.counts_buf.reserve(R.slices, R.s);
@@ -1392,6 +1401,49 @@ static void pr_dense(srd_engine& e, std::vector<PipeRun*>& runs) {
   }
 }
 
+// Key space, in bits, of the largest bitmap of unions kept (2^34 bits are 2
+// GiB a rule).
+constexpr uint32_t kUnionBits = 34;
+
+// After pr_dense: a marking run whose rule has a union pipeline traverses
+// that one, into the scratch's bitmap, and multiplies the unions out
+// afterwards.  Without room for the bitmap the rule itself is traversed.
+static void pr_union(srd_engine& e, PipeRun& R, uint64_t iteration) {
+  if (!R.dense || !R.a.mark_prod || !e.mark_union) return;
+  const SrdPipelineExt* x = e.exts.find(R.d->rule)->second;
+  if (!x->uni) return;
+  PipeScratch& sc = *R.x;
+  const uint32_t sh = R.a.mark_shift;
+  if (2 * sh > kUnionBits) return;
+  const uint64_t words = std::max<uint64_t>((uint64_t(1) << (2 * sh)) / 32, kDenseBlockWords);
+  if (sc.uni_bits.n < words) {
+    const uint64_t bytes = e.dense_bytes - sc.uni_bits.n * 4 + words * 4;
+    if (bytes > e.device_bytes / 8) return;
+    e.dense_bytes = bytes;
+    sc.uni_bits.alloc(words, R.s);
+    fill_u32(sc.uni_bits.p, 0, words, R.s);
+    sc.uni_sum.alloc(dense_sum_words(words), R.s);
+    fill_u32(sc.uni_sum.p, 0, dense_sum_words(words), R.s);
+  }
+  const uint32_t k = R.d->dest[0].arity;
+  UnionProducts& u = R.uni;
+  u.bits = sc.uni_bits.p;
+  u.sum = reinterpret_cast<uint8_t*>(sc.uni_sum.p);
+  u.words = words;
+  u.ushift = sh;
+  u.minor = x->uni_minor;
+  u.row_shift = sh * (k - 1 - x->uni_row_col);
+  u.root_shift = x->uni_root_col >= 0 ? sh * (k - 1 - uint32_t(x->uni_root_col)) : 64u;
+  u.own = R.a.views.v[x->uni_view];
+  u.mark_bits = R.a.mark_bits;
+  u.mark_sum = R.a.mark_sum;
+  R.t = x->uni;
+  pr_views(e, R, iteration);
+  R.a.mark_bits = u.bits;
+  R.a.mark_sum = u.sum;
+  R.a.mark_shift = sh;
+}
+
 // Run pipelines -- one, or the members of a parallel group -- phase by
 // phase.  A group's members each get a stream and scratch of their own (a
 // member counting probes or needing the chunked or overflow path finishes
@@ -1435,6 +1487,7 @@ static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc
       {
         std::vector<PipeRun*> me{&R};
         pr_dense(e, me);
+        pr_union(e, R, iteration);
       }
       if (R.a.n_root > 0) {
         pr_root(e, R);
@@ -1473,6 +1526,7 @@ static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc
     std::vector<PipeRun*> all;
     for (auto& R : runs) all.push_back(&R);
     pr_dense(e, all);
+    for (auto& R : runs) pr_union(e, R, iteration);
   }
   // every member reads indexes built on the engine's stream (and the
   // bitmaps cleared there)
@@ -3464,6 +3518,7 @@ srd_engine* srd_engine_create_ext(const char* text, const SrdPipelineDesc* pipes
       e->xcd_ranges = std::min<uint32_t>(std::max<uint32_t>(uint32_t(std::atoi(c)), 1), SRD_XCDS);
     if (const char* c = std::getenv("SRDATALOG_MARK_CHUNK_SLICES"))
       e->mark_chunk_slices = std::strtoull(c, nullptr, 10);
+    if (const char* c = std::getenv("SRDATALOG_MARK_UNION")) e->mark_union = !(*c == '0' && c[1] == 0);
     if (const char* c = std::getenv("SRDATALOG_MARK_PRODUCTS"))
       e->mark_products = !(*c == '0' && c[1] == 0);
     if (const char* c = std::getenv("SRDATALOG_DENSE_MAX_BITS"))

@@ -173,14 +173,12 @@ __device__ __forceinline__ void prod_flush(const SrdLaunchArgs& A, uint64_t kb, 
   }
 }
 
-// Mark rows [r0, r1) of cr times the sorted values [mb, me) of cm: bit
-// kb + (row << rshift) + value.  lw / lm: 128 LDS words of the calling wave,
-// lm all zero on entry and left so.  Wave-uniform arguments, all 64 lanes.
-__device__ __forceinline__ void prod_mark(const SrdLaunchArgs& A, uint64_t kb, uint32_t rshift,
-                                          const uint32_t* __restrict__ cm, uint32_t mb, uint32_t me,
-                                          const uint32_t* __restrict__ cr, uint32_t r0, uint32_t r1,
-                                          uint32_t* lw, uint64_t* lm) {
-  if (r1 <= r0) return;
+// Fold the sorted values [mb, me) of cm into (word, mask) pairs and hand them
+// to flush(n), n <= 64 at a time, in lw / lm: 128 LDS words of the calling
+// wave, lm all zero on entry and left so.  Wave-uniform arguments, all 64 lanes.
+template <class F>
+__device__ __forceinline__ void fold_pairs(const uint32_t* __restrict__ cm, uint32_t mb, uint32_t me,
+                                           uint32_t* lw, uint64_t* lm, F&& flush) {
   const uint32_t lane = srd::lane_id();
   uint32_t n = 0, prev = ~0u;
   constexpr uint32_t L = 4;  // values loaded ahead, in 64s
@@ -191,10 +189,9 @@ __device__ __forceinline__ void prod_mark(const SrdLaunchArgs& A, uint64_t kb, u
       for (uint32_t i = 0; i < L; ++i)
         ahead[i] = pos + 64u * i + lane < me ? cm[pos + 64u * i + lane] : 0u;
     }
-    const uint32_t got = q == 0 ? ahead[0] : (q == 1 ? ahead[1] : (q == 2 ? ahead[2] : ahead[3]));
+    const uint32_t v = q == 0 ? ahead[0] : (q == 1 ? ahead[1] : (q == 2 ? ahead[2] : ahead[3]));
     const uint32_t cnt = min(64u, me - pos);
     const bool in = lane < cnt;
-    const uint32_t v = got;
     const uint32_t w = in ? v >> 6 : ~0u;
     uint32_t up = __shfl_up(w, 1, 64);
     if (lane == 0) up = prev;
@@ -211,7 +208,7 @@ __device__ __forceinline__ void prod_mark(const SrdLaunchArgs& A, uint64_t kb, u
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (n > 64) {  // 64 complete pairs; the last one may still grow
-      prod_flush(A, kb, rshift, cr, r0, r1, 64, lw, lm);
+      flush(64u);
       n -= 64;
       const uint32_t w2 = lw[64 + lane];
       const uint64_t m2 = lm[64 + lane];
@@ -223,11 +220,87 @@ __device__ __forceinline__ void prod_mark(const SrdLaunchArgs& A, uint64_t kb, u
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
   }
-  if (n) prod_flush(A, kb, rshift, cr, r0, r1, n, lw, lm);
+  if (n) flush(n);
   __builtin_amdgcn_wave_barrier();
   lm[lane] = 0;
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
+// Mark rows [r0, r1) of cr times the sorted values [mb, me) of cm: bit
+// kb + (row << rshift) + value (lw, lm: fold_pairs).
+__device__ __forceinline__ void prod_mark(const SrdLaunchArgs& A, uint64_t kb, uint32_t rshift,
+                                          const uint32_t* __restrict__ cm, uint32_t mb, uint32_t me,
+                                          const uint32_t* __restrict__ cr, uint32_t r0, uint32_t r1,
+                                          uint32_t* lw, uint64_t* lm) {
+  if (r1 <= r0) return;
+  fold_pairs(cm, mb, me, lw, lm,
+             [&](uint32_t n) { prod_flush(A, kb, rshift, cr, r0, r1, n, lw, lm); });
+}
+
+// Mark the sorted values [b, e) of col in the one row at bit kb (a multiple of
+// 64).  Thousands of items mark the row of a popular root key, from every
+// XCD: the words are read at device scope, past caches that would show them
+// clear, and set 64 bits at a time (bit by bit behind plain loads, the atomics
+// of one such row took 8 ms).
+__device__ __forceinline__ void run_mark(const SrdLaunchArgs& A, uint64_t kb,
+                                         const uint32_t* __restrict__ col, uint32_t b, uint32_t e,
+                                         uint32_t* lw, uint64_t* lm) {
+  const uint32_t lane = srd::lane_id();
+  uint64_t* row = reinterpret_cast<uint64_t*>(A.mark_bits) + (kb >> 6);
+  fold_pairs(col, b, e, lw, lm, [&](uint32_t n) {
+    if (lane < n) {
+      const uint32_t w = lw[lane];
+      const uint64_t m = lm[lane];
+      const uint64_t cur = __hip_atomic_load(row + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (m & ~cur) {
+        atomicOr(reinterpret_cast<unsigned long long*>(row + w), (unsigned long long)m);
+        mark_block(A, kb + (uint64_t(w) << 6));
+      }
+    }
+  });
+}
+
+// The same for the ranges of the lanes `mine`, all of one row, through their
+// keys' bitmaps (view v, lane's slot hb, first and last value of its range):
+// the bitmaps are OR-ed together 64 words at a time and the row is updated
+// once for all of them, one load per 64 words of a range of thousands.
+__device__ __forceinline__ void run_mark_bits(const SrdLaunchArgs& A, uint64_t kb, const IndexView& v,
+                                              uint64_t mine, uint32_t hb, uint32_t first, uint32_t last) {
+  const uint32_t lane = srd::lane_id();
+  const bool in = (mine >> lane) & 1u;
+  const uint32_t hi = srd::wave_max(in ? last >> 6 : 0u);
+  const uint32_t lo = ~srd::wave_max(in ? ~(first >> 6) : 0u);
+  uint64_t* row = reinterpret_cast<uint64_t*>(A.mark_bits) + (kb >> 6);
+  const uint64_t* bm = reinterpret_cast<const uint64_t*>(v.bm);
+  const uint64_t bw = v.bm_words >> 1;
+  constexpr uint32_t U = 4;
+  for (uint32_t w0 = lo; w0 <= hi; w0 += 64) {
+    const uint32_t w = w0 + lane;
+    const bool on = w <= hi && w < bw;
+    uint64_t acc = 0;
+    for (uint64_t m = mine; m;) {
+      uint64_t x[U];
+#pragma unroll
+      for (uint32_t q = 0; q < U; ++q) {
+        // past the last range: the one before again
+        const uint32_t o = uint32_t(__builtin_ctzll(m));
+        x[q] = on ? bm[uint64_t(__builtin_amdgcn_readlane(hb, o)) * bw + w] : 0;
+        const uint64_t rest = m & (m - 1);
+        if (q + 1 < U && rest) m = rest;
+      }
+      m &= m - 1;
+#pragma unroll
+      for (uint32_t q = 0; q < U; ++q) acc |= x[q];
+    }
+    if (acc) {
+      const uint64_t cur = __hip_atomic_load(row + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (acc & ~cur) {
+        atomicOr(reinterpret_cast<unsigned long long*>(row + w), (unsigned long long)acc);
+        mark_block(A, kb + (uint64_t(w) << 6));
+      }
+    }
+  }
 }
 
 // Row r of nr at the part num/den of a product's cost: cuts at equal costs

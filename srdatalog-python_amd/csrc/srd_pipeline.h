@@ -258,6 +258,16 @@ struct SrdPipelineExt {
   // second level, whose items are weighed, 3 = a deeper one, 0 = no such level
   uint32_t mark_prod;
   SrdLaunchFn mark_dyn;   // device-sized mark mode; nullptr outside recursive steps
+  // two-level rules whose product splits into a source that depends on the
+  // level-1 variable and one (view uni_view, its column 1) that depends on
+  // the root key alone: the pipeline that derives (root key, value of the
+  // first), marked in a bitmap of its own and multiplied out by
+  // union_products.  uni_minor: the first source's variable is the
+  // destination's last column (else its row column); uni_row_col, uni_root_col:
+  // index columns of the row variable and, or -1, of the root variable.
+  const struct SrdPipelineDesc* uni;
+  uint32_t uni_view, uni_minor, uni_row_col;
+  int32_t uni_root_col;
 };
 
 #ifdef __cplusplus

@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "srd_devloop.h"
+#include "srd_join.h"
 #include "srd_runtime.h"
 
 namespace srd {
@@ -633,7 +634,7 @@ void build_heavy_bitmaps(const Index& x, uint32_t min_len, uint64_t max_bytes, W
   h.built_for = x.cols.p;
   h.built_n = x.n;
   if (x.arity != 2 || x.r == 0 || x.col_max.size() < 2 || max_bytes == 0) return;
-  const uint32_t words = (x.col_max[1] >> 5) + 1;
+  const uint32_t words = ((x.col_max[1] >> 5) + 2) & ~1u;  // whole 64-bit words
   DevBuf<uint32_t> flag(x.r, s), ends;
   DevBuf<uint64_t> pos(uint64_t(x.r) + 1, s);
   for (;;) {
@@ -3491,6 +3492,120 @@ void dl_inst(const DevCtl* c, uint32_t r, const uint32_t* col0, const uint32_t* 
   SRD_CHECK(hipGetLastError());
 }
 
+
+// ================================================ products of unions ====
+// One workgroup column (blockIdx.x) per root key, kUnionParts workgroups a
+// key; every wave takes its share of the rows (minor) or of U's words.
+// What bounds it is the latency of a wave's word loads; the unions themselves
+// are marked by the rule's union pipeline.  Andersen at 1/10: the four rules'
+// products, walked per (key, level-1 value) before, took 169 ms of kernel
+// time a fixpoint, these 20 ms and the union marking 9 ms.
+constexpr uint32_t kUnionParts = 4;
+
+__global__ __launch_bounds__(kBlock) void union_products_kernel(UnionProducts u) {
+  __shared__ uint32_t s_w[kWavesPerBlock][128], s_rows[kWavesPerBlock][128];
+  __shared__ uint64_t s_m[kWavesPerBlock][128];
+  const uint32_t wv = threadIdx.x / kWave, l = lane_id();
+  uint32_t* lw = s_w[wv];
+  uint64_t* lm = s_m[wv];
+  uint32_t* rows = s_rows[wv];
+  lm[l] = lm[64 + l] = 0;
+  SrdLaunchArgs A;
+  A.mark_bits = u.mark_bits;
+  A.mark_sum = u.mark_sum;
+  const uint64_t* bits = reinterpret_cast<const uint64_t*>(u.bits);
+  const uint32_t nwords = uint32_t((uint64_t(1) << u.ushift) >> 6);
+  const uint32_t share = blockIdx.y * kWavesPerBlock + wv, shares = kUnionParts * kWavesPerBlock;
+  const uint32_t* c1 = u.own.cols + u.own.stride;
+  for (uint32_t g = blockIdx.x; g < u.own.r; g += gridDim.x) {
+    const uint32_t key = u.own.root_vals[g];
+    const uint64_t kb64 = uint64_t(key) << u.ushift;
+    // (a row's blocks: more than one only for rows beyond 2^18 values)
+    if (!u.sum[kb64 >> 18] && u.ushift <= 18) continue;
+    const uint32_t b = u.own.root_offs[g], e = u.own.root_offs[g + 1];
+    const uint64_t kb = u.root_shift < 64 ? uint64_t(key) << u.root_shift : 0;
+    const uint64_t* row = bits + (kb64 >> 6);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (u.minor) {
+      // rows: own values of this wave's share; pairs: U's non-zero words
+      const uint32_t r0 = b + uint32_t(uint64_t(e - b) * share / shares);
+      const uint32_t r1 = b + uint32_t(uint64_t(e - b) * (share + 1) / shares);
+      if (r0 == r1) continue;
+      uint32_t n = 0;
+      for (uint32_t w0 = 0; w0 < nwords; w0 += kWave) {
+        const uint64_t x = w0 + l < nwords ? row[w0 + l] : 0;
+        const uint64_t nz = ballot(x != 0);
+        if (x) {
+          const uint32_t at = n + popc_below(nz);
+          lw[at] = w0 + l;
+          lm[at] = x;
+        }
+        n += uint32_t(__popcll(nz));
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if (n >= 64) {
+          srdj::prod_flush(A, kb, u.row_shift, c1, r0, r1, 64, lw, lm);
+          n -= 64;
+          const uint32_t w2 = lw[64 + l];
+          const uint64_t m2 = lm[64 + l];
+          __builtin_amdgcn_wave_barrier();
+          lw[l] = w2;
+          lm[l] = m2;
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+      }
+      if (n) srdj::prod_flush(A, kb, u.row_shift, c1, r0, r1, n, lw, lm);
+    } else {
+      // pairs: own values, folded once; rows: U's values in this wave's share
+      // of its words, 64 and more at a time
+      srdj::fold_pairs(c1, b, e, lw, lm, [&](uint32_t np) {
+        uint32_t n = 0;
+        auto out = [&] {
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+          srdj::prod_flush(A, kb, u.row_shift, rows, 0, n, np, lw, lm);
+          __builtin_amdgcn_wave_barrier();
+          n = 0;
+        };
+        for (uint32_t w0 = share * kWave; w0 < nwords; w0 += shares * kWave) {
+          const uint64_t x = w0 + l < nwords ? row[w0 + l] : 0;
+          for (uint64_t nz = ballot(x != 0); nz; nz &= nz - 1) {
+            const int j = __builtin_ctzll(nz);
+            const uint64_t xj = read_lane_u64(x, j);
+            if ((xj >> l) & 1u) rows[n + popc_below(xj)] = ((w0 + uint32_t(j)) << 6) + l;
+            n += uint32_t(__popcll(xj));
+            if (n >= 64) out();
+          }
+        }
+        if (n) out();
+      });
+    }
+  }
+}
+
+// Zero the marked blocks of a bitmap and their bytes.
+__global__ __launch_bounds__(kBlock) void clear_blocks_kernel(uint4* bits, uint8_t* sum) {
+  const uint64_t b = blockIdx.x;
+  const bool on = sum[b] != 0;
+  __syncthreads();
+  if (!on) return;
+  for (uint32_t i = threadIdx.x; i < kDenseBlockWords / 4; i += kBlock)
+    bits[b * (kDenseBlockWords / 4) + i] = uint4{0, 0, 0, 0};
+  if (threadIdx.x == 0) sum[b] = 0;
+}
+
+void union_products(const UnionProducts& u, hipStream_t s) {
+  if (u.own.r == 0) return;
+  if (u.own.arity < 2 || u.ushift < 6) fail("union_products: bad operand");
+  TimeScope t("join.union_products", s);
+  union_products_kernel<<<dim3(std::min<uint32_t>(u.own.r, 8192), kUnionParts), kBlock, 0, s>>>(u);
+  SRD_CHECK(hipGetLastError());
+  clear_blocks_kernel<<<uint32_t(u.words / kDenseBlockWords), kBlock, 0, s>>>(
+      reinterpret_cast<uint4*>(u.bits), u.sum);
+  SRD_CHECK(hipGetLastError());
+}
 
 // ================================================== dense iterations ====
 // A block of 2^18 keys is 4096 words of 64 keys: 64 chunks of one word per

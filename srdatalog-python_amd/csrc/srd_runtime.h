@@ -325,6 +325,25 @@ inline uint64_t dense_sum_words(uint64_t words) { return (words / kDenseBlockWor
 uint64_t dense_extract(uint32_t* bits, uint32_t* sum, uint64_t words, uint32_t k, uint32_t shift,
                        DevBuf<uint32_t>& out, uint64_t& stride, Workspace& ws, hipStream_t s);
 
+// Products of the unions a union pipeline marked (SrdPipelineExt::uni): for
+// every root key r of `own`, U[r] x own's column-1 values under r into the
+// destination's bitmap (kernel args of its mark mode), then U cleared.
+// U: 2^(2 * ushift) bits, value d of key r at bit (r << ushift) + d, and its
+// block bytes.
+struct UnionProducts {
+  uint32_t* bits;        // U
+  uint8_t* sum;
+  uint64_t words;        // u32 words of U
+  uint32_t ushift;
+  uint32_t minor;        // U holds last-column values (else row values)
+  uint32_t row_shift;    // bit shifts of the row variable and of the root
+  uint32_t root_shift;   // variable in the destination's key (64: not in it)
+  IndexView own;
+  uint32_t* mark_bits;   // the destination's bitmap
+  uint8_t* mark_sum;
+};
+void union_products(const UnionProducts& u, hipStream_t s);
+
 // Fill n words with value (a kernel, safe under stream capture).
 void fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 void fill_u64(uint64_t* p, uint64_t value, uint64_t n, hipStream_t s);

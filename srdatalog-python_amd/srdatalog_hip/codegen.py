@@ -79,8 +79,10 @@ class PipelineGen:
 
   def __init__(self, ep: M.ExecutePipeline, arity: dict[str, int], uid: int,
                coop_search: bool = False, ring: bool = True, dyn: bool = False,
-               cart_tiles: bool = True):
+               cart_tiles: bool = True, only_mark: bool = False):
     self.ep = ep
+    # a union rule (union_gen): root, weigh and mark launches only
+    self.only_mark = only_mark
     # large two-source cartesian products at a nested last level are walked
     # in register tiles instead of the flattened per-item decode
     self.cart_tiles = cart_tiles
@@ -273,6 +275,38 @@ class PipelineGen:
     return {"jm": jm, "jr": 1 - jm, "cr": row.index(cart[1 - jm]),
             "bound": [(c, v) for c, v in enumerate(row) if v not in cart], "k": len(row)}
 
+  def union_gen(self) -> "PipelineGen | None":
+    """The rule's union pipeline, or None: with root variable r, level-1
+    variable l and a product of a source that depends on l (its variable d)
+    and one that depends on r alone, and l not in the head, the tuples of a
+    root key are (union over l of the first source's values) x (the second
+    source's).  The union pipeline derives the pairs (r, d); marked in a bitmap
+    they are the unions, and union_products multiplies them out, once per
+    root key instead of once per (r, l)."""
+    if self.only_mark or len(self.levels) != 2:
+      return None
+    r, lv1, lv2 = self.root, *self.levels
+    p = self.prod_level(lv2)
+    if not p or not isinstance(lv1, M.ColumnJoin) or any(v != r.var for _, v in p["bound"]):
+      return None
+    dep = [lv1.var in s_.prefix for s_ in lv2.sources]
+    if dep[0] == dep[1]:
+      return None
+    jd = dep.index(True)
+    own = lv2.sources[1 - jd]
+    if list(own.prefix) != [r.var] or len(own.index) < 2:
+      return None
+    vd = lv2.var_from_source[jd][0]
+    if vd in (r.var, lv1.var):
+      return None
+    ep = M.ExecutePipeline(rule=self.ep.rule, ops=[
+      r, lv1, *self.filters,
+      M.CartesianJoin(vars=[vd], var_from_source=[[vd]], sources=[lv2.sources[jd]]),
+      M.InsertInto(rel=self.dests[0].rel, ver=self.dests[0].ver, index=[0, 1], terms=[r.var, vd])])
+    g = PipelineGen(ep, self.arity, 0, only_mark=True, ring=False, cart_tiles=False)
+    g.ns = self.ns + "_union"
+    return g
+
   def prod_base(self, p: dict, get) -> str:
     """Bit of the product's tuple with zero row and last column: the bound
     variables at their index columns."""
@@ -324,9 +358,17 @@ class PipelineGen:
     last column, so a membership bitmap can replace the search."""
     return (not r.full0 and not r.uniform and r.depth == 1 and self.view_arity(r.view) == 2)
 
+  def union_bitmaps(self) -> bool:
+    """A union rule whose values are the last column of a two-column view
+    below its level-1 key: a long range's bitmap stands for its list."""
+    s_ = self.levels[1].sources[0]
+    return len(s_.prefix) == 1 and self.view_arity(self.vid(s_)) == 2
+
   def bm_views(self) -> set:
     """Views that the second level of the join searches at depth 1."""
     out = set()
+    if self.only_mark:
+      return {self.vid(self.levels[1].sources[0])} if self.union_bitmaps() else out
     for lv in self.levels[1:2]:
       for s_ in lv.sources:
         if len(s_.prefix) == 1 and self.view_arity(self.vid(s_)) == 2:
@@ -721,7 +763,7 @@ class PipelineGen:
             "  };"]
     slots = self.root_slots()
     ns = len(slots)
-    if any(self.prod_level(lv) for lv in self.levels[-1:]):
+    if self.only_mark or any(self.prod_level(lv) for lv in self.levels[-1:]):
       o += ["  // mark mode: the (word, mask) pairs of the product being walked",
             "  uint32_t* lw_ = nullptr;",
             "  uint64_t* lm_ = nullptr;",
@@ -1008,6 +1050,31 @@ class PipelineGen:
                f"max(uint32_t({sizes[0]}), uint32_t({sizes[1]})) >= SRD_CART_TILE_DIM"
                + (" && !(MODE == 6 && A.mark_prod)" if p else "") + ";")
       o.append(f"{ind}if (big{t}) sz{t} = 0;")
+    if self.only_mark and li == 1 and isinstance(lv, M.CartesianJoin) and not rngs[0].full0:
+      # long ranges of the union rule: the wave marks them one owner at a time
+      r0, vr = rngs[0], self.var(self.dests[0].terms[0])
+      rl = lambda v: f"__builtin_amdgcn_readlane({v}, ow_)"
+      o += [f"{ind}if constexpr (MODE == 6) {{",
+            f"{ind}  const bool long_ = {hvar} && sz{t} >= 64;",
+            f"{ind}  if (long_) sz{t} = 0;",
+            *([f"{ind}  const uint32_t hs_ = (long_ && V.v[{r0.view}].n_hv && {r0.e} - {r0.b} >= "
+               f"V.v[{r0.view}].bm_min) ? srdj::heavy_slot(V.v[{r0.view}], {r0.b}) : ~0u;",
+               f"{ind}  const uint32_t hf_ = hs_ != ~0u ? {self.col_expr(r0.view, r0.depth)}[{r0.b}] : 0u;",
+               f"{ind}  const uint32_t hl_ = hs_ != ~0u ? {self.col_expr(r0.view, r0.depth)}[{r0.e} - 1] : 0u;",
+               f"{ind}  for (uint64_t bh_ = srd::ballot(hs_ != ~0u); bh_;) {{",
+               f"{ind}    const uint32_t ow_ = uint32_t(__builtin_ctzll(bh_));",
+               f"{ind}    const uint64_t mine_ = srd::ballot(hs_ != ~0u && {vr} == {rl(vr)}) & bh_;",
+               f"{ind}    bh_ &= ~mine_;",
+               f"{ind}    srdj::run_mark_bits(A, uint64_t({rl(vr)}) << A.mark_shift, V.v[{r0.view}], mine_, hs_, hf_, hl_);",
+               f"{ind}  }}",
+               f"{ind}  const bool list_ = long_ && hs_ == ~0u;"]
+              if self.union_bitmaps() else [f"{ind}  const bool list_ = long_;"]),
+            f"{ind}  for (uint64_t bl_ = srd::ballot(list_); bl_; bl_ &= bl_ - 1) {{",
+            f"{ind}    const uint32_t ow_ = uint32_t(__builtin_ctzll(bl_));",
+            f"{ind}    srdj::run_mark(A, uint64_t({rl(vr)}) << A.mark_shift, "
+            f"{self.col_expr(r0.view, r0.depth)}, {rl(f'uint32_t({r0.b})')}, {rl(f'uint32_t({r0.e})')}, lw_, lm_);",
+            f"{ind}  }}",
+            f"{ind}}}"]
     o += bm_code
     o.append(f"{ind}const uint64_t inc{t} = srd::wave_incl_scan<uint64_t>(sz{t});")
     o.append(f"{ind}const uint64_t tot{t} = srdj::uniform_from(inc{t}, 63);")
@@ -1233,6 +1300,21 @@ class PipelineGen:
 
   # --------------------------------------------------------- assembly ----
   def gen_kernels(self) -> str:
+    if self.only_mark:
+      return "\n".join([
+          f"namespace {self.ns} {{", self.gen_root(), "", self.gen_run(), "",
+          "void launch_root(const SrdLaunchArgs* a, hipStream_t s) {",
+          "  root_k<false><<<(a->n_root + 255u) / 256u, 256, 0, s>>>(*a);",
+          "}",
+          "void launch_mark(const SrdLaunchArgs* a, hipStream_t s) {",
+          "  run_k<6, false><<<a->grid_blocks, 256, 0, s>>>(*a);",
+          "}",
+          "void launch_weigh(const SrdLaunchArgs* a, hipStream_t s) {",
+          "  run_k<4, false><<<a->grid_blocks, 256, 0, s>>>(*a);",
+          "}",
+          "static const SrdPipelineDesc k_desc =",
+          self.gen_desc() + ";",
+          f"}}  // namespace {self.ns}", ""])
     out = [f"namespace {self.ns} {{", self.gen_root(), "", self.gen_run(), "",
            "void launch_root(const SrdLaunchArgs* a, hipStream_t s) {",
            "  root_k<false><<<(a->n_root + 255u) / 256u, 256, 0, s>>>(*a);",
@@ -1286,7 +1368,16 @@ class PipelineGen:
 
   def gen_ext(self) -> str:
     dyn = f"&{self.ns}::launch_mark_dyn" if self.dyn and self.mark_ok() else "nullptr"
-    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}, {dyn}}}"
+    uni = "nullptr, 0, 0, 0, -1"
+    g = self.union_gen()
+    if g:
+      lv = self.levels[1]
+      p = self.prod_level(lv)
+      minor = self.levels[0].var in lv.sources[p["jm"]].prefix
+      own = lv.sources[p["jr"] if minor else p["jm"]]
+      root = p["bound"][0][0] if p["bound"] else -1
+      uni = f"&{g.ns}::k_desc, {self.vid(own)}, {1 if minor else 0}, {p['cr']}, {root}"
+    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}, {dyn}, {uni}}}"
 
   def gen_desc(self) -> str:
     views = []
@@ -1309,7 +1400,12 @@ class PipelineGen:
             f"{len(roots)}, {{{', '.join(str(r) for r in roots)}}}, {len(dests)}, "
             f"{{{', '.join(dests)}}}, {1 if self.ep.count else 0}, {grain}, "
             f"{1 if self.direct_ok() else 0}, "
-            f"&{self.ns}::launch_root, &{self.ns}::launch_count, &{self.ns}::launch_write, "
+            + (f"&{self.ns}::launch_root, nullptr, nullptr, nullptr, nullptr, &{self.ns}::launch_weigh, 0, "
+               f"nullptr, nullptr, nullptr, nullptr, nullptr, &{self.ns}::launch_mark}}"
+               if self.only_mark else self.gen_launches()))
+
+  def gen_launches(self) -> str:
+    return (f"&{self.ns}::launch_root, &{self.ns}::launch_count, &{self.ns}::launch_write, "
             f"&{self.ns}::launch_fused, &{self.ns}::launch_direct, "
             f"{'&' + self.ns + '::launch_weigh' if len(self.levels) >= 2 else 'nullptr'}, "
             f"{1 if self.sorted_output() else 0}, &{self.ns}::launch_probe, "
@@ -1549,6 +1645,9 @@ def generate_program_source(name: str, decls: list[RelDecl], prog: M.Program) ->
          ""]
   for g in gens:
     out.append(g.gen_kernels())
+    u = g.union_gen()
+    if u:
+      out.append(u.gen_kernels())
   out.append("static const SrdPipelineDesc k_pipes[] = {")
   out.append(",\n".join(g.gen_desc() for g in gens) if gens else "")
   out.append("};")

@@ -200,6 +200,8 @@ void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>&
     }
 }
 
+void union_products(const UnionProducts&, hipStream_t) { fail("union_products: not in the host-only build"); }
+
 // Dense iterations need rules with device-sized mark launches, which the
 // host-only pipelines do not have.
 void dense_set_rows(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uint64_t*, uint8_t*,
