@@ -2,23 +2,15 @@
 //
 // Callers that cannot call hipMalloc -- code under HIP graph capture, tight
 // serving loops, harnesses that forbid allocation -- pass device columns in
-// and device buffers out; every intermediate (packed keys in two buffers,
-// digit histograms, the radix passes' look-back words, dedup tile counts,
-// the device-side plan) lives in `scratch`, a file-scope device array of
-// kNoAllocScratchBytes that each GPU the library runs on holds until the
-// process ends.  The sort is the device-planned radix sort + dedup
-// (build_index_dev): row count, key layout and pass schedule are decided by
-// kernels, so the call enqueues a fixed launch sequence and never reads
-// anything back.
+// and device buffers out; every intermediate (rows in buckets, run and
+// splitter tables, look-back words) lives in `scratch`, a file-scope device
+// array of kNoAllocScratchBytes that each GPU the library runs on holds until
+// the process ends.  The sort is build_index_dev's: one launch up to 4,096
+// rows, two up to kNoAllocMaxRows, nothing read back, and every table cleared
+// by the call that uses it, so a captured call can be replayed.
 //
-// The scratch is always carved for kNoAllocMaxRows rows whatever n is, so
-// its look-back words sit at fixed addresses and are only ever written as
-// look-back words; a new look-back epoch per pass (a counter kept in the
-// scratch and advanced by a kernel) makes the words of earlier calls read as
-// "not yet published", and the words are cleared by a kernel at set-up and
-// whenever the 16-bit epoch wraps.  Every call on a GPU
-// shares that GPU's array: calls that overlap on one GPU (two streams, two
-// threads) race on it.
+// Every call on a GPU shares that GPU's array: calls that overlap on one GPU
+// (two streams, two threads) race on it.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -34,7 +26,7 @@ void capi_set_error(const std::string& msg);
 
 namespace {
 constexpr uint64_t kNoAllocMaxRows = uint64_t(1) << 20;
-// devsort_scratch_bytes(2^20) = 34,643,712 bytes (checked at set-up)
+// devsort_scratch_bytes(2^20) = 34,096,384 bytes (checked at set-up)
 constexpr uint64_t kNoAllocScratchBytes = uint64_t(34) << 20;
 constexpr int kNoAllocMaxDevices = 64;
 }  // namespace
@@ -49,8 +41,8 @@ std::mutex g_na_mu;
 void* g_na_ptr[kNoAllocMaxDevices] = {};
 
 // Device address of `scratch` on the current device `dev`, resolved once per
-// device; the first call also clears the look-back words on stream s.
-void* noalloc_scratch(int dev, hipStream_t s) {
+// device.
+void* noalloc_scratch(int dev) {
   if (g_na_ptr[dev]) return g_na_ptr[dev];
   if (srd::devsort_scratch_bytes(kNoAllocMaxRows) > kNoAllocScratchBytes)
     throw std::runtime_error("srd_prim_sort_dedup_noalloc: scratch array smaller than the sort needs");
@@ -59,7 +51,6 @@ void* noalloc_scratch(int dev, hipStream_t s) {
   if (e != hipSuccess || !p)
     throw std::runtime_error(std::string("srd_prim_sort_dedup_noalloc: hipGetSymbolAddress failed: ") +
                              hipGetErrorString(e));
-  srd::devsort_clear_lookback(p, kNoAllocMaxRows, s);
   g_na_ptr[dev] = p;
   return p;
 }
@@ -87,7 +78,7 @@ extern "C" int srd_prim_sort_dedup_noalloc(const uint32_t* cols, uint64_t stride
     const uint32_t* in[4] = {};
     for (uint32_t c = 0; c < k; ++c) in[c] = cols + uint64_t(c) * stride;
     std::lock_guard<std::mutex> g(g_na_mu);
-    void* sp = noalloc_scratch(dev, s);
+    void* sp = noalloc_scratch(dev);
     // w = 1 holds any two 32-bit columns; three or four need two key words
     srd::build_index_dev(in, k, kNoAllocMaxRows, nullptr, n, k <= 2 ? 1u : 2u, sp, out_cols,
                          out_stride, root_vals, root_offs, counts, /*ticket=*/true, s,

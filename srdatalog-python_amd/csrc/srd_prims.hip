@@ -13,7 +13,9 @@
 //    offset with a decoupled look-back over earlier tiles, then writes its
 //    keys from an LDS-sorted copy so that each digit run is a coalesced
 //    store.  Tile order is the block id when the run is alone on the GPU and
-//    a ticket from an atomic counter when other runs may share it.
+//    a ticket from an atomic counter when other runs may share it.  Up to
+//    4,096 rows are sorted by one workgroup in one launch, up to 2^20 in two
+//    (buckets between sampled splitters, each sorted in LDS).
 //  * dedup unpacks the sorted keys straight into the index columns and
 //    emits the distinct column-0 values with their row offsets in the same
 //    pass.
@@ -1236,6 +1238,44 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid) {
   return m;
 }
 
+// Inclusive scan over the whole wave in DPP moves (a shuffle through LDS costs
+// several times one); every lane must be active.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_scan32(uint32_t v, uint32_t id, Op op) {
+#define SRD_DPP(CTRL, ROWS) \
+  v = op(v, uint32_t(__builtin_amdgcn_update_dpp(int(id), int(v), CTRL, ROWS, 0xF, false)))
+  SRD_DPP(0x111, 0xF);  // row_shr 1, 2, 4, 8
+  SRD_DPP(0x112, 0xF);
+  SRD_DPP(0x114, 0xF);
+  SRD_DPP(0x118, 0xF);
+  SRD_DPP(0x142, 0xA);  // row_bcast 15 into rows 1 and 3
+  SRD_DPP(0x143, 0xC);  // row_bcast 31 into rows 2 and 3
+#undef SRD_DPP
+  return v;
+}
+
+__device__ __forceinline__ uint32_t wave_add32(uint32_t v) {
+  return __builtin_amdgcn_readlane(wave_scan32(v, 0, [](uint32_t a, uint32_t b) { return a + b; }), 63);
+}
+__device__ __forceinline__ uint32_t wave_max32(uint32_t v) {
+  return __builtin_amdgcn_readlane(wave_scan32(v, 0, [](uint32_t a, uint32_t b) { return max(a, b); }), 63);
+}
+__device__ __forceinline__ uint32_t wave_min32(uint32_t v) { return ~wave_max32(~v); }
+
+// block_excl_scan with DPP scans and one barrier: `wsum` is not read after the
+// call's own reads, and must not be written again before the next barrier.
+template <int NW>
+__device__ __forceinline__ uint32_t block_scan32(uint32_t v, uint32_t* wsum) {
+  const uint32_t inc = wave_scan32(v, 0, [](uint32_t a, uint32_t b) { return a + b; });
+  const uint32_t w = threadIdx.x / kWave;
+  if (lane_id() == kWave - 1) wsum[w] = inc;
+  __syncthreads();
+  uint32_t base = 0;
+#pragma unroll
+  for (int i = 0; i < NW - 1; ++i) base += uint32_t(i) < w ? wsum[i] : 0;
+  return base + inc - v;
+}
+
 // Decoupled look-back by one whole wave: the 64 lanes read the status words
 // of the 64 tiles before `tile` at once (lane 0 the nearest), wait until every
 // word up to the nearest inclusive prefix is published, and add the
@@ -1266,8 +1306,9 @@ __device__ __forceinline__ uint64_t wave_lookback(uint64_t* base, uint64_t strid
       __builtin_amdgcn_s_sleep(1);
       continue;
     }
+    // counts of 46 bits, summed in two halves that 64 lanes cannot overflow
     const uint64_t mine = ((need >> l) & 1ull) ? (v & kLbMask) : 0;
-    excl += wave_sum<uint64_t>(mine);
+    excl += uint64_t(wave_add32(uint32_t(mine) & ((1u << 23) - 1))) + (uint64_t(wave_add32(uint32_t(mine >> 23))) << 23);
     if (pm) break;
     hi -= 64;
   }
@@ -1609,13 +1650,371 @@ __global__ __launch_bounds__(kBlock) void dedup_write_kernel(
   }
 }
 
+// ================================================= sort: in one workgroup ====
+// Rows as raw keys: column c of k is the 32-bit field k-1-c of a 64-bit key
+// (W = 1, k <= 2) or a 128-bit one (W = 2), field 0 lowest.
+template <int W>
+__device__ __forceinline__ uint32_t key_field(uint64_t lo, uint64_t hi, uint32_t f) {
+  const uint64_t v = W == 2 && f >= 2 ? hi : lo;
+  return uint32_t(f & 1u ? v >> 32 : v);
+}
+
+template <int W>
+__device__ __forceinline__ void raw_key(const uint32_t* const* in, uint32_t k, uint64_t row,
+                                        uint64_t& lo, uint64_t& hi) {
+  lo = hi = 0;
+#pragma unroll
+  for (uint32_t c = 0; c < 2u * W; ++c) {
+    if (c >= k) continue;
+    const uint32_t f = k - 1 - c;
+    const uint64_t v = uint64_t(in[c][row]) << (f & 1u ? 32 : 0);
+    if (W == 2 && f >= 2) hi |= v;
+    else lo |= v;
+  }
+}
+
+template <int W>
+__device__ __forceinline__ bool key_le(uint64_t al, uint64_t ah, uint64_t bl, uint64_t bh) {
+  if (W == 1) return al <= bl;
+  return ah < bh || (ah == bh && al <= bl);
+}
+
+template <int W, int BT, int ITEMS>
+struct SortMem {
+  static constexpr int kWaves = BT / kWave;
+  uint64_t key[W][BT * ITEMS];
+  alignas(16) uint32_t wcnt[kWaves][kRadix];
+  uint32_t local[kRadix];
+  uint32_t wsum[kWaves];
+  uint32_t least[2 * W], most[2 * W];  // of each field
+  uint64_t diff[2][kWaves];
+  uint32_t firsts[ITEMS * kWaves];  // per wave and item: rows | roots << 16
+};
+
+// Position of item i of this thread among the rows of a workgroup: wave,
+// item, lane, `items` items a thread.
+__device__ __forceinline__ uint32_t row_pos(uint32_t items, uint32_t i) {
+  return ((threadIdx.x / kWave) * items + i) * kWave + lane_id();
+}
+
+// Stable LSD passes over the low `total` bits of a PW-word key.
+template <int PW, int W, int BT, int ITEMS>
+__device__ __forceinline__ void block_passes(uint64_t (&lo)[ITEMS], uint64_t (&hi)[ITEMS], uint32_t m,
+                                             uint32_t items, uint32_t total,
+                                             SortMem<W, BT, ITEMS>& sm) {
+  constexpr int WAVES = BT / kWave;
+  const uint32_t tid = threadIdx.x, w = tid / kWave;
+  for (uint32_t at = 0; at < total; at += kRadixBits) {
+    for (uint32_t j = tid; j < uint32_t(WAVES) * kRadix; j += BT) (&sm.wcnt[0][0])[j] = 0;
+    __syncthreads();
+    uint32_t rank[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      if (uint32_t(i) >= items) continue;
+      const bool valid = row_pos(items, i) < m;
+      const uint32_t d = valid ? digit_of<PW>(lo[i], hi[i], at) : 0;
+      const uint64_t peers = match_digit(d, valid);
+      const uint32_t before = valid ? sm.wcnt[w][d] : 0;
+      rank[i] = before + popc_below(peers);
+      if (valid && popc_below(peers) == 0) sm.wcnt[w][d] = before + __popcll(peers);
+    }
+    __syncthreads();
+    uint32_t tot = 0;
+    if (tid < uint32_t(kRadix))
+#pragma unroll
+      for (int j = 0; j < WAVES; ++j) {
+        const uint32_t c = sm.wcnt[j][tid];
+        sm.wcnt[j][tid] = tot;
+        tot += c;
+      }
+    const uint32_t start = block_scan32<WAVES>(tot, sm.wsum);
+    if (tid < uint32_t(kRadix)) sm.local[tid] = start;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      if (uint32_t(i) >= items || row_pos(items, i) >= m) continue;
+      const uint32_t d = digit_of<PW>(lo[i], hi[i], at);
+      const uint32_t q = sm.local[d] + sm.wcnt[w][d] + rank[i];
+      sm.key[0][q] = lo[i];
+      if (PW == 2) sm.key[W - 1][q] = hi[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const uint32_t p = row_pos(items, i);
+      if (uint32_t(i) >= items || p >= m) continue;
+      lo[i] = sm.key[0][p];
+      if (PW == 2) hi[i] = sm.key[W - 1][p];
+    }
+  }
+  __syncthreads();
+}
+
+// Sort the m raw keys a workgroup holds in registers (row_pos order); the
+// sorted keys are left in the registers and in sm.key.  The keys are put in
+// bins by the top bits of those in which they differ (squeezed together field
+// by field), about as many bins as rows, and every key then counts the
+// smaller ones of its bin: one pass over LDS, where a radix sort takes one a
+// digit (4,096 pairs: 24 us in five passes, 6.7 us so).  Keys that crowd
+// into few bins are sorted by the radix passes, a 128-bit key with at most 64
+// differing bits as one word.
+constexpr uint32_t kBinCrowd = 64;  // most keys of a bin that count each other
+
+template <int W, int BT, int ITEMS>
+__device__ __forceinline__ void block_sort(uint64_t (&lo)[ITEMS], uint64_t (&hi)[ITEMS], uint32_t m,
+                                           uint32_t items, SortMem<W, BT, ITEMS>& sm) {
+  constexpr int WAVES = BT / kWave;
+  constexpr uint32_t NB = WAVES * kRadix;  // bins: sm.wcnt
+  constexpr uint32_t LG = __builtin_ctz(NB), PER = NB / BT;
+  constexpr int GR = ITEMS < 4 ? ITEMS : 4;  // items whose loads are in flight together
+  static_assert(PER == 4, "a thread scans four bins");
+  const uint32_t tid = threadIdx.x, w = tid / kWave, l = lane_id();
+  uint32_t* bin = &sm.wcnt[0][0];
+  reinterpret_cast<uint4*>(bin)[tid] = make_uint4(0, 0, 0, 0);
+  if (tid < 2u * W) {
+    sm.least[tid] = ~0u;
+    sm.most[tid] = 0;
+  }
+  __syncthreads();
+  // each field counts from its least value, in the bits its range needs
+  uint32_t base[2 * W], wd[2 * W], total = 0;
+#pragma unroll
+  for (int f = 0; f < 2 * W; ++f) {
+    uint32_t a = ~0u, b = 0;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+      if (uint32_t(i) < items && row_pos(items, i) < m) {
+        const uint32_t v = key_field<W>(lo[i], hi[i], f);
+        a = min(a, v);
+        b = max(b, v);
+      }
+    a = wave_min32(a);
+    b = wave_max32(b);
+    if (l == 0) {
+      atomicMin(&sm.least[f], a);
+      atomicMax(&sm.most[f], b);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int f = 0; f < 2 * W; ++f) {
+    const uint32_t a = __builtin_amdgcn_readfirstlane(sm.least[f]), b = __builtin_amdgcn_readfirstlane(sm.most[f]);
+    base[f] = a;
+    wd[f] = b > a ? 32u - uint32_t(__builtin_clz(b - a)) : 0u;
+    total += wd[f];
+  }
+  // top LG of the bits in use, field by field from the top
+  auto bin_of = [&](uint64_t a, uint64_t b) {
+    uint32_t d = 0, room = LG;
+#pragma unroll
+    for (int f = 2 * W - 1; f >= 0; --f) {
+      const uint32_t take = min(wd[f], room);
+      d = (d << take) | (take ? (key_field<W>(a, b, f) - base[f]) >> (wd[f] - take) : 0);
+      room -= take;
+    }
+    return d;
+  };
+  uint32_t rank[ITEMS];
+#pragma unroll
+  for (int g = 0; g < ITEMS; g += GR) {
+    if (uint32_t(g) >= items) continue;
+#pragma unroll
+    for (int i = g; i < g + GR; ++i) {
+      rank[i] = 0;
+      if (uint32_t(i) < items && row_pos(items, i) < m) rank[i] = atomicAdd(&bin[bin_of(lo[i], hi[i])], 1u);
+    }
+  }
+  __syncthreads();
+  const uint4 c4 = reinterpret_cast<const uint4*>(bin)[tid];
+  const uint32_t crowd = wave_max32(max(max(c4.x, c4.y), max(c4.z, c4.w)));
+  if (l == 0) sm.local[w] = crowd;
+  const uint32_t first = block_scan32<WAVES>(c4.x + c4.y + c4.z + c4.w, sm.wsum);
+  uint32_t most = 0;
+#pragma unroll
+  for (int j = 0; j < WAVES; ++j) most = max(most, sm.local[j]);
+  if (most <= kBinCrowd) {
+    reinterpret_cast<uint4*>(bin)[tid] =
+        make_uint4(first, first + c4.x, first + c4.x + c4.y, first + c4.x + c4.y + c4.z);
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < ITEMS; g += GR) {
+      if (uint32_t(g) >= items) continue;
+#pragma unroll
+      for (int i = g; i < g + GR; ++i) {
+        if (uint32_t(i) >= items || row_pos(items, i) >= m) continue;
+        rank[i] += bin[bin_of(lo[i], hi[i])];
+        sm.key[0][rank[i]] = lo[i];
+        if (W == 2) sm.key[W - 1][rank[i]] = hi[i];
+      }
+    }
+    __syncthreads();
+    // Each thread places the keys that now lie at its own positions: bins are
+    // a key or two long, so a wave reads one stretch of LDS.
+#pragma unroll
+    for (int g = 0; g < ITEMS; g += GR) {
+      if (uint32_t(g) >= items) continue;
+      uint32_t s[GR], e[GR];
+#pragma unroll
+      for (int i = 0; i < GR; ++i) {
+        const uint32_t p = row_pos(items, g + i);
+        s[i] = e[i] = 0;
+        if (uint32_t(g + i) >= items || p >= m) continue;
+        lo[g + i] = sm.key[0][p];
+        hi[g + i] = W == 2 ? sm.key[W - 1][p] : 0;
+        const uint32_t d = bin_of(lo[g + i], hi[g + i]);
+        s[i] = bin[d];
+        e[i] = d + 1 < NB ? bin[d + 1] : m;
+        rank[g + i] = s[i];
+      }
+      bool more = true;
+      while (more) {
+        more = false;
+#pragma unroll
+        for (int i = 0; i < GR; ++i) {
+          if (s[i] >= e[i]) continue;
+          const uint32_t j = s[i]++;
+          const uint64_t kl = sm.key[0][j], kh = W == 2 ? sm.key[W - 1][j] : 0;
+          const bool same = kl == lo[g + i] && (W == 1 || kh == hi[g + i]);
+          rank[g + i] += same ? j < row_pos(items, g + i) : key_le<W>(kl, kh, lo[g + i], hi[g + i]);
+          more |= s[i] < e[i];
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      if (uint32_t(i) >= items || row_pos(items, i) >= m) continue;
+      sm.key[0][rank[i]] = lo[i];
+      if (W == 2) sm.key[W - 1][rank[i]] = hi[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const uint32_t p = row_pos(items, i);
+      if (uint32_t(i) >= items || p >= m) continue;
+      lo[i] = sm.key[0][p];
+      if (W == 2) hi[i] = sm.key[W - 1][p];
+    }
+    return;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    unsigned __int128 v = 0;
+#pragma unroll
+    for (int f = 2 * W - 1; f >= 0; --f)
+      v = (v << wd[f]) | (uint64_t(key_field<W>(lo[i], hi[i], f) - base[f]) & ((uint64_t(1) << wd[f]) - 1));
+    lo[i] = uint64_t(v);
+    hi[i] = uint64_t(v >> 64);
+  }
+  if (W == 2 && total > 64) block_passes<W, W, BT, ITEMS>(lo, hi, m, items, total, sm);
+  else block_passes<1, W, BT, ITEMS>(lo, hi, m, items, total, sm);
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t p = row_pos(items, i);
+    if (uint32_t(i) >= items || p >= m) continue;
+    unsigned __int128 v = (static_cast<unsigned __int128>(W == 2 && total > 64 ? hi[i] : 0) << 64) | lo[i];
+    uint64_t r[W] = {};
+#pragma unroll
+    for (int f = 0; f < 2 * W; ++f) {
+      const uint32_t x = base[f] + uint32_t(uint64_t(v) & ((uint64_t(1) << wd[f]) - 1));
+      r[f / 2] |= uint64_t(x) << (f & 1 ? 32 : 0);
+      v >>= wd[f];
+    }
+    lo[i] = r[0];
+    hi[i] = W == 2 ? r[W - 1] : 0;
+    sm.key[0][p] = lo[i];
+    if (W == 2) sm.key[W - 1][p] = hi[i];
+  }
+  __syncthreads();
+}
+
+// First rows of their value (bit i of fu) and of their column 0 (fr) among
+// the sorted rows in sm.key; the row before the first is (plo, phi) if
+// has_prev.  Every thread gets the totals u, r and its wave's offsets.
+template <int W, int BT, int ITEMS>
+__device__ __forceinline__ void block_firsts(const uint64_t (&lo)[ITEMS], const uint64_t (&hi)[ITEMS],
+                                             uint32_t m, uint32_t items, uint32_t k, bool has_prev,
+                                             uint64_t plo, uint64_t phi, SortMem<W, BT, ITEMS>& sm,
+                                             uint32_t& fu, uint32_t& fr, uint32_t& pu, uint32_t& pr,
+                                             uint32_t& u, uint32_t& r) {
+  constexpr int WAVES = BT / kWave;
+  static_assert(BT * ITEMS < 65536, "counts share a word");
+  const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  fu = fr = 0;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (uint32_t(i) >= items) continue;
+    const uint32_t p = row_pos(items, i);
+    bool a = false, b = false;
+    if (p < m) {
+      const uint64_t ql = p ? sm.key[0][p - 1] : plo, qh = W == 1 ? 0 : p ? sm.key[W - 1][p - 1] : phi;
+      const bool none = p == 0 && !has_prev;
+      a = none || lo[i] != ql || (W == 2 && hi[i] != qh);
+      b = none || key_field<W>(lo[i], hi[i], k - 1) != key_field<W>(ql, qh, k - 1);
+    }
+    fu |= uint32_t(a) << i;
+    fr |= uint32_t(b) << i;
+    const uint64_t mu = ballot(a), mr = ballot(b);
+    if (l == 0) sm.firsts[w * items + i] = uint32_t(__popcll(mu)) | uint32_t(__popcll(mr)) << 16;
+  }
+  __syncthreads();
+  uint32_t all = 0, before = 0;
+#pragma unroll
+  for (uint32_t j = l; j < uint32_t(ITEMS) * WAVES; j += kWave) {
+    const uint32_t c = j < items * WAVES ? sm.firsts[j] : 0;
+    all += c;
+    before += j < w * items ? c : 0;
+  }
+  all = wave_add32(all);
+  before = wave_add32(before);
+  u = all & 0xFFFFu;
+  r = all >> 16;
+  pu = before & 0xFFFFu;
+  pr = before >> 16;
+}
+
+struct SortOut {
+  uint32_t* cols;        // k columns, `stride` apart
+  uint64_t stride;
+  uint32_t* root_vals;
+  uint32_t* root_offs;
+};
+
+// Row `row` (and root g, if it is one) of the result.
+template <int W>
+__device__ __forceinline__ void put_row(const SortOut& o, uint32_t k, uint64_t row, uint64_t lo,
+                                        uint64_t hi, bool root, uint64_t g) {
+#pragma unroll
+  for (uint32_t c = 0; c < 2u * W; ++c)
+    if (c < k) o.cols[uint64_t(c) * o.stride + row] = key_field<W>(lo, hi, k - 1 - c);
+  if (root) {
+    o.root_vals[g] = key_field<W>(lo, hi, k - 1);
+    o.root_offs[g] = uint32_t(row);
+  }
+}
+
+// Write the first rows of block_firsts from result row pu, root pr on.
+template <int W, int ITEMS>
+__device__ __forceinline__ void block_write(const uint64_t (&lo)[ITEMS], const uint64_t (&hi)[ITEMS],
+                                            uint32_t items, uint32_t k, uint32_t fu, uint32_t fr,
+                                            uint64_t pu, uint64_t pr, const SortOut& o) {
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (uint32_t(i) >= items) continue;
+    const bool a = (fu >> i) & 1u, b = (fr >> i) & 1u;
+    const uint64_t mu = ballot(a), mr = ballot(b);
+    if (a) put_row<W>(o, k, pu + popc_below(mu), lo[i], hi[i], b, pr + popc_below(mr));
+    pu += __popcll(mu);
+    pr += __popcll(mr);
+  }
+}
+
 // ========================================================= sort: small ====
 // The whole sort + dedup + root build of up to kSmallRows rows in one launch
-// of one workgroup: column maxima, key layout, an LSD radix sort in LDS (keys
-// in registers between passes, digits that are equal in all keys skipped),
-// dedup and every output.  Launches and the gaps between them are what
-// bounds a small sort: 1,000 pairs took 97 us in 19 launches and take 12.5 us
-// in one.  Rows beyond 4,096 no longer fit the registers of one workgroup.
+// of one workgroup.  Launches and the gaps between them are what bounds a
+// small sort: 1,000 pairs took 97 us in 19 launches and take 6.5 us in
+// one.  Rows beyond 4,096 no longer fit the registers of one workgroup.
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallItems = 4;
@@ -1623,202 +2022,48 @@ constexpr uint64_t kSmallRows = uint64_t(kSmallBlock) * kSmallItems;
 
 struct SmallSort {
   const uint32_t* in[kMaxCols];
-  uint32_t* cols;        // out columns, `stride` apart
-  uint64_t stride;
-  uint32_t* root_vals;
-  uint32_t* root_offs;
+  SortOut out;
   uint64_t* counts;      // distinct rows, distinct column-0 values, 0
   uint32_t* maxima;      // per column (may be null)
   uint32_t n, k;
 };
 
-// The workgroup's OR of v, the same in every thread.
-__device__ __forceinline__ uint64_t small_or(uint64_t v, uint64_t* s_w) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
-  if (lane_id() == 0) s_w[threadIdx.x / kWave] = v;
-  __syncthreads();
-  uint64_t r = 0;
-  for (int j = 0; j < kSmallWaves; ++j) r |= s_w[j];
-  __syncthreads();
-  return r;
-}
-
 template <int W, int ITEMS>
 __global__ __launch_bounds__(kSmallBlock) void small_sort_kernel(SmallSort a) {
-  constexpr uint32_t ROWS = kSmallBlock * ITEMS;
-  __shared__ uint64_t s_key[W][ROWS];
-  __shared__ uint32_t s_wcnt[kSmallWaves][kRadix];
-  __shared__ uint32_t s_local[kRadix];
-  __shared__ uint32_t s_max[kSmallWaves][4];
-  __shared__ uint64_t s_or[kSmallWaves];
-  __shared__ uint32_t s_wsum[kSmallWaves];
-  __shared__ uint32_t s_u[ITEMS * kSmallWaves], s_r[ITEMS * kSmallWaves];
+  __shared__ SortMem<W, kSmallBlock, ITEMS> sm;
+  __shared__ uint32_t s_max[kSmallWaves][2 * W];
   const uint32_t tid = threadIdx.x, w = tid / kWave, l = lane_id();
   const uint32_t n = a.n, k = a.k;
-
-  // maxima (rows in the order of the passes: wave, item, lane)
-#pragma unroll
-  for (uint32_t c = 0; c < 4; ++c) {
-    if (c >= k) continue;
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const uint32_t p = w * (kWave * ITEMS) + i * kWave + l;
-      if (p < n) m = max(m, a.in[c][p]);
-    }
-    m = wave_max(m);
-    if (l == 0) s_max[w][c] = m;
-  }
-  __syncthreads();
-  uint32_t shift[4] = {}, bits[4] = {}, total = 0;
-#pragma unroll
-  for (int c = 3; c >= 0; --c) {
-    if (c >= int(k)) continue;
-    uint32_t m = 0;
-    for (int j = 0; j < kSmallWaves; ++j) m = max(m, s_max[j][c]);
-    if (tid == 0 && a.maxima) a.maxima[c] = m;
-    const uint32_t b = m ? 32u - uint32_t(__builtin_clz(m)) : 0u;
-    shift[c] = total;
-    bits[c] = b;
-    total += b;
-  }
   uint64_t lo[ITEMS], hi[ITEMS];
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
-    const uint32_t p = w * (kWave * ITEMS) + i * kWave + l;
+    const uint32_t p = row_pos(ITEMS, i);
     lo[i] = hi[i] = 0;
-    if (p < n)
-#pragma unroll
-      for (uint32_t c = 0; c < 4; ++c) {
-        if (c >= k) continue;
-        const uint64_t v = a.in[c][p];
-        const uint32_t s = shift[c];
-        if (s >= 64) {
-          hi[i] |= v << (s - 64);
-        } else {
-          lo[i] |= v << s;
-          if (W == 2 && s > 32) hi[i] |= v >> (64 - s);
-        }
-      }
+    if (p < n) raw_key<W>(a.in, k, p, lo[i], hi[i]);
   }
-  // bits in which any key differs from the first row's
+  if (a.maxima) {
+#pragma unroll
+    for (uint32_t c = 0; c < 2u * W; ++c) {
+      if (c >= k) continue;
+      uint32_t m = 0;
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) m = max(m, key_field<W>(lo[i], hi[i], k - 1 - c));
+      m = wave_max(m);
+      if (l == 0) s_max[w][c] = m;
+    }
+    __syncthreads();
+    if (tid < k) {
+      uint32_t m = 0;
+      for (int j = 0; j < kSmallWaves; ++j) m = max(m, s_max[j][tid]);
+      a.maxima[tid] = m;
+    }
+  }
+  block_sort<W, kSmallBlock, ITEMS>(lo, hi, n, ITEMS, sm);
+  uint32_t fu, fr, pu, pr, u, r;
+  block_firsts<W, kSmallBlock, ITEMS>(lo, hi, n, ITEMS, k, false, 0, 0, sm, fu, fr, pu, pr, u, r);
+  block_write<W, ITEMS>(lo, hi, ITEMS, k, fu, fr, pu, pr, a.out);
   if (tid == 0) {
-    s_key[0][0] = lo[0];
-    if (W == 2) s_key[W - 1][0] = hi[0];
-  }
-  __syncthreads();
-  const uint64_t lo0 = s_key[0][0], hi0 = W == 2 ? s_key[W - 1][0] : 0;
-  uint64_t dl = 0, dh = 0;
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i)
-    if (w * (kWave * ITEMS) + i * kWave + l < n) {
-      dl |= lo[i] ^ lo0;
-      dh |= hi[i] ^ hi0;
-    }
-  dl = small_or(dl, s_or);
-  if (W == 2) dh = small_or(dh, s_or);
-
-  for (uint32_t at = 0; at < total; at += kRadixBits) {
-    if (digit_of<W>(dl, dh, at) == 0) continue;
-    for (uint32_t j = tid; j < kSmallWaves * kRadix; j += kSmallBlock) (&s_wcnt[0][0])[j] = 0;
-    __syncthreads();
-    uint32_t rank[ITEMS], dig[ITEMS];
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const bool valid = w * (kWave * ITEMS) + i * kWave + l < n;
-      const uint32_t d = valid ? digit_of<W>(lo[i], hi[i], at) : 0;
-      dig[i] = d;
-      const uint64_t peers = match_digit(d, valid);
-      const uint32_t before = valid ? s_wcnt[w][d] : 0;
-      rank[i] = before + popc_below(peers);
-      if (valid && popc_below(peers) == 0) s_wcnt[w][d] = before + __popcll(peers);
-    }
-    __syncthreads();
-    uint32_t tot = 0;
-    if (tid < uint32_t(kRadix))
-      for (int j = 0; j < kSmallWaves; ++j) {
-        const uint32_t c = s_wcnt[j][tid];
-        s_wcnt[j][tid] = tot;
-        tot += c;
-      }
-    uint32_t all;
-    const uint32_t start = block_excl_scan<uint32_t, kSmallWaves>(tot, s_wsum, &all);
-    if (tid < uint32_t(kRadix)) s_local[tid] = start;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i)
-      if (w * (kWave * ITEMS) + i * kWave + l < n) {
-        const uint32_t q = s_local[dig[i]] + s_wcnt[w][dig[i]] + rank[i];
-        s_key[0][q] = lo[i];
-        if (W == 2) s_key[W - 1][q] = hi[i];
-      }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const uint32_t p = w * (kWave * ITEMS) + i * kWave + l;
-      if (p < n) {
-        lo[i] = s_key[0][p];
-        if (W == 2) hi[i] = s_key[W - 1][p];
-      }
-    }
-    __syncthreads();
-  }
-  // rows in order (wave, item, lane): predecessors from LDS
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    const uint32_t p = w * (kWave * ITEMS) + i * kWave + l;
-    if (p < n) {
-      s_key[0][p] = lo[i];
-      if (W == 2) s_key[W - 1][p] = hi[i];
-    }
-  }
-  __syncthreads();
-  uint64_t mu[ITEMS], mr[ITEMS];
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    const uint32_t p = w * (kWave * ITEMS) + i * kWave + l;
-    bool fu = false, fr = false;
-    if (p < n) {
-      const uint64_t pl = p ? s_key[0][p - 1] : 0, ph = W == 2 && p ? s_key[W - 1][p - 1] : 0;
-      fu = p == 0 || lo[i] != pl || (W == 2 && hi[i] != ph);
-      fr = p == 0 || key_col<W>(lo[i], hi[i], shift[0], bits[0]) != key_col<W>(pl, ph, shift[0], bits[0]);
-    }
-    mu[i] = ballot(fu);
-    mr[i] = ballot(fr);
-    if (l == 0) {
-      s_u[w * ITEMS + i] = __popcll(mu[i]);
-      s_r[w * ITEMS + i] = __popcll(mr[i]);
-    }
-  }
-  __syncthreads();
-  uint32_t pu = 0, pr = 0, u = 0, r = 0;
-  for (uint32_t j = 0; j < uint32_t(ITEMS * kSmallWaves); ++j) {
-    if (j < w * ITEMS) {
-      pu += s_u[j];
-      pr += s_r[j];
-    }
-    u += s_u[j];
-    r += s_r[j];
-  }
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    if ((mu[i] >> l) & 1u) {
-      const uint32_t row = pu + popc_below(mu[i]);
-#pragma unroll
-      for (uint32_t c = 0; c < 4; ++c)
-        if (c < k) a.cols[uint64_t(c) * a.stride + row] = key_col<W>(lo[i], hi[i], shift[c], bits[c]);
-      if ((mr[i] >> l) & 1u) {
-        const uint32_t g = pr + popc_below(mr[i]);
-        a.root_vals[g] = key_col<W>(lo[i], hi[i], shift[0], bits[0]);
-        a.root_offs[g] = row;
-      }
-    }
-    pu += __popcll(mu[i]);
-    pr += __popcll(mr[i]);
-  }
-  if (tid == 0) {
-    a.root_offs[r] = u;
+    a.out.root_offs[r] = u;
     a.counts[0] = u;
     a.counts[1] = r;
     a.counts[2] = 0;
@@ -1835,6 +2080,485 @@ static void small_sort(const SmallSort& a, hipStream_t s) {
   else SRD_SMALL(kSmallItems);
 #undef SRD_SMALL
   SRD_CHECK(hipGetLastError());
+}
+
+// ======================================================= sort: buckets ====
+// Sort + dedup + roots of up to kBucketRows rows in two launches, row count on
+// the device.  The radix sort below takes 19 launches for pairs and 23 for
+// triples, and what bounds it at these sizes is each launch's own latency:
+// its passes move 1 M rows in 23 us where the copy takes 4, and 100 k rows,
+// 25 tiles chained through the look-back, in 14 us; a skipped pass is 4 us.
+//   bucket_part  every workgroup sorts the same sample of the rows, takes
+//                every s-th as a splitter, and orders its tile of rows by
+//                bucket (the number of splitters not above the row).  Rows
+//                equal to a splitter are dropped: the splitter itself is a
+//                row of the result, so a value that repeats often fills no
+//                bucket.
+//   bucket_sort  one workgroup a bucket gathers its runs from the tiles,
+//                sorts them in LDS, and takes its place in the result by a
+//                look-back over the buckets.
+// Equal rows are one row of the result, so the order within a bucket's runs
+// is free and no pass needs the tiles in order.  Measured: 1 M pairs of 20-bit
+// values 205 -> 73 us, 100 k triples of 24-bit values 209 -> 36 us.
+constexpr uint64_t kBucketRows = uint64_t(1) << 20;
+constexpr int kPartBlock = 1024, kPartItems = 4;  // tile: up to 4,096 rows
+constexpr uint32_t kPartTiles = 256;
+constexpr int kBinBlock = 512, kBinItems = 16;    // bucket in LDS: up to 8,192 rows
+constexpr uint32_t kBins = 512;
+constexpr uint32_t kBinRows = kBinBlock * kBinItems;
+
+// Buckets of a sort of n rows: 512 to 1,024 rows each until all kBins are in
+// use (2,048 rows at the largest n).  Smaller buckets mean more hops of the
+// look-back, larger ones fewer CUs at work.
+__host__ __device__ inline uint32_t bucket_bins(uint64_t n) {
+  uint32_t b = 8;
+  while (b < kBins && uint64_t(b) * 1024 <= n) b *= 2;
+  return b;
+}
+
+// Rows a tile: as few as kPartTiles tiles allow, at least one a thread.
+__host__ __device__ inline uint32_t part_rows(uint64_t n) {
+  const uint64_t r = (n + kPartTiles - 1) / kPartTiles;
+  return uint32_t(r <= uint64_t(kPartBlock) ? kPartBlock : (r + kWave - 1) / kWave * kWave);
+}
+
+struct BucketSort {
+  const uint32_t* in[4];
+  uint32_t k;
+  uint64_t n_host, cap;
+  const uint64_t* n_dev;       // row count on the device (may be null)
+  uint64_t* part[2];           // rows by tile and bucket: low words, high words
+  uint64_t* spill[2];          // rows of buckets beyond kBinRows
+  uint32_t* runs;              // [tile][bucket] first | end << 16, within the tile
+  uint64_t* split[2];          // splitters
+  uint64_t* lookback;          // per bucket
+  uint32_t* ctl;               // ticket, look-back error, spill rows
+  uint32_t* stats;             // per tile: 4 column maxima, order flags (may be null)
+  SortOut out;
+  uint64_t* counts;            // distinct rows, distinct column-0 values, error bits
+  uint32_t* maxima;            // 4 column maxima, order flags (with stats)
+  uint32_t ticket;             // take the bucket from a ticket instead of the block id
+};
+
+__device__ __forceinline__ uint64_t bucket_n(const BucketSort& a) {
+  const uint64_t n = a.n_dev ? *a.n_dev : a.n_host;
+  return n > a.cap ? a.cap : n;
+}
+
+template <int W>
+__global__ __launch_bounds__(kPartBlock) void bucket_part_kernel(BucketSort a) {
+  __shared__ SortMem<W, kPartBlock, kPartItems> sm;
+  __shared__ uint64_t s_split[W][kBins];
+  __shared__ uint32_t s_cnt[kBins];
+  __shared__ uint32_t s_stat[5], s_kept;
+  const uint32_t tid = threadIdx.x, l = lane_id(), k = a.k;
+  const uint64_t n = bucket_n(a);
+  if (blockIdx.x == 0) {
+    // state of this sort's second launch
+    if (tid < kBins) a.lookback[tid] = 0;
+    if (tid < 4) a.ctl[tid] = 0;
+  }
+  const uint32_t rows = part_rows(n);
+  const uint64_t base = uint64_t(blockIdx.x) * rows;
+  if (base >= n) return;
+  const uint32_t bins = bucket_bins(n);
+  // The sample: eight rows a bucket, at least one a thread, one from each of
+  // S equal stretches of the rows at a scattered place.  With eight, a bucket
+  // of four times its share (what LDS holds at 2,048 rows a bucket) is a
+  // chance of 1e-7; it is sorted all the same, more slowly.
+  const uint32_t S = max(8u * bins, uint32_t(kPartBlock)), items = S / kPartBlock;
+  uint64_t lo[kPartItems], hi[kPartItems];
+  static_assert(kBucketRows << 11 <= uint64_t(1) << 31, "the sample's positions are computed in 32 bits");
+  const uint32_t step = (uint32_t(n) << 11) / S, gap = step >> 11;
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i) {
+    lo[i] = hi[i] = 0;
+    if (uint32_t(i) >= items) continue;
+    const uint32_t j = row_pos(items, i);
+    const uint32_t p = (j * step >> 11) + ((j * 2654435761u >> 16) * gap >> 16);
+    raw_key<W>(a.in, k, p, lo[i], hi[i]);
+  }
+  if (tid < kBins) s_cnt[tid] = 0;
+  if (tid < 5) s_stat[tid] = 0;
+  block_sort<W, kPartBlock, kPartItems>(lo, hi, S, items, sm);
+  if (tid < bins) {
+    // one more than the splitters there are: the last is never read
+    const uint32_t q = min((tid + 1) * (S / bins), S - 1);
+#pragma unroll
+    for (int wd = 0; wd < W; ++wd) {
+      const uint64_t v = sm.key[wd][q];
+      s_split[wd][tid] = v;
+      if (blockIdx.x == 0) a.split[wd][tid] = v;
+    }
+  }
+  __syncthreads();
+
+  const uint32_t count = uint32_t(min<uint64_t>(rows, n - base));
+  uint32_t bin[kPartItems], rank[kPartItems];
+  uint32_t mx[2 * W] = {}, fl = 0;
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i)
+    raw_key<W>(a.in, k, base + min(i * kPartBlock + tid, count - 1), lo[i], hi[i]);
+  uint32_t b[kPartItems] = {};
+  for (uint32_t half = bins / 2; half; half >>= 1)
+#pragma unroll
+    for (int i = 0; i < kPartItems; ++i) {
+      const uint32_t q = b[i] + half - 1;
+      if (key_le<W>(s_split[0][q], W == 2 ? s_split[W - 1][q] : 0, lo[i], hi[i])) b[i] += half;
+    }
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i) {
+    const uint32_t p = i * kPartBlock + tid;
+    bin[i] = ~0u;
+    rank[i] = 0;
+    if (p >= count) continue;
+    if (a.stats) {
+#pragma unroll
+      for (uint32_t c = 0; c < 2u * W; ++c)
+        if (c < k) mx[c] = max(mx[c], key_field<W>(lo[i], hi[i], k - 1 - c));
+      if (base + p > 0) {
+        uint64_t ql, qh;
+        raw_key<W>(a.in, k, base + p - 1, ql, qh);
+        if (key_le<W>(lo[i], hi[i], ql, qh)) fl |= lo[i] == ql && hi[i] == qh ? 2u : 1u;
+      }
+    }
+    const uint32_t q = b[i];
+    if (q && s_split[0][q - 1] == lo[i] && (W == 1 || s_split[W - 1][q - 1] == hi[i])) continue;
+    bin[i] = q;
+    rank[i] = atomicAdd(&s_cnt[q], 1u);
+  }
+  if (a.stats) {
+#pragma unroll
+    for (uint32_t c = 0; c < 2u * W; ++c) {
+      const uint32_t v = wave_max32(mx[c]);
+      if (l == 0 && v) atomicMax(&s_stat[c], v);
+    }
+    const uint32_t f = (ballot(fl & 1u) ? 1u : 0u) | (ballot(fl & 2u) ? 2u : 0u);
+    if (l == 0 && f) atomicOr(&s_stat[4], f);
+  }
+  __syncthreads();
+  const uint32_t c = tid < kBins ? s_cnt[tid] : 0;
+  const uint32_t first = block_scan32<kPartBlock / kWave>(c, sm.wsum);
+  if (tid == kPartBlock - 1) s_kept = first;
+  if (tid < bins) {
+    s_cnt[tid] = first;
+    a.runs[blockIdx.x * kBins + tid] = first | ((first + c) << 16);
+  }
+  if (a.stats && tid < 5) a.stats[blockIdx.x * 5 + tid] = s_stat[tid];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i) {
+    if (bin[i] == ~0u) continue;
+    const uint32_t q = s_cnt[bin[i]] + rank[i];
+    sm.key[0][q] = lo[i];
+    if (W == 2) sm.key[W - 1][q] = hi[i];
+  }
+  __syncthreads();
+  const uint32_t kept = s_kept;
+  for (uint32_t p = tid; p < kept; p += kPartBlock)
+#pragma unroll
+    for (int wd = 0; wd < W; ++wd) a.part[wd][base + p] = sm.key[wd][p];
+}
+
+// Take the place of a bucket of u rows and r roots in the result: the sums
+// over the buckets before it (every thread gets them).  u and r share a
+// look-back word, 23 bits each.
+__device__ __forceinline__ void bucket_place(const BucketSort& a, uint32_t b, uint32_t u, uint32_t r,
+                                             uint64_t* s_place, uint64_t& pu, uint64_t& pr) {
+  static_assert(kBucketRows < (uint64_t(1) << 23), "a count fits 23 bits");
+  const uint64_t mine = uint64_t(u) | uint64_t(r) << 23;
+  if (threadIdx.x < uint32_t(kWave)) {
+    if (threadIdx.x == 0) lb_store(&a.lookback[b], lb_pack(1, b ? kLbAgg : kLbPrefix, mine));
+    const uint64_t before = wave_lookback(a.lookback, 1, b, 1, &a.ctl[1]);
+    if (threadIdx.x == 0) {
+      if (b) lb_store(&a.lookback[b], lb_pack(1, kLbPrefix, before + mine));
+      *s_place = before;
+    }
+  }
+  __syncthreads();
+  pu = *s_place & ((1u << 23) - 1);
+  pr = *s_place >> 23;
+}
+
+// A bucket beyond LDS, sorted by its workgroup in device memory: LSD passes
+// between its runs (buffer 0, position p found as above) and its share of the
+// spill rows (buffer 1).  Right at any size: what keeps it rare is the
+// sample.
+template <int W>
+struct SpillRows {
+  uint64_t* part[2];
+  uint64_t* spill[2];
+  const uint32_t *pref, *src;
+  uint32_t buf;
+  __device__ __forceinline__ uint32_t at(uint32_t to, uint32_t p) const {
+    if (to) return p;
+    uint32_t t = 0;
+    for (uint32_t step = kPartTiles / 2; step; step >>= 1)
+      if (pref[t + step] <= p) t += step;
+    return src[t] + p;
+  }
+  __device__ __forceinline__ void load(uint32_t p, uint64_t& lo, uint64_t& hi) const {
+    const uint32_t q = at(buf, p);
+    lo = (buf ? spill : part)[0][q];
+    hi = W == 2 ? (buf ? spill : part)[W - 1][q] : 0;
+  }
+  __device__ __forceinline__ void store(uint32_t p, uint64_t lo, uint64_t hi) const {
+    const uint32_t q = at(buf ^ 1u, p);
+    (buf ? part : spill)[0][q] = lo;
+    if (W == 2) (buf ? part : spill)[W - 1][q] = hi;
+  }
+};
+
+template <int W, class Mem>
+__device__ __forceinline__ void spill_sort(SpillRows<W>& x, uint32_t m, Mem& sm) {
+  constexpr int WAVES = kBinBlock / kWave, IT = 4;
+  const uint32_t tid = threadIdx.x, w = tid / kWave, l = lane_id();
+  uint64_t lo0, hi0, dl = 0, dh = 0;
+  x.load(0, lo0, hi0);
+  for (uint32_t p = tid; p < m; p += kBinBlock) {
+    uint64_t lo, hi;
+    x.load(p, lo, hi);
+    dl |= lo ^ lo0;
+    dh |= hi ^ hi0;
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    dl |= __shfl_xor(dl, o, kWave);
+    dh |= __shfl_xor(dh, o, kWave);
+  }
+  if (l == 0) {
+    sm.diff[0][w] = dl;
+    sm.diff[1][w] = dh;
+  }
+  __syncthreads();
+  dl = dh = 0;
+  for (int j = 0; j < WAVES; ++j) {
+    dl |= sm.diff[0][j];
+    dh |= sm.diff[1][j];
+  }
+  for (uint32_t at = 0; at < 64u * W; at += kRadixBits) {
+    if (digit_of<W>(dl, dh, at) == 0) continue;
+    if (tid < uint32_t(kRadix)) sm.local[tid] = 0;
+    __syncthreads();
+    for (uint32_t p = tid; p < m; p += kBinBlock) {
+      uint64_t lo, hi;
+      x.load(p, lo, hi);
+      atomicAdd(&sm.local[digit_of<W>(lo, hi, at)], 1u);
+    }
+    __syncthreads();
+    uint32_t all;
+    const uint32_t start =
+        block_excl_scan<uint32_t, WAVES>(tid < uint32_t(kRadix) ? sm.local[tid] : 0, sm.wsum, &all);
+    if (tid < uint32_t(kRadix)) sm.local[tid] = start;
+    for (uint32_t c0 = 0; c0 < m; c0 += kBinBlock * IT) {
+      for (uint32_t j = tid; j < uint32_t(WAVES) * kRadix; j += kBinBlock) (&sm.wcnt[0][0])[j] = 0;
+      __syncthreads();
+      uint64_t lo[IT], hi[IT];
+      uint32_t rank[IT];
+#pragma unroll
+      for (int i = 0; i < IT; ++i) {
+        const uint32_t p = c0 + row_pos(IT, i);
+        const bool valid = p < m;
+        lo[i] = hi[i] = 0;
+        if (valid) x.load(p, lo[i], hi[i]);
+        const uint32_t d = valid ? digit_of<W>(lo[i], hi[i], at) : 0;
+        const uint64_t peers = match_digit(d, valid);
+        const uint32_t before = valid ? sm.wcnt[w][d] : 0;
+        rank[i] = before + popc_below(peers);
+        if (valid && popc_below(peers) == 0) sm.wcnt[w][d] = before + __popcll(peers);
+      }
+      __syncthreads();
+      if (tid < uint32_t(kRadix)) {
+        uint32_t run = sm.local[tid];
+        for (int j = 0; j < WAVES; ++j) {
+          const uint32_t c = sm.wcnt[j][tid];
+          sm.wcnt[j][tid] = run;
+          run += c;
+        }
+        sm.local[tid] = run;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+        if (c0 + row_pos(IT, i) < m)
+          x.store(sm.wcnt[w][digit_of<W>(lo[i], hi[i], at)] + rank[i], lo[i], hi[i]);
+      __syncthreads();
+    }
+    x.buf ^= 1u;
+  }
+}
+
+// One walk over a sorted spilled bucket: with out, its first rows are written
+// from result row pu, root pr on; u and r are their numbers.
+template <int W, class Mem>
+__device__ __forceinline__ void spill_rows(const SpillRows<W>& x, uint32_t m, uint32_t k, bool has_prev,
+                                        uint64_t plo, uint64_t phi, bool own, uint64_t slo, uint64_t shi,
+                                        Mem& sm, const SortOut* out, uint64_t pu, uint64_t pr,
+                                        uint32_t& u, uint32_t& r) {
+  constexpr int WAVES = kBinBlock / kWave;
+  const uint32_t tid = threadIdx.x, w = tid / kWave, l = lane_id();
+  const uint32_t mm = m + (own ? 1u : 0u);
+  u = r = 0;
+  for (uint32_t c0 = 0; c0 < mm; c0 += kBinBlock) {
+    const uint32_t p = c0 + tid;
+    bool a = false, b = false;
+    uint64_t lo = slo, hi = shi, ql = plo, qh = phi;
+    if (p < mm) {
+      if (p < m) x.load(p, lo, hi);
+      if (p > 0) x.load(p - 1, ql, qh);
+      const bool none = p == 0 && !has_prev;
+      a = none || lo != ql || (W == 2 && hi != qh);
+      b = none || key_field<W>(lo, hi, k - 1) != key_field<W>(ql, qh, k - 1);
+    }
+    const uint64_t mu = ballot(a), mr = ballot(b);
+    if (l == 0) sm.firsts[w] = uint32_t(__popcll(mu)) | uint32_t(__popcll(mr)) << 16;
+    __syncthreads();
+    for (uint32_t j = 0; j < uint32_t(WAVES); ++j) {
+      if (j == w && out && a)
+        put_row<W>(*out, k, pu + u + popc_below(mu), lo, hi, b, pr + r + popc_below(mr));
+      u += sm.firsts[j] & 0xFFFFu;
+      r += sm.firsts[j] >> 16;
+    }
+    __syncthreads();
+  }
+}
+
+template <int W>
+__global__ __launch_bounds__(kBinBlock, W == 1 ? 4 : 2) void bucket_sort_kernel(BucketSort a) {
+  constexpr int WAVES = kBinBlock / kWave;
+  __shared__ SortMem<W, kBinBlock, kBinItems> sm;
+  __shared__ uint32_t s_pref[kPartTiles], s_src[kPartTiles];
+  __shared__ uint64_t s_place;
+  __shared__ uint32_t s_word[5];
+  const uint32_t tid = threadIdx.x, w = tid / kWave, l = lane_id(), k = a.k;
+  const uint64_t n = bucket_n(a);
+  const uint32_t bins = bucket_bins(n);
+  if (a.ticket) {
+    if (tid == 0) s_word[0] = atomicAdd(&a.ctl[0], 1u);
+    __syncthreads();
+  }
+  const uint32_t b = a.ticket ? s_word[0] : blockIdx.x;
+  if (b >= bins) return;  // launched for a capacity above the rows
+  const bool last = b + 1 == bins;
+
+  // Runs: position p of the bucket is part[s_src[t] + p] in the last tile t
+  // with s_pref[t] <= p.
+  const uint32_t rows = part_rows(n), tiles = uint32_t((n + rows - 1) / rows);
+  uint32_t run = 0;
+  if (tid < tiles) run = a.runs[tid * kBins + b];
+  const uint32_t at = block_scan32<WAVES>((run >> 16) - (run & 0xFFFFu), sm.wsum);
+  if (tid == kBinBlock - 1) s_word[2] = at;  // (its own run is empty)
+  if (tid < kPartTiles) {
+    s_pref[tid] = at;
+    s_src[tid] = tid * rows + (run & 0xFFFFu) - at;
+  }
+  __syncthreads();
+  const uint32_t m = s_word[2];
+  // The bucket's own rows, then the splitter that ends it unless an earlier
+  // bucket has it; the row before its first is the splitter before it.
+  const bool has_prev = b > 0 && n > 0;
+  const uint64_t plo = has_prev ? a.split[0][b - 1] : 0, phi = W == 2 && has_prev ? a.split[W - 1][b - 1] : 0;
+  const uint64_t slo = n && !last ? a.split[0][b] : 0, shi = W == 2 && n && !last ? a.split[W - 1][b] : 0;
+  const bool own = n && !last && (b == 0 || slo != plo || (W == 2 && shi != phi));
+  uint64_t pu, pr;
+  uint32_t u, r;
+  if (m + 1 <= kBinRows) {
+    const uint32_t mm = m + (own ? 1u : 0u), items = max((mm + kBinBlock - 1) / kBinBlock, 1u);
+    uint64_t lo[kBinItems], hi[kBinItems];
+    // four positions of a thread at a time, those past the end clamped, so
+    // that their searches and loads overlap
+#pragma unroll
+    for (int g = 0; g < kBinItems; g += 4) {
+      if (uint32_t(g) >= items || m == 0) {
+        for (int i = g; i < g + 4; ++i) lo[i] = hi[i] = 0;
+        continue;
+      }
+      uint32_t p[4], t[4] = {};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = min(row_pos(items, g + i), m - 1);
+#pragma unroll
+      for (uint32_t step = kPartTiles / 2; step; step >>= 1)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (s_pref[t[i] + step] <= p[i]) t[i] += step;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t q = s_src[t[i]] + p[i];
+        lo[g + i] = a.part[0][q];
+        hi[g + i] = W == 2 ? a.part[W - 1][q] : 0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kBinItems; ++i)
+      if (own && uint32_t(i) < items && row_pos(items, i) == m) {
+        lo[i] = slo;
+        hi[i] = shi;
+      }
+    block_sort<W, kBinBlock, kBinItems>(lo, hi, mm, items, sm);
+    uint32_t fu, fr, wu, wr;
+    block_firsts<W, kBinBlock, kBinItems>(lo, hi, mm, items, k, has_prev, plo, phi, sm, fu, fr, wu, wr, u, r);
+    bucket_place(a, b, u, r, &s_place, pu, pr);
+    block_write<W, kBinItems>(lo, hi, items, k, fu, fr, pu + wu, pr + wr, a.out);
+  } else {
+    if (tid == 0) s_word[1] = atomicAdd(&a.ctl[2], m);
+    __syncthreads();
+    const uint32_t room = s_word[1];
+    SpillRows<W> x{{a.part[0], a.part[1]}, {a.spill[0] + room, a.spill[1] + room}, s_pref, s_src, 0};
+    spill_sort<W>(x, m, sm);
+    spill_rows<W>(x, m, k, has_prev, plo, phi, own, slo, shi, sm, nullptr, 0, 0, u, r);
+    bucket_place(a, b, u, r, &s_place, pu, pr);
+    spill_rows<W>(x, m, k, has_prev, plo, phi, own, slo, shi, sm, &a.out, pu, pr, u, r);
+  }
+  if (!last) return;
+  if (tid == 0) {
+    a.out.root_offs[pr + r] = uint32_t(pu + u);
+    if (a.counts) {
+      const uint64_t rows_in = a.n_dev ? *a.n_dev : a.n_host;
+      a.counts[0] = pu + u;
+      a.counts[1] = pr + r;
+      a.counts[2] = (__hip_atomic_load(&a.ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 1u : 0u) |
+                    (rows_in > a.cap ? 2u : 0u);
+    }
+  }
+  if (!a.stats) return;
+  __syncthreads();
+  if (tid < 5) s_word[tid] = 0;
+  __syncthreads();
+  if (tid < tiles) {
+    for (uint32_t c = 0; c < 4; ++c) atomicMax(&s_word[c], a.stats[tid * 5 + c]);
+    atomicOr(&s_word[4], a.stats[tid * 5 + 4]);
+  }
+  __syncthreads();
+  if (tid < 5) a.maxima[tid] = s_word[tid];
+}
+
+static void bucket_sort(const BucketSort& a, hipStream_t s, bool timed = true) {
+  const uint64_t n = a.n_dev ? a.cap : a.n_host;
+  const uint32_t tiles = uint32_t(std::min<uint64_t>((n + kPartBlock - 1) / kPartBlock, kPartTiles));
+  {
+    TimeScope t(timed ? "sort.part" : nullptr, s, double(n) * (4.0 * a.k + (a.k <= 2 ? 8 : 16)));
+    if (a.k <= 2) bucket_part_kernel<1><<<tiles, kPartBlock, 0, s>>>(a);
+    else bucket_part_kernel<2><<<tiles, kPartBlock, 0, s>>>(a);
+    SRD_CHECK(hipGetLastError());
+  }
+  TimeScope t(timed ? "sort.buckets" : nullptr, s, double(n) * (4.0 * a.k + (a.k <= 2 ? 8 : 16)));
+  if (a.k <= 2) bucket_sort_kernel<1><<<bucket_bins(n), kBinBlock, 0, s>>>(a);
+  else bucket_sort_kernel<2><<<bucket_bins(n), kBinBlock, 0, s>>>(a);
+  SRD_CHECK(hipGetLastError());
+}
+
+static uint64_t align256(uint64_t b) { return (b + 255) & ~uint64_t(255); }
+
+// Bytes of a sort's tables (all but its rows), and the tables in them.
+constexpr uint64_t kBucketRuns = uint64_t(kPartTiles) * kBins * 4;
+constexpr uint64_t kBucketTables = kBucketRuns + 3 * uint64_t(kBins) * 8 + 256 + kPartTiles * 5 * 4;
+
+static void bucket_tables(BucketSort& a, uint8_t* p) {
+  a.runs = reinterpret_cast<uint32_t*>(p);
+  a.split[0] = reinterpret_cast<uint64_t*>(p + kBucketRuns);
+  a.split[1] = a.split[0] + kBins;
+  a.lookback = a.split[1] + kBins;
+  a.ctl = reinterpret_cast<uint32_t*>(a.lookback + kBins);
+  a.stats = a.ctl + 64;
 }
 
 // ==================================================== sort: host driver ====
@@ -1859,10 +2583,7 @@ void build_index(const uint32_t* const* in, uint32_t k, uint64_t n, Index& out, 
     ws.small_out.reserve(3 + kMaxCols, s);
     SmallSort a{};
     for (uint32_t c = 0; c < k; ++c) a.in[c] = in[c];
-    a.cols = out.cols.p;
-    a.stride = out.stride;
-    a.root_vals = out.root_vals.p;
-    a.root_offs = out.root_offs.p;
+    a.out = {out.cols.p, out.stride, out.root_vals.p, out.root_offs.p};
     a.counts = ws.small_out.p;
     a.maxima = reinterpret_cast<uint32_t*>(ws.small_out.p + 3);
     a.n = uint32_t(n);
@@ -1876,6 +2597,64 @@ void build_index(const uint32_t* const* in, uint32_t k, uint64_t n, Index& out, 
     const uint32_t* mx = reinterpret_cast<const uint32_t*>(h + 3);
     for (uint32_t c = 0; c < k; ++c)
       out.col_max[c] = col_max && col_max->size() == k ? (*col_max)[c] : mx[c];
+    return;
+  }
+
+  if (n <= kBucketRows && k <= 4 && !presorted) {
+    // two launches and one read-back
+    const int W = k <= 2 ? 1 : 2;
+    for (int b = 0; b < 2; ++b)
+      for (int wd = 0; wd < W; ++wd) ws.keys[b][wd].reserve(n, s);
+    ws.bucket.reserve(kBucketTables, s);
+    ws.small_out.reserve(3 + kMaxCols, s);
+    out.stride = round_stride(n);
+    out.cols.alloc(out.stride * k, s);
+    out.root_vals.alloc(n, s);
+    out.root_offs.alloc(n + 1, s);
+    BucketSort a{};
+    for (uint32_t c = 0; c < k; ++c) a.in[c] = in[c];
+    a.k = k;
+    a.n_host = a.cap = n;
+    for (int wd = 0; wd < W; ++wd) {
+      a.part[wd] = ws.keys[0][wd].p;
+      a.spill[wd] = ws.keys[1][wd].p;
+    }
+    bucket_tables(a, ws.bucket.p);
+    a.out = {out.cols.p, out.stride, out.root_vals.p, out.root_offs.p};
+    a.counts = ws.small_out.p;
+    a.maxima = reinterpret_cast<uint32_t*>(ws.small_out.p + 3);
+    a.ticket = ws.ticket_order;
+    bucket_sort(a, s);
+    uint64_t* h = reinterpret_cast<uint64_t*>(pinned_words(ws, 2 * (3 + kMaxCols)));
+    SRD_CHECK(hipMemcpyAsync(h, ws.small_out.p, (3 + kMaxCols) * 8, hipMemcpyDeviceToHost, s));
+    SRD_CHECK(hipStreamSynchronize(s));
+    if (h[2] != 0) fail("build_index: radix sort look-back did not resolve");
+    out.n = h[0];
+    out.r = uint32_t(h[1]);
+    const uint32_t* mx = reinterpret_cast<const uint32_t*>(h + 3);
+    const bool hint = col_max && col_max->size() == k;
+    for (uint32_t c = 0; c < k; ++c) out.col_max[c] = hint ? (*col_max)[c] : mx[c];
+    if (!hint && mx[4] == 0 && adopt && adopt->p) {
+      // strictly increasing: the caller's columns are the index
+      out.cols = *adopt;
+      out.stride = adopt_stride;
+    } else if (out.n <= n / 2) {
+      // many repeats: keep only what the distinct rows need
+      DevBuf<uint32_t> cols, vals, offs;
+      const uint64_t st = round_stride(out.n);
+      cols.alloc(st * k, s);
+      vals.alloc(out.r, s);
+      offs.alloc(uint64_t(out.r) + 1, s);
+      SRD_CHECK(hipMemcpy2DAsync(cols.p, st * 4, out.cols.p, out.stride * 4, out.n * 4, k,
+                                 hipMemcpyDeviceToDevice, s));
+      SRD_CHECK(hipMemcpyAsync(vals.p, out.root_vals.p, uint64_t(out.r) * 4, hipMemcpyDeviceToDevice, s));
+      SRD_CHECK(hipMemcpyAsync(offs.p, out.root_offs.p, (uint64_t(out.r) + 1) * 4,
+                               hipMemcpyDeviceToDevice, s));
+      out.cols = cols;
+      out.root_vals = vals;
+      out.root_offs = offs;
+      out.stride = st;
+    }
     return;
   }
 
@@ -2117,8 +2896,6 @@ struct DevSortScratch {
   uint64_t* scan_tmp;       // multi-level scan partials (scan_noalloc_words)
 };
 
-static uint64_t align256(uint64_t b) { return (b + 255) & ~uint64_t(255); }
-
 // u64 words of partial sums a scan of n entries needs beyond its output.
 static uint64_t scan_noalloc_words(uint64_t n) {
   if (n <= kTile) return 0;
@@ -2149,6 +2926,7 @@ static void scan_noalloc(const T* in, uint64_t* out, uint64_t n, uint64_t* tmp, 
 // out), so one scratch serves every key width without moving its look-back
 // words: a look-back word is only ever written as one.
 uint64_t devsort_scratch_bytes(uint64_t cap) {
+  if (cap <= kBucketRows) return 4 * align256(cap * 8) + kBucketTables;
   const uint64_t lb_tiles = (cap + kOsMinTile - 1) / kOsMinTile;
   const uint64_t dt = (cap + kTile - 1) / kTile;
   uint64_t b = align256(sizeof(DevPlan));
@@ -2485,14 +3263,32 @@ void build_index_dev(const uint32_t* const* in, uint32_t k, uint64_t cap, const 
     TimeScope t(timed ? "sort.small" : nullptr, s);
     SmallSort a{};
     for (uint32_t c = 0; c < k; ++c) a.in[c] = in[c];
-    a.cols = out_cols;
-    a.stride = out_stride;
-    a.root_vals = root_vals;
-    a.root_offs = root_offs;
+    a.out = {out_cols, out_stride, root_vals, root_offs};
     a.counts = counts_out;
     a.n = uint32_t(n_host);
     a.k = k;
     small_sort(a, s);
+    return;
+  }
+  if (cap <= kBucketRows) {
+    if (w != (k <= 2 ? 1u : 2u)) fail("build_index_dev: two key words from three columns on");
+    BucketSort a{};
+    for (uint32_t c = 0; c < k; ++c) a.in[c] = in[c];
+    a.k = k;
+    a.n_host = n_host;
+    a.n_dev = n_dev;
+    a.cap = cap;
+    uint8_t* p = static_cast<uint8_t*>(scratch);
+    for (int i = 0; i < 2; ++i) {
+      a.part[i] = reinterpret_cast<uint64_t*>(p + i * align256(cap * 8));
+      a.spill[i] = reinterpret_cast<uint64_t*>(p + (2 + i) * align256(cap * 8));
+    }
+    bucket_tables(a, p + 4 * align256(cap * 8));
+    a.stats = nullptr;
+    a.out = {out_cols, out_stride, root_vals, root_offs};
+    a.counts = counts_out;
+    a.ticket = ticket;
+    bucket_sort(a, s, timed);
     return;
   }
   DevSortScratch x = carve_devsort(scratch, cap);
@@ -2566,6 +3362,7 @@ void build_index_dev(const uint32_t* const* in, uint32_t k, uint64_t cap, const 
 }
 
 void devsort_clear_lookback(void* scratch, uint64_t cap, hipStream_t s) {
+  if (cap <= kBucketRows) return;  // each sort clears its own
   DevSortScratch x = carve_devsort(scratch, cap);
   fill_u64(x.lookback, 0, x.lookback_words, s);
   fill_u32(x.epoch_ctr, 0, 1, s);

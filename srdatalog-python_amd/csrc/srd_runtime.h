@@ -191,7 +191,8 @@ struct Workspace {
   DevBuf<uint64_t> tile_scan;    // per-tile offsets
   DevBuf<uint8_t> flags;
   DevBuf<uint32_t> hostbuf_dev;  // staging for values read back
-  DevBuf<uint64_t> small_out;    // counts and maxima of a one-launch sort
+  DevBuf<uint64_t> small_out;    // counts and maxima of a sort without passes
+  DevBuf<uint8_t> bucket;        // run, splitter and look-back tables of a bucket sort
   uint32_t epoch = 0;            // lookback epoch (avoids per-pass clears)
   DevBuf<uint64_t> mp_lb;        // merge-path set-difference inter-tile state
   DevBuf<uint64_t> mp_split;     // merge-path tile split points
@@ -230,15 +231,17 @@ void build_index_from(const Index& src, const std::vector<uint32_t>& perm, Index
 // Device-planned sort + dedup: build_index without host read-backs or
 // allocations.  Rows: n_dev (device word, may be null) or n_host, at most
 // `cap` (launch shapes come from cap).  w = key words (1 suffices for k <= 2;
-// 2 for k <= 4 columns of any width).  scratch: devsort_scratch_bytes(cap)
-// bytes, 256-byte aligned; its layout depends on cap alone, so a scratch
-// reused across calls must always be given the same cap (its look-back
-// words would otherwise overlap earlier calls' keys).  Outputs: out_cols (k columns, out_stride apart,
+// 2 for k <= 4 columns of any width; up to 2^20 rows of capacity exactly
+// these).  scratch: devsort_scratch_bytes(cap) bytes, 256-byte aligned; its
+// layout depends on cap alone, so a scratch reused across calls must always be
+// given the same cap (beyond 2^20 rows its look-back words would otherwise
+// overlap earlier calls' keys).  Outputs: out_cols (k columns, out_stride apart,
 // cap rows), root_vals (cap), root_offs (cap + 1) and, if counts_out is not
 // null, counts_out[0..2] = distinct rows, distinct column-0 values, error
 // bits (1: a look-back did not resolve, 2: rows above cap, 4: key wider
-// than w words).  The look-back epochs are kept in the scratch itself and
-// advanced by a kernel, so a captured sort can be replayed; ticket: take tile order
+// than w words).  A captured sort can be replayed: up to 2^20 rows each sort
+// clears its own look-back words, beyond that their epochs are kept in the
+// scratch and advanced by a kernel; ticket: take tile order
 // from tickets (required when other work may share the GPU); timed: record
 // the launches in the kernel timing (false: no events are created).
 uint64_t devsort_scratch_bytes(uint64_t cap);
@@ -247,7 +250,7 @@ void build_index_dev(const uint32_t* const* in, uint32_t k, uint64_t cap, const 
                      uint64_t out_stride, uint32_t* root_vals, uint32_t* root_offs,
                      uint64_t* counts_out, bool ticket, hipStream_t s, bool timed = true);
 // Zero the look-back words and epoch of a devsort scratch (once, before its
-// first use).
+// first use; nothing to do up to 2^20 rows).
 void devsort_clear_lookback(void* scratch, uint64_t cap, hipStream_t s);
 
 // ------------------------------------------------ device-sized primitives --
