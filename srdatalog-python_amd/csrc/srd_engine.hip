@@ -266,6 +266,7 @@ struct srd_engine {
   std::vector<srd::Step> steps;
   std::map<std::string, const SrdPipelineDesc*> pipes;
   std::map<std::string, const SrdPipelineExt*> exts;
+  std::set<std::string> copies;  // rules whose source index is their result (see pr_copy)
   hipStream_t s = nullptr;
   srd::Workspace ws;
   std::string err;
@@ -329,6 +330,9 @@ struct srd_engine {
   // SRDATALOG_MARK_UNION=0: products are walked per level-1 value, never per
   // root key over the union of its values
   bool mark_union = true;
+  // SRDATALOG_COPY_SHARE=0: rules that only copy a relation derive its rows
+  // one by one like any other.
+  bool copy_share = true;
   uint64_t mark_chunk_slices = 0;  // SRDATALOG_MARK_CHUNK_SLICES (0: one launch per traversal)
   uint32_t weigh_ranges = SRD_XCDS;  // SRDATALOG_WEIGH_RANGES: of the weigh launch
   // column-1 bitmaps of heavy keys for views nested levels search
@@ -811,6 +815,7 @@ struct PipeRun {
   hipStream_t s = nullptr;
   SrdLaunchArgs a;
   std::vector<uint32_t> view_max[SRD_MAX_VIEWS];
+  const Index* view_index[SRD_MAX_VIEWS] = {};
   uint64_t* host = nullptr;   // 4 pinned words for this pipeline's read-backs
   uint64_t total = 0;         // tuples emitted
   uint64_t slices = 0;
@@ -875,6 +880,7 @@ static void pr_views(srd_engine& e, PipeRun& R, uint64_t iteration) {
     else
       x = &new_index(e, r, order);
     R.view_max[v] = x->col_max;
+    R.view_index[v] = x;
     if (vs.want_bitmaps && x->arity == 2 && e.bitmap_bytes) {
       const HeavyBits* h = x->heavy.get();
       if (!h || h->built_for != x->cols.p || h->built_n != x->n) {
@@ -1448,6 +1454,36 @@ static void pr_union(srd_engine& e, PipeRun& R, uint64_t iteration) {
 // phase.  A group's members each get a stream and scratch of their own (a
 // member counting probes or needing the chunked or overflow path finishes
 // on the engine's stream, after the others).
+// A rule that copies a relation column by column, in the column order of the
+// index it reads: that index, already sorted and without repeats, becomes a
+// part of NEW as it is (indexes share their columns).  Deriving the rows
+// instead marks or writes them, extracts or sorts them and builds their roots
+// again: 320 us for the 2.2e5 edges of an R-MAT graph of scale 14.
+static bool pr_copy(srd_engine& e, PipeRun& R) {
+  if (!e.copy_share || e.two_pass || e.no_direct || e.count_probes || !e.copies.count(R.d->rule)) return false;
+  const SrdDestSpec& to = R.d->dest[0];
+  Relation& r = e.rels[rel_id(e, to.rel)];
+  const Order order(to.cols, to.cols + to.arity);
+  if (!r.newv.empty() || (r.raw_n > 0 && r.raw_order != order) ||
+      (!r.new_parts.empty() && r.new_parts_order != order))
+    return false;
+  const Index& x = *R.view_index[R.a.drv_view];
+  if (x.n > 0) {
+    Index part;
+    copy_index(x, part, e.s);
+    add_new_part(e, r, order, std::move(part));
+  }
+  // join_tuples leaves out the tuples of rules that mark a bitmap: this rule's
+  // count where it would have written rows
+  uint32_t bound = value_bound(e);
+  for (uint32_t m : R.view_max[R.a.drv_view]) bound = std::max(bound, m);
+  const uint64_t bits = uint64_t(std::max<uint32_t>(32 - __builtin_clz(bound | 1u), 1)) * r.arity;
+  R.total = bits <= 40 && (uint64_t(1) << bits) <= e.dense_max_bits ? 0 : x.n;
+  R.mode = 1;
+  R.a.n_root = 0;  // nothing left to run
+  return true;
+}
+
 static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc*>& ds,
                           uint64_t iteration) {
   const size_t P = ds.size();
@@ -1484,7 +1520,7 @@ static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc
       R.s = e.s;
       R.host = pins;
       pr_views(e, R, iteration);
-      {
+      if (!pr_copy(e, R)) {
         std::vector<PipeRun*> me{&R};
         pr_dense(e, me);
         pr_union(e, R, iteration);
@@ -1524,9 +1560,10 @@ static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc
   }
   {
     std::vector<PipeRun*> all;
-    for (auto& R : runs) all.push_back(&R);
+    for (auto& R : runs)
+      if (!pr_copy(e, R)) all.push_back(&R);
     pr_dense(e, all);
-    for (auto& R : runs) pr_union(e, R, iteration);
+    for (PipeRun* R : all) pr_union(e, *R, iteration);
   }
   // every member reads indexes built on the engine's stream (and the
   // bitmaps cleared there)
@@ -3518,6 +3555,7 @@ srd_engine* srd_engine_create_ext(const char* text, const SrdPipelineDesc* pipes
       e->xcd_ranges = std::min<uint32_t>(std::max<uint32_t>(uint32_t(std::atoi(c)), 1), SRD_XCDS);
     if (const char* c = std::getenv("SRDATALOG_MARK_CHUNK_SLICES"))
       e->mark_chunk_slices = std::strtoull(c, nullptr, 10);
+    if (const char* c = std::getenv("SRDATALOG_COPY_SHARE")) e->copy_share = !(*c == '0' && c[1] == 0);
     if (const char* c = std::getenv("SRDATALOG_MARK_UNION")) e->mark_union = !(*c == '0' && c[1] == 0);
     if (const char* c = std::getenv("SRDATALOG_MARK_PRODUCTS"))
       e->mark_products = !(*c == '0' && c[1] == 0);
@@ -3571,6 +3609,21 @@ srd_engine* srd_engine_create_ext(const char* text, const SrdPipelineDesc* pipes
     }
     for (uint32_t i = 0; i < n; ++i) e->pipes[pipes[i].rule] = &pipes[i];
     for (uint32_t i = 0; i < n_exts; ++i) e->exts[exts[i].rule] = &exts[i];
+    // a copy's rows enter NEW in its own column order: every rule that writes
+    // the relation has to write that order
+    for (uint32_t i = 0; i < n_exts; ++i) {
+      const auto d = e->pipes.find(exts[i].rule);
+      if (!exts[i].copy || d == e->pipes.end()) continue;
+      const SrdDestSpec& to = d->second->dest[0];
+      bool same = true;
+      for (uint32_t j = 0; j < n; ++j)
+        for (uint32_t k = 0; k < pipes[j].n_dest; ++k) {
+          const SrdDestSpec& o = pipes[j].dest[k];
+          same = same && (std::strcmp(o.rel, to.rel) != 0 ||
+                          (o.arity == to.arity && std::equal(o.cols, o.cols + o.arity, to.cols)));
+        }
+      if (same) e->copies.insert(exts[i].rule);
+    }
     parse_program(*e, text);
   } catch (const std::exception& ex) {
     std::cerr << "srdatalog_init: " << ex.what() << std::endl;

@@ -268,6 +268,9 @@ struct SrdPipelineExt {
   const struct SrdPipelineDesc* uni;
   uint32_t uni_view, uni_minor, uni_row_col;
   int32_t uni_root_col;
+  // the rule copies one relation: its row, in the destination's index order, is
+  // the scanned index's row
+  uint32_t copy;
 };
 
 #ifdef __cplusplus

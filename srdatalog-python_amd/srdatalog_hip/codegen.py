@@ -324,6 +324,15 @@ class PipelineGen:
     return 1 <= len(d.index) <= 4 and all(isinstance(d.terms[c], str) and not is_const(d.terms[c])
                                           for c in d.index)
 
+  def copy_ok(self) -> bool:
+    """The rule scans one index and writes its rows as they are, in the
+    destination's index order."""
+    if not isinstance(self.root, M.Scan) or not self.direct_ok() or not self.mark_ok():
+      return False
+    d, row = self.dests[0], list(self.root.vars)
+    return (not self.root.prefix and len(row) == len(self.root.index) and len(set(row)) == len(row)
+            and "_" not in row and row == [d.terms[c] for c in d.index])
+
   def direct_ok(self) -> bool:
     """Every level-1 item yields exactly one tuple: no filters, and either a
     scan root, a root join with no nested level, or a cartesian last level
@@ -1377,7 +1386,7 @@ class PipelineGen:
       own = lv.sources[p["jr"] if minor else p["jm"]]
       root = p["bound"][0][0] if p["bound"] else -1
       uni = f"&{g.ns}::k_desc, {self.vid(own)}, {1 if minor else 0}, {p['cr']}, {root}"
-    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}, {dyn}, {uni}}}"
+    return f"  {{\"{self.ep.rule}\", {self.prod_kind()}, {dyn}, {uni}, {1 if self.copy_ok() else 0}}}"
 
   def gen_desc(self) -> str:
     views = []
