@@ -1254,6 +1254,21 @@ __device__ __forceinline__ uint32_t wave_scan32(uint32_t v, uint32_t id, Op op) 
   return v;
 }
 
+// The same for sums of 64-bit values.
+__device__ __forceinline__ uint64_t wave_scan64(uint64_t v) {
+#define SRD_DPP(CTRL, ROWS)                                                                        \
+  v += uint64_t(uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v)), CTRL, ROWS, 0xF, false))) | \
+       uint64_t(uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v >> 32)), CTRL, ROWS, 0xF, false))) << 32
+  SRD_DPP(0x111, 0xF);
+  SRD_DPP(0x112, 0xF);
+  SRD_DPP(0x114, 0xF);
+  SRD_DPP(0x118, 0xF);
+  SRD_DPP(0x142, 0xA);
+  SRD_DPP(0x143, 0xC);
+#undef SRD_DPP
+  return v;
+}
+
 __device__ __forceinline__ uint32_t wave_add32(uint32_t v) {
   return __builtin_amdgcn_readlane(wave_scan32(v, 0, [](uint32_t a, uint32_t b) { return a + b; }), 63);
 }
@@ -4457,7 +4472,7 @@ __global__ __launch_bounds__(kDenseWg) void dense_count_blocks_kernel(const Dens
     const uint64_t at = w0 + uint64_t(w * kDenseWaveChunks + i) * kWave + l;
     x[i] = r.nw[at];
     if (r.fl) x[i] &= ~r.fl[at];
-    const uint32_t pc = wave_sum<uint32_t>(__popcll(x[i]));
+    const uint32_t pc = wave_add32(__popcll(x[i]));
     if (l == 0) s_cnt[w * kDenseWaveChunks + i] = pc;
   }
   __syncthreads();
@@ -4477,7 +4492,8 @@ __global__ __launch_bounds__(kDenseWg) void dense_count_blocks_kernel(const Dens
   __syncthreads();
   if (w != 0) return;
   const uint32_t rmine = r.k > 1 ? s_root[l] : 0u;
-  const uint32_t cincl = wave_incl_scan<uint32_t>(mine), rincl = wave_incl_scan<uint32_t>(rmine);
+  const auto add = [](uint32_t p, uint32_t q) { return p + q; };
+  const uint32_t cincl = wave_scan32(mine, 0, add), rincl = wave_scan32(rmine, 0, add);
   r.chunk[b * kDenseChunks + l] = chunk_pack(cincl - mine, rincl - rmine, cont);
   if (l == kWave - 1) r.blk[b] = uint64_t(cincl) | (uint64_t(rincl) << kDenseRowBits);
 }
@@ -4507,7 +4523,8 @@ __global__ __launch_bounds__(kBlock) void dense_emit_blocks_kernel(const DenseCt
     const uint64_t ck = r.chunk[b * kDenseChunks + ch];
     const uint64_t first = chunk_firsts(x, rs, ck >> 63);
     const uint32_t p = __popcll(x);
-    const uint32_t base = row0 + uint32_t(ck & 0xFFFFFu) + wave_incl_scan<uint32_t>(p) - p;
+    const uint32_t base =
+        row0 + uint32_t(ck & 0xFFFFFu) + wave_scan32(p, 0, [](uint32_t a, uint32_t b) { return a + b; }) - p;
     const uint32_t groot = root0 + uint32_t((ck >> 20) & 0xFFFFFu);
     for (uint64_t nz = ballot(x != 0); nz; nz &= nz - 1) {
       const int j = __builtin_ctzll(nz);
@@ -4549,37 +4566,45 @@ static uint32_t dense_emit_parts(const DenseRel& r) {
   return r.nblocks <= 256 ? 16u : (r.nblocks <= 2048 ? 4u : 1u);
 }
 
-// Exclusive scan of n u64 in place by one workgroup; returns the total.
+// Exclusive scan of n u64 in place by one workgroup; returns the total.  Up to
+// eight items a lane, no more than spread n over all waves: a scan of 1,000
+// keys is one item a lane, its wave scans DPP moves (dense_plan_kernel
+// 3.7 us, with eight items on two waves and shuffles 6.8).
 __device__ __forceinline__ uint64_t scan_u64_wg(const uint64_t* in, uint64_t* out, uint64_t n,
                                                 uint64_t* s_w) {
   constexpr int V = 8;
   const uint32_t w = threadIdx.x / kWave, l = lane_id();
+  const uint32_t per = uint32_t(min<uint64_t>((n + kDenseWg - 1) / kDenseWg, V));
   uint64_t carry = 0;
-  for (uint64_t t0 = 0; t0 < n; t0 += uint64_t(V) * kDenseWg) {
-    // lane l of wave w: items t0 + (w*V + i)*64 + l
-    uint64_t v[V], run = 0;
+  for (uint64_t t0 = 0; t0 < n; t0 += uint64_t(per) * kDenseWg) {
+    // lane l of wave w: items t0 + (w*per + i)*64 + l
+    uint64_t v[V], off = 0;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      const uint64_t at = t0 + uint64_t(w * V + i) * kWave + l;
-      v[i] = at < n ? in[at] : 0;
-      run += v[i];
+      const uint64_t at = t0 + uint64_t(w * per + i) * kWave + l;
+      v[i] = uint32_t(i) < per && at < n ? in[at] : 0;
     }
-    run = wave_sum<uint64_t>(run);
+    // each item's inclusive sum in its wave, the wave's items before it added
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      if (uint32_t(i) >= per) continue;
+      const uint64_t inc = wave_scan64(v[i]);
+      v[i] = off + inc - v[i];
+      off += read_lane_u64(inc, kWave - 1);
+    }
     __syncthreads();  // s_w of the tile before is read
-    if (l == 0) s_w[w] = run;
+    if (l == 0) s_w[w] = off;
     __syncthreads();
-    uint64_t off = carry;
+    uint64_t before = carry;
     for (int j = 0; j < kDenseWgWaves; ++j) {
       const uint64_t x = s_w[j];
-      if (uint32_t(j) < w) off += x;
+      if (uint32_t(j) < w) before += x;
       carry += x;
     }
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      const uint64_t inc = wave_incl_scan<uint64_t>(v[i]);
-      const uint64_t at = t0 + uint64_t(w * V + i) * kWave + l;
-      if (at < n) out[at] = off + inc - v[i];
-      off += read_lane_u64(inc, kWave - 1);
+      const uint64_t at = t0 + uint64_t(w * per + i) * kWave + l;
+      if (uint32_t(i) < per && at < n) out[at] = before + v[i];
     }
   }
   return carry;
