@@ -331,6 +331,22 @@ def split_nonrec_program() -> Program:
   return Program(rules=[(q(x, z) <= a(x, y) & ~b(y) & SPLIT & c(x, z)).named("SplitTest")])
 
 
+def products_program() -> Program:
+  """Rules that end in a product of two sources, in the forms that decide
+  how the product is marked; written for this package's tests."""
+  r, x, y = (Var(n) for n in ("r", "x", "y"))
+  a = Relation("A", 2, input_file="A.csv")
+  u = Relation("U", 1, input_file="U.csv")
+  s = Relation("S", 1, input_file="S.csv")
+  indep = Relation("Indep", 2, print_size=True)
+  indep_key = Relation("IndepKey", 3, print_size=True)
+  return Program(rules=[
+    # one side does not depend on the root key
+    (indep(x, y) <= a(r, x) & u(r) & s(y)).named("IndepPairs"),
+    (indep_key(r, x, y) <= a(r, x) & u(r) & s(y)).named("IndepTriples"),
+  ])
+
+
 PROGRAMS = {
   "tc": tc_program,
   "sg": sg_program,
@@ -352,6 +368,7 @@ PROGRAMS = {
   "typelookup": typelookup_program,
   "cspa": cspa_program,
   "galen": galen_program,
+  "products": products_program,
 }
 
 

@@ -1,0 +1,23 @@
+"""Which products the generator marks row by row, and which it leaves to the
+tuple walk: the rules of the `products` program, and its source whole."""
+from srdatalog_hip import codegen, compiler, programs
+
+
+def gens():
+  prog = programs.PROGRAMS["products"]()
+  arity = {d.name: d.arity for d in compiler.relation_decls(prog)}
+  mir = compiler.compile_to_mir(prog)
+  return {ep.rule: codegen.PipelineGen(ep, arity, i) for i, ep in enumerate(mir.pipelines())}
+
+
+def test_every_rule_is_generated():
+  prog = programs.PROGRAMS["products"]()
+  src = codegen.generate_program_source("products", compiler.relation_decls(prog),
+                                        compiler.compile_to_mir(prog))
+  for rule in gens():
+    assert f'{{"{rule}"' in src
+
+
+def test_a_side_without_the_root_key_is_walked_by_tuples():
+  g = gens()
+  assert g["IndepPairs"].prod_kind() == 0 and g["IndepTriples"].prod_kind() == 0
