@@ -256,7 +256,8 @@ class PipelineGen:
     left to apply, and a destination index whose last column is one of the
     two variables (`m`, from source `jm`) and one other column the other one
     (`r`, from `jr`, at index column `cr`); the remaining columns are
-    bound.  Under the root both sources depend on its key."""
+    bound.  Under the root both sources depend on its key, and the rule has
+    no check."""
     if not self.mark_ok() or not isinstance(lv, M.CartesianJoin) or lv is not self.levels[-1]:
       return None
     if isinstance(self.root, M.Scan):
@@ -264,9 +265,10 @@ class PipelineGen:
     if len(lv.sources) != 2 or not all(len(vs) == 1 for vs in lv.var_from_source or ()):
       return None
     if lv is self.levels[0]:
-      # the walk under the root reads a key's ranges from the root launch
+      # the walk under the root reads a key's ranges from the root launch and
+      # applies no check (one below the root is applied before its product)
       slots = self.root_slots()
-      if any((self.vid(s_), tuple(s_.prefix)) not in slots for s_ in lv.sources):
+      if self.filters or any((self.vid(s_), tuple(s_.prefix)) not in slots for s_ in lv.sources):
         return None
     cart = [vs[0] for vs in lv.var_from_source]
     for f in self.filters:

@@ -336,14 +336,20 @@ def products_program() -> Program:
   how the product is marked; written for this package's tests."""
   r, x, y = (Var(n) for n in ("r", "x", "y"))
   a = Relation("A", 2, input_file="A.csv")
+  c = Relation("C", 2, input_file="C.csv")
   u = Relation("U", 1, input_file="U.csv")
   s = Relation("S", 1, input_file="S.csv")
   indep = Relation("Indep", 2, print_size=True)
   indep_key = Relation("IndepKey", 3, print_size=True)
+  neg = Relation("RootNeg", 2, print_size=True)
+  filt = Relation("RootFilter", 2, print_size=True)
   return Program(rules=[
     # one side does not depend on the root key
     (indep(x, y) <= a(r, x) & u(r) & s(y)).named("IndepPairs"),
     (indep_key(r, x, y) <= a(r, x) & u(r) & s(y)).named("IndepTriples"),
+    # a check on the root key alone
+    (neg(x, y) <= a(r, x) & c(r, y) & ~u(r)).named("RootNegation"),
+    (filt(x, y) <= a(r, x) & c(r, y) & Filter(("r",), "return r != 3u;")).named("RootFilter"),
   ])
 
 

@@ -21,3 +21,8 @@ def test_every_rule_is_generated():
 def test_a_side_without_the_root_key_is_walked_by_tuples():
   g = gens()
   assert g["IndepPairs"].prod_kind() == 0 and g["IndepTriples"].prod_kind() == 0
+
+
+def test_a_checked_root_key_is_walked_by_tuples():
+  g = gens()
+  assert g["RootNegation"].prod_kind() == 0 and g["RootFilter"].prod_kind() == 0

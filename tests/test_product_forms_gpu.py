@@ -24,7 +24,7 @@ def inputs(seed, dense):
     return np.unique(e.astype(np.uint32), axis=0)
 
   rows = 2000 if dense else 60
-  return {"A": rel(keys, top, rows),
+  return {"A": rel(keys, top, rows), "C": rel(keys, top, rows),
           "U": np.array([[0], [2], [3], [7]], np.uint32),
           "S": np.unique(rng.integers(0, top, 200 if dense else 9).astype(np.uint32)).reshape(-1, 1)}
 
@@ -38,12 +38,14 @@ def by_key(rows):
 
 def model(i):
   """Relation -> set of tuples."""
-  a = by_key(i["A"])
+  a, c = by_key(i["A"]), by_key(i["C"])
   u = set(i["U"][:, 0].tolist())
   s = i["S"][:, 0].tolist()
   return {
     "Indep": {(x, y) for r in a if r in u for x in a[r] for y in s},
     "IndepKey": {(r, x, y) for r in a if r in u for x in a[r] for y in s},
+    "RootNeg": {(x, y) for r in a if r in c and r not in u for x in a[r] for y in c[r]},
+    "RootFilter": {(x, y) for r in a if r in c and r != 3 for x in a[r] for y in c[r]},
   }
 
 
