@@ -294,7 +294,9 @@ class PipelineGen:
       return None
     r, lv1, lv2 = self.root, *self.levels
     p = self.prod_level(lv2)
-    if not p or not isinstance(lv1, M.ColumnJoin) or any(v != r.var for _, v in p["bound"]):
+    # union_products adds the root variable at one index column at most
+    if (not p or not isinstance(lv1, M.ColumnJoin) or len(p["bound"]) > 1
+        or any(v != r.var for _, v in p["bound"])):
       return None
     dep = [lv1.var in s_.prefix for s_ in lv2.sources]
     if dep[0] == dep[1]:

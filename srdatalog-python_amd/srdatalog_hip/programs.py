@@ -334,8 +334,9 @@ def split_nonrec_program() -> Program:
 def products_program() -> Program:
   """Rules that end in a product of two sources, in the forms that decide
   how the product is marked; written for this package's tests."""
-  r, x, y = (Var(n) for n in ("r", "x", "y"))
+  l, r, x, y = (Var(n) for n in ("l", "r", "x", "y"))
   a = Relation("A", 2, input_file="A.csv")
+  b = Relation("B", 2, input_file="B.csv")
   c = Relation("C", 2, input_file="C.csv")
   u = Relation("U", 1, input_file="U.csv")
   s = Relation("S", 1, input_file="S.csv")
@@ -343,6 +344,7 @@ def products_program() -> Program:
   indep_key = Relation("IndepKey", 3, print_size=True)
   neg = Relation("RootNeg", 2, print_size=True)
   filt = Relation("RootFilter", 2, print_size=True)
+  twice = Relation("RootTwice", 4, print_size=True)
   return Program(rules=[
     # one side does not depend on the root key
     (indep(x, y) <= a(r, x) & u(r) & s(y)).named("IndepPairs"),
@@ -350,6 +352,8 @@ def products_program() -> Program:
     # a check on the root key alone
     (neg(x, y) <= a(r, x) & c(r, y) & ~u(r)).named("RootNegation"),
     (filt(x, y) <= a(r, x) & c(r, y) & Filter(("r",), "return r != 3u;")).named("RootFilter"),
+    # the root variable in two columns of the head
+    (twice(r, r, x, y) <= a(r, l) & b(l, x) & c(r, y)).named("RootTwice"),
   ])
 
 

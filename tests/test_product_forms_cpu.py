@@ -26,3 +26,10 @@ def test_a_side_without_the_root_key_is_walked_by_tuples():
 def test_a_checked_root_key_is_walked_by_tuples():
   g = gens()
   assert g["RootNegation"].prod_kind() == 0 and g["RootFilter"].prod_kind() == 0
+
+
+def test_a_union_adds_the_root_variable_once():
+  """union_products knows one index column of the root variable."""
+  g = gens()["RootTwice"]
+  assert g.union_gen() is None and g.prod_kind() == 2
+  assert g.gen_ext().strip() == '{"RootTwice", 2, nullptr, nullptr, 0, 0, 0, -1, 0}'

@@ -17,14 +17,14 @@ def inputs(seed, dense):
   """Few keys with products of hundreds to thousands of tuples, ids below 400
   (so that four columns are marked too)."""
   rng = np.random.default_rng(seed)
-  keys, mids, top = 9, 30, 400
+  keys, top = 9, 400
 
   def rel(n_left, n_right, rows):
     e = np.stack([rng.integers(0, n_left, rows), rng.integers(0, n_right, rows)], 1)
     return np.unique(e.astype(np.uint32), axis=0)
 
   rows = 2000 if dense else 60
-  return {"A": rel(keys, top, rows), "C": rel(keys, top, rows),
+  return {"A": rel(keys, top, rows), "B": rel(top, top, 4 * rows), "C": rel(keys, top, rows),
           "U": np.array([[0], [2], [3], [7]], np.uint32),
           "S": np.unique(rng.integers(0, top, 200 if dense else 9).astype(np.uint32)).reshape(-1, 1)}
 
@@ -38,7 +38,7 @@ def by_key(rows):
 
 def model(i):
   """Relation -> set of tuples."""
-  a, c = by_key(i["A"]), by_key(i["C"])
+  a, b, c = by_key(i["A"]), by_key(i["B"]), by_key(i["C"])
   u = set(i["U"][:, 0].tolist())
   s = i["S"][:, 0].tolist()
   return {
@@ -46,6 +46,8 @@ def model(i):
     "IndepKey": {(r, x, y) for r in a if r in u for x in a[r] for y in s},
     "RootNeg": {(x, y) for r in a if r in c and r not in u for x in a[r] for y in c[r]},
     "RootFilter": {(x, y) for r in a if r in c and r != 3 for x in a[r] for y in c[r]},
+    "RootTwice": {(r, r, x, y) for r in a if r in c
+                  for x in {v for m in a[r] for v in b.get(m, ())} for y in c[r]},
   }
 
 
