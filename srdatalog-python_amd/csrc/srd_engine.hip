@@ -2961,11 +2961,18 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
         if (q != hipErrorNotReady) SRD_CHECK(q);
       }
     }
+    // The words beside the tick may already be a later block's, whose tick is
+    // still on its way.  An overflow ends everything sent, so the state is
+    // taken once the stream is idle: the control block with its tick, and the
+    // polled overflow cleared before anything more runs.
     if (seen->overflow) {
       SRD_CHECK(hipMemcpyAsync(pin + ctl_at, ctl, sizeof(DenseCtl), hipMemcpyDeviceToHost, s));
       SRD_CHECK(hipStreamSynchronize(s));
       std::memcpy(&h, pin + ctl_at, sizeof(h));
       const uint64_t need = seen->need;
+      tick = h.tick;
+      seen->overflow = 0;
+      if (!h.overflow) fail("dense iterations: an overflow without its control block");
       if (e.trace) {
         std::fprintf(stderr, "[srd]   dense iterations: overflow %u at iteration %llu, %llu rows\n",
                      h.overflow, (unsigned long long)h.iter, (unsigned long long)need);
@@ -3009,9 +3016,9 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
     if (seen->done || seen->iter >= max_iters) break;
   }
   // state back to the relations: FULL as an index, DELTA, the recorded sizes
-  const uint64_t iters = seen->iter;
+  // (the whole record, as the number of iterations comes with it)
   uint64_t* back = reinterpret_cast<uint64_t*>(pin + back_at);
-  std::vector<std::vector<uint64_t>> rec(nr, std::vector<uint64_t>(iters));
+  std::vector<std::vector<uint64_t>> rec(nr, std::vector<uint64_t>(h.iter_cap));
   for (size_t j = 0; j < nr; ++j) {
     DenseRel f = rels[j].d;
     f.nw = f.fl;
@@ -3019,12 +3026,13 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
     f.fl = nullptr;
     dense_index_count(f, s);
     SRD_CHECK(hipMemcpyAsync(back + j, f.blk + f.nblocks, 8, hipMemcpyDeviceToHost, s));
-    if (iters) SRD_CHECK(hipMemcpyAsync(rec[j].data(), rels[j].d.rec, iters * 8, hipMemcpyDeviceToHost, s));
+    SRD_CHECK(hipMemcpyAsync(rec[j].data(), rels[j].d.rec, h.iter_cap * 8, hipMemcpyDeviceToHost, s));
   }
   SRD_CHECK(hipMemcpyAsync(back + kDevRels, row_ctrs.p, row_ctrs.n * 8, hipMemcpyDeviceToHost, s));
   SRD_CHECK(hipMemcpyAsync(pin + ctl_at, ctl, sizeof(DenseCtl), hipMemcpyDeviceToHost, s));
   SRD_CHECK(hipStreamSynchronize(s));
   std::memcpy(&h, pin + ctl_at, sizeof(h));
+  const uint64_t iters = h.iter;
   const uint32_t bound = value_bound(e);
   for (size_t j = 0; j < nr; ++j) {
     DenseRelState& R = rels[j];

@@ -28,8 +28,17 @@ inline const char* hipGetErrorString(hipError_t) { return "cpu-sim error"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (void*)1; return 0; }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+// A build whose launches run on a thread of their own (dense_cpu.cpp) defines
+// this: op 0 waits until everything enqueued has run, op 1 tells whether it
+// has.  Without it every call has run when it returns.
+extern "C" __attribute__((weak)) int sim_stream_op(int op);
+inline hipError_t hipStreamSynchronize(hipStream_t) {
+  if (sim_stream_op) sim_stream_op(0);
+  return hipSuccess;
+}
+inline hipError_t hipStreamQuery(hipStream_t) {
+  return !sim_stream_op || sim_stream_op(1) ? hipSuccess : hipErrorNotReady;
+}
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 // Everything runs in program order on the host: events and waits do nothing
 // but report to sim_stream_event (op 0: a record on s, 1: s waits), which
@@ -91,6 +100,7 @@ inline hipError_t hipMemGetInfo(size_t* fr, size_t* tot) {
   return hipSuccess;
 }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  if (sim_stream_op) sim_stream_op(0);
   if (n) std::memmove(d, s, n);
   return hipSuccess;
 }

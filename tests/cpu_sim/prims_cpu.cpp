@@ -19,6 +19,7 @@ void check(hipError_t e, const char* what) {
 
 static PoolStats g_stats;
 void pool_init(int) {}
+#ifndef SIM_DENSE  // dense_cpu.cpp has its own: limits, and blocks in use by its device thread
 void* pool_alloc(uint64_t bytes, hipStream_t) {
   g_stats.in_use += bytes;
   g_stats.peak = std::max(g_stats.peak, g_stats.in_use);
@@ -28,15 +29,16 @@ void pool_free(void* p, uint64_t bytes, hipStream_t) {
   g_stats.in_use -= bytes;
   std::free(p);
 }
-void pool_retire_stream(hipStream_t) {}
-PoolStats pool_stats() { return g_stats; }
-hipStream_t stream_acquire() { return (void*)1; }
-void stream_release(hipStream_t) {}
 void* pinned_acquire(uint64_t bytes, uint64_t* got) {
   *got = bytes;
   return std::malloc(bytes ? bytes : 1);
 }
 void pinned_release(void* p, uint64_t) { std::free(p); }
+#endif
+void pool_retire_stream(hipStream_t) {}
+PoolStats pool_stats() { return g_stats; }
+hipStream_t stream_acquire() { return (void*)1; }
+void stream_release(hipStream_t) {}
 std::recursive_mutex& capture_mutex() {
   static std::recursive_mutex m;
   return m;
@@ -172,8 +174,14 @@ uint64_t dense_extract(uint32_t* bits, uint32_t* sum, uint64_t words, uint32_t k
   return n;
 }
 
-void fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t) { std::fill(p, p + n, v); }
-void fill_u64(uint64_t* p, uint64_t v, uint64_t n, hipStream_t) { std::fill(p, p + n, v); }
+void fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t) {
+  if (sim_stream_op) sim_stream_op(0);
+  std::fill(p, p + n, v);
+}
+void fill_u64(uint64_t* p, uint64_t v, uint64_t n, hipStream_t) {
+  if (sim_stream_op) sim_stream_op(0);
+  std::fill(p, p + n, v);
+}
 
 void export_rows(const Index& x, uint32_t* host_out, const uint32_t* bounds, uint32_t n_bounds,
                  Workspace&, hipStream_t) {
@@ -203,7 +211,8 @@ void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>&
 void union_products(const UnionProducts&, hipStream_t) { fail("union_products: not in the host-only build"); }
 
 // Dense iterations need rules with device-sized mark launches, which the
-// host-only pipelines do not have.
+// host-only pipelines do not have (dense_cpu.cpp has both).
+#ifndef SIM_DENSE
 void dense_set_rows(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uint64_t*, uint8_t*,
                     hipStream_t) {
   fail("dense_set_rows: not in the host-only build");
@@ -220,6 +229,7 @@ void dense_inst(const DenseCtl*, uint32_t, const uint32_t*, const uint32_t*, uin
 }
 void dense_index_count(const DenseRel&, hipStream_t) { fail("dense_index_count: not in the host-only build"); }
 void dense_index_emit(const DenseRel&, hipStream_t) { fail("dense_index_emit: not in the host-only build"); }
+#endif
 
 void cost_items(const uint64_t* pref, uint64_t n, uint64_t w, uint64_t S, uint64_t* out,
                 hipStream_t) {

@@ -1,0 +1,124 @@
+"""The host side of the iterations on bitmaps (run_step_dense) against a
+simulated device (tests/cpu_sim/dense_cpu.cpp): relation and deltas against
+the oracle where a DELTA buffer grows while the host is still reading the
+report before it."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import build_cpu_sim
+from srdatalog_hip import codegen, compiler, programs
+from srdatalog_hip import datasets as ds
+
+_u32p = ctypes.POINTER(ctypes.c_uint32)
+
+
+@pytest.fixture(scope="module")
+def lib():
+  lib = ctypes.CDLL(build_cpu_sim("libdense_cpu.so"))
+  lib.cpu_dense_engine.restype = ctypes.c_void_p
+  lib.cpu_dense_engine.argtypes = [ctypes.c_char_p]
+  lib.srd_engine_ok.argtypes = [ctypes.c_void_p]
+  lib.srd_engine_load_rows.argtypes = [ctypes.c_void_p, ctypes.c_char_p, _u32p, ctypes.c_uint64,
+                                       ctypes.c_uint32]
+  lib.srd_engine_run.argtypes = [ctypes.c_void_p, ctypes.c_ulonglong]
+  lib.srd_engine_export.argtypes = [ctypes.c_void_p, ctypes.c_char_p, _u32p, ctypes.c_uint64,
+                                    ctypes.POINTER(ctypes.c_uint64)]
+  lib.srd_engine_delta_sizes.argtypes = [ctypes.c_void_p, ctypes.c_char_p,
+                                         ctypes.POINTER(ctypes.c_ulonglong), ctypes.c_ulonglong]
+  lib.srd_engine_destroy.argtypes = [ctypes.c_void_p]
+  lib.srd_engine_set_quiet.argtypes = [ctypes.c_void_p, ctypes.c_int]
+  for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit"):
+    getattr(lib, f).argtypes = [ctypes.c_uint64]
+  lib.sim_fail_allocs.argtypes = [ctypes.c_int64]
+  for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations"):
+    getattr(lib, f).restype = ctypes.c_uint64
+  return lib
+
+
+@pytest.fixture(autouse=True)
+def plain_settings(monkeypatch, lib):
+  for k in ("DEVLOOP", "DEVLOOP_GRAPH", "DEVLOOP_CAPS", "DEVLOOP_BATCH", "DEVLOOP_MAX_BYTES",
+            "DEVLOOP_MAX_ROWS", "DEVLOOP_DENSE", "DENSE_DELTA_ROWS", "DENSE_MAX_BITS", "JOIN_MODE"):
+    monkeypatch.delenv("SRDATALOG_" + k, raising=False)
+  lib.sim_reset()
+
+
+class Engine:
+  def __init__(self, lib):
+    prog = programs.tc_program()
+    text = codegen.program_text(compiler.relation_decls(prog), compiler.compile_to_mir(prog))
+    self.lib, self.e = lib, ctypes.c_void_p(lib.cpu_dense_engine(text.encode()))
+    assert lib.srd_engine_ok(self.e) == 1
+    lib.srd_engine_set_quiet(self.e, 1)
+
+  def run(self, edges, max_iters=0):
+    edges = np.ascontiguousarray(edges, dtype=np.uint32)
+    self.lib.srd_engine_load_rows(self.e, b"ArcInput", edges.ctypes.data_as(_u32p), edges.shape[0], 2)
+    return self.lib.srd_engine_run(self.e, max_iters)
+
+  def path(self):
+    n = ctypes.c_uint64()
+    self.lib.srd_engine_export(self.e, b"Path", None, 0, ctypes.byref(n))
+    out = np.empty((max(n.value, 1), 2), np.uint32)
+    self.lib.srd_engine_export(self.e, b"Path", out.ctypes.data_as(_u32p), n.value, ctypes.byref(n))
+    cnt = self.lib.srd_engine_delta_sizes(self.e, b"Path", None, 0)
+    buf = (ctypes.c_ulonglong * max(cnt, 1))()
+    self.lib.srd_engine_delta_sizes(self.e, b"Path", buf, cnt)
+    return out[:n.value], [int(buf[i]) for i in range(cnt)]
+
+  def close(self):
+    self.lib.srd_engine_destroy(self.e)
+
+
+@pytest.fixture
+def engine(lib):
+  engines = []
+
+  def make():
+    engines.append(Engine(lib))
+    return engines[-1]
+  yield make
+  for e in engines:
+    e.close()
+
+
+def check(got, edges, max_iters=0):
+  want = oracle.run("tc", {"ArcInput": edges}, **({"max_iters": max_iters} if max_iters else {}))
+  np.testing.assert_array_equal(got[0], want.relations["Path"])
+  assert got[1] == want.deltas["Path"]
+
+
+def fan(width, tail):
+  """`width` sources into a chain of two, out to `width` targets that all
+  enter a chain of `tail`: the first iteration derives few pairs, the second
+  width * width of them."""
+  s, t = np.arange(width), 100 + np.arange(width)
+  chain = [(50, 51)] + [(200 + i, 201 + i) for i in range(tail)]
+  return np.array([(a, 50) for a in s] + [(51, b) for b in t] + [(b, 200) for b in t] + chain, np.uint32)
+
+
+@pytest.mark.parametrize("n,m,seed", [(2, 2, 0), (40, 60, 1), (200, 500, 2), (600, 1500, 3)])
+def test_bitmap_iterations_match_the_oracle(lib, engine, n, m, seed):
+  e = ds.tc_edges(seed, n, m)
+  eng = engine()
+  for _ in range(2):
+    assert eng.run(e) == 0
+    check(eng.path(), e)
+  assert eng.run(e, 2) == 0
+  check(eng.path(), e, 2)
+  assert lib.sim_dense_iterations() > 0 and lib.sim_late_writes() == 0
+
+
+def test_growing_delta_while_the_report_is_half_there(lib, engine, monkeypatch):
+  """The second iteration overflows DELTA; the host takes the first one's
+  report while the second's flag is already stored and its count is not."""
+  monkeypatch.setenv("SRDATALOG_DENSE_DELTA_ROWS", "128")
+  e = fan(30, 20)
+  lib.sim_split_report(2)
+  eng = engine()
+  assert eng.run(e) == 0
+  check(eng.path(), e)
