@@ -101,11 +101,14 @@ struct DevBuf {
   void alloc(uint64_t count, hipStream_t st) {
     release();
     s = st;
-    n = count;
     if (count) {
-      p = static_cast<T*>(pool_alloc(count * sizeof(T), st));
+      // (empty if this throws: a size without memory would pass for a buffer
+      // of that size the next time it is reserved)
+      T* q = static_cast<T*>(pool_alloc(count * sizeof(T), st));
       const uint64_t bytes = count * sizeof(T);
-      owner = std::shared_ptr<void>(p, [bytes, st](void* q) { pool_free(q, bytes, st); });
+      owner = std::shared_ptr<void>(q, [bytes, st](void* b) { pool_free(b, bytes, st); });
+      p = q;
+      n = count;
     }
   }
   // Grow to at least `count` elements (contents not preserved).

@@ -118,6 +118,17 @@ extern "C" void sim_fail_allocs(int64_t bytes) { g_fail_above = bytes; }
 extern "C" void sim_pool_limit(uint64_t bytes) { g_limit = bytes; }
 extern "C" uint64_t sim_pool_used() { return g_used; }
 extern "C" uint64_t sim_late_writes() { return g_late_writes; }
+// Size of a buffer whose growth failed.
+extern "C" uint64_t sim_size_after_failure() {
+  srd::DevBuf<uint32_t> b(64, nullptr);
+  g_limit = g_used + 1024;
+  try {
+    b.reserve(1 << 20, nullptr);
+  } catch (const std::exception&) {
+  }
+  g_limit = 0;
+  return b.p ? ~uint64_t(0) : b.n;
+}
 extern "C" uint64_t sim_dense_iterations() { return g_plans; }
 
 namespace srd {

@@ -34,7 +34,7 @@ def lib():
   for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit"):
     getattr(lib, f).argtypes = [ctypes.c_uint64]
   lib.sim_fail_allocs.argtypes = [ctypes.c_int64]
-  for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations"):
+  for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations", "sim_size_after_failure"):
     getattr(lib, f).restype = ctypes.c_uint64
   return lib
 
@@ -122,3 +122,9 @@ def test_growing_delta_while_the_report_is_half_there(lib, engine, monkeypatch):
   eng = engine()
   assert eng.run(e) == 0
   check(eng.path(), e)
+
+
+def test_a_buffer_that_could_not_grow_is_empty(lib):
+  """Not a size without memory, which the next reserve would take for a
+  buffer of that size."""
+  assert lib.sim_size_after_failure() == 0
