@@ -1320,6 +1320,21 @@ static uint32_t value_bound(const srd_engine& e) {
   return b;
 }
 
+// A clear bitmap of `words` words and its block bytes in place of the buffers'
+// earlier one, charged to the engine; both empty if there is no memory.
+static void new_bitmap(srd_engine& e, DevBuf<uint32_t>& bits, DevBuf<uint32_t>& sum, uint64_t words,
+                       hipStream_t s) {
+  e.dense_bytes -= bits.n * 4;
+  bits.release();
+  sum.release();
+  DevBuf<uint32_t> b(words, s), m(dense_sum_words(words), s);
+  fill_u32(b.p, 0, words, s);
+  fill_u32(m.p, 0, m.n, s);
+  bits = std::move(b);
+  sum = std::move(m);
+  e.dense_bytes += words * 4;
+}
+
 // After the runs' views are prepared and before any of them launches: the
 // destinations whose key space fits dense_max_bits take their NEW as a
 // bitmap that the runs writing them mark (mode 6).  A destination some run
@@ -1372,11 +1387,7 @@ static void pr_dense(srd_engine& e, std::vector<PipeRun*>& runs) {
                              1) * kDenseBlockWords;
       if (r.dense_bits.n < words) {
         if (e.dense_bytes - r.dense_bits.n * 4 + words * 4 > e.device_bytes / 8) continue;
-        e.dense_bytes = e.dense_bytes - r.dense_bits.n * 4 + words * 4;
-        r.dense_bits.alloc(words, e.s);
-        fill_u32(r.dense_bits.p, 0, words, e.s);
-        r.dense_sum.alloc(dense_sum_words(words), e.s);
-        fill_u32(r.dense_sum.p, 0, dense_sum_words(words), e.s);
+        new_bitmap(e, r.dense_bits, r.dense_sum, words, e.s);
       }
       r.dense_words = words;
       r.dense_shift = sh;
@@ -1423,13 +1434,8 @@ static void pr_union(srd_engine& e, PipeRun& R, uint64_t iteration) {
   if (2 * sh > kUnionBits) return;
   const uint64_t words = std::max<uint64_t>((uint64_t(1) << (2 * sh)) / 32, kDenseBlockWords);
   if (sc.uni_bits.n < words) {
-    const uint64_t bytes = e.dense_bytes - sc.uni_bits.n * 4 + words * 4;
-    if (bytes > e.device_bytes / 8) return;
-    e.dense_bytes = bytes;
-    sc.uni_bits.alloc(words, R.s);
-    fill_u32(sc.uni_bits.p, 0, words, R.s);
-    sc.uni_sum.alloc(dense_sum_words(words), R.s);
-    fill_u32(sc.uni_sum.p, 0, dense_sum_words(words), R.s);
+    if (e.dense_bytes - sc.uni_bits.n * 4 + words * 4 > e.device_bytes / 8) return;
+    new_bitmap(e, sc.uni_bits, sc.uni_sum, words, R.s);
   }
   const uint32_t k = R.d->dest[0].arity;
   UnionProducts& u = R.uni;
@@ -2806,13 +2812,7 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
     R.d.k = r.arity;
     R.d.shift = plan.shift[j];
     R.d.nblocks = uint32_t(words / kDenseBlockWords);
-    if (r.dense_bits.n < words || r.dense_sum.n < sum_words) {
-      e.dense_bytes = e.dense_bytes - r.dense_bits.n * 4 + words * 4;
-      r.dense_bits.alloc(words, s);
-      fill_u32(r.dense_bits.p, 0, words, s);
-      r.dense_sum.alloc(sum_words, s);
-      fill_u32(r.dense_sum.p, 0, sum_words, s);
-    }
+    if (r.dense_bits.n < words) new_bitmap(e, r.dense_bits, r.dense_sum, words, s);
     R.fl.alloc(words, s);
     fill_u32(R.fl.p, 0, words, s);
     R.fsum.alloc(sum_words, s);
@@ -3120,6 +3120,34 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
 }  // namespace srd
 
 namespace srd {
+
+// A run that ends in an error may leave marks in its bitmaps (NEW of the
+// relations, unions of the rules), and launches that still set them: they
+// are given back once those have run, and the next run allocates clear ones.
+static void drop_marks(srd_engine& e) {
+  (void)hipStreamSynchronize(e.s);
+  for (hipStream_t g : e.group_s) (void)hipStreamSynchronize(g);
+  auto drop = [&](DevBuf<uint32_t>& bits, DevBuf<uint32_t>& sum) {
+    e.dense_bytes -= bits.n * 4;
+    bits.release();
+    sum.release();
+  };
+  for (auto& r : e.rels) {
+    drop(r.dense_bits, r.dense_sum);
+    r.dense_on = false;
+  }
+  for (auto& x : e.scratch) drop(x->uni_bits, x->uni_sum);
+}
+
+template <class F>
+static void run_or_drop(srd_engine& e, F&& f) {
+  try {
+    f();
+  } catch (...) {
+    drop_marks(e);
+    throw;
+  }
+}
 
 static void run_program(srd_engine& e, uint64_t max_iters) {
   reset_state(e);
@@ -3725,7 +3753,9 @@ int srd_engine_run(srd_engine* e, unsigned long long max_iters) {
   bool any_decl = false;
   for (auto& r : e->rels) any_decl |= !r.input_file.empty();
   if (any_decl && !any_input) return 1;
-  return eguard(e, 2, [&] { run_program(*e, max_iters ? max_iters : uint64_t(2147483647)); });
+  return eguard(e, 2, [&] {
+    run_or_drop(*e, [&] { run_program(*e, max_iters ? max_iters : uint64_t(2147483647)); });
+  });
 }
 
 unsigned long long srd_engine_size(srd_engine* e, const char* rel) {
@@ -3846,7 +3876,7 @@ int srd_engine_shutdown(srd_engine* e) {
 
 int srd_engine_run_begin(srd_engine* e) {
   if (!e) return 1;
-  return eguard(e, 2, [&] { run_begin(*e); });
+  return eguard(e, 2, [&] { run_or_drop(*e, [&] { run_begin(*e); }); });
 }
 
 int srd_engine_run_iterations(srd_engine* e, unsigned long long k, unsigned long long* done,
@@ -3854,7 +3884,8 @@ int srd_engine_run_iterations(srd_engine* e, unsigned long long k, unsigned long
   if (!e) return 1;
   return eguard(e, 2, [&] {
     bool c = false;
-    const uint64_t d = run_iters(*e, k, &c);
+    uint64_t d = 0;
+    run_or_drop(*e, [&] { d = run_iters(*e, k, &c); });
     if (done) *done = d;
     if (converged) *converged = c ? 1 : 0;
   });

@@ -9,8 +9,8 @@
 #include <condition_variable>
 #include <deque>
 #include <functional>
+#include <map>
 #include <mutex>
-#include <set>
 #include <thread>
 
 #include "tc_pipes_cpu.cpp"
@@ -70,7 +70,7 @@ std::atomic<uint64_t> g_limit{0}, g_used{0}, g_late_writes{0};
 std::atomic<int64_t> g_fail_above{-1};   // allocations of at least this many bytes fail once iterations run
 std::atomic<bool> g_running{false};      // a run has enqueued its first iteration
 std::mutex g_pin_mu;
-std::set<const void*> g_pins;            // pinned blocks handed out
+std::map<const char*, uint64_t> g_pins;   // pinned blocks handed out
 
 void wait_for(const std::function<bool()>& f) {
   for (int i = 0; i < 4000 && !f(); ++i) std::this_thread::sleep_for(std::chrono::milliseconds(1));
@@ -78,8 +78,8 @@ void wait_for(const std::function<bool()>& f) {
 
 bool pinned_alive(const void* p) {
   std::lock_guard<std::mutex> g(g_pin_mu);
-  auto it = g_pins.upper_bound(p);
-  return it != g_pins.begin();  // blocks are page-sized and larger than what is written
+  auto it = g_pins.upper_bound(static_cast<const char*>(p));
+  return it != g_pins.begin() && std::prev(it)->first + std::prev(it)->second > p;
 }
 
 void enqueue(std::function<void()> f) { g_dev->put(std::move(f)); }
@@ -147,14 +147,14 @@ void pool_free(void* p, uint64_t bytes, hipStream_t) {
 }
 void* pinned_acquire(uint64_t bytes, uint64_t* got) {
   *got = bytes;
-  void* p = std::calloc(1, bytes ? bytes : 1);
+  char* p = static_cast<char*>(std::calloc(1, bytes ? bytes : 1));
   std::lock_guard<std::mutex> g(g_pin_mu);
-  g_pins.insert(p);
+  g_pins[p] = bytes;
   return p;
 }
 void pinned_release(void* p, uint64_t) {
   std::lock_guard<std::mutex> g(g_pin_mu);
-  g_pins.erase(p);  // kept allocated: a late write is counted, not a crash
+  g_pins.erase(static_cast<char*>(p));  // kept allocated: a late write is counted, not a crash
 }
 
 static uint64_t words_of(const DenseRel& r) { return uint64_t(r.nblocks) * (kDenseBlockWords / 2); }

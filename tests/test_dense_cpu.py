@@ -128,3 +128,16 @@ def test_a_buffer_that_could_not_grow_is_empty(lib):
   """Not a size without memory, which the next reserve would take for a
   buffer of that size."""
   assert lib.sim_size_after_failure() == 0
+
+
+@pytest.mark.parametrize("nth", [1, 2, 4])
+def test_a_run_after_a_failed_one_starts_clear(lib, engine, nth):
+  """A launch fails in the middle of the iterations: the marks that the failed
+  run left in NEW are no part of the next one."""
+  eng = engine()
+  lib.sim_fail_book(nth)
+  assert eng.run(ds.tc_edges(4, 50, 200)) != 0
+  lib.sim_fail_book(0)
+  e = ds.tc_edges(5, 40, 60)
+  assert eng.run(e) == 0
+  check(eng.path(), e)
