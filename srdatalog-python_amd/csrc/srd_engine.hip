@@ -2849,8 +2849,13 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
   const uint64_t back_at = pin_at + 256, back_bytes = row_ctrs.n * 8 + 8 * kDevRels;
   uint64_t pin_bytes = 0;
   uint8_t* pin = static_cast<uint8_t*>(pinned_acquire(back_at + back_bytes, &pin_bytes));
-  std::unique_ptr<uint8_t, std::function<void(uint8_t*)>> pin_guard(
-      pin, [pin_bytes](uint8_t* q) { pinned_release(q, pin_bytes); });
+  // The launches sent write their reports into the block: if this throws, they
+  // run before another user gets it.
+  bool reports = true;
+  std::unique_ptr<uint8_t, std::function<void(uint8_t*)>> pin_guard(pin, [&reports, pin_bytes, s](uint8_t* q) {
+    if (reports) (void)hipStreamSynchronize(s);
+    pinned_release(q, pin_bytes);
+  });
   DenseCtl* ctl = reinterpret_cast<DenseCtl*>(dev.p + ctl_at);
   volatile DenseSeen* seen = reinterpret_cast<DenseSeen*>(pin + pin_at);
   std::memset(pin + pin_at, 0, sizeof(DenseSeen));
@@ -3031,6 +3036,7 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
   SRD_CHECK(hipMemcpyAsync(back + kDevRels, row_ctrs.p, row_ctrs.n * 8, hipMemcpyDeviceToHost, s));
   SRD_CHECK(hipMemcpyAsync(pin + ctl_at, ctl, sizeof(DenseCtl), hipMemcpyDeviceToHost, s));
   SRD_CHECK(hipStreamSynchronize(s));
+  reports = false;
   std::memcpy(&h, pin + ctl_at, sizeof(h));
   const uint64_t iters = h.iter;
   const uint32_t bound = value_bound(e);

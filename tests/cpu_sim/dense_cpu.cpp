@@ -64,6 +64,7 @@ Device* g_dev = nullptr;  // one per test run (sim_reset), so that a run's rest 
 std::atomic<uint64_t> g_split_tick{0};   // book that is half published when the host looks (0: none)
 std::atomic<bool> g_half{false};         // it stored its overflow flag, its tick not yet
 std::atomic<bool> g_drained{false};      // the host has waited for the stream since
+std::atomic<bool> g_hold{false};         // iterations wait for the host to wait for them
 std::atomic<bool> g_tail{false};         // and has enqueued launches since
 std::atomic<uint64_t> g_plans{0}, g_books{0}, g_fail_book{0}, g_queries{0};
 std::atomic<uint64_t> g_limit{0}, g_used{0}, g_late_writes{0};
@@ -109,10 +110,16 @@ extern "C" void sim_reset() {
   delete g_dev;
   g_dev = new Device();
   g_split_tick = g_plans = g_books = g_fail_book = g_queries = g_limit = g_late_writes = 0;
-  g_half = g_drained = g_tail = g_running = false;
+  g_half = g_drained = g_tail = g_running = g_hold = false;
   g_fail_above = -1;
 }
 extern "C" void sim_split_report(uint64_t tick) { g_split_tick = tick; }
+// The device starts on what is enqueued only when the host waits for it (or
+// asks three times).
+extern "C" void sim_hold() {
+  std::lock_guard<std::mutex> g(g_dev->mu);
+  g_hold = true;
+}
 extern "C" void sim_fail_book(uint64_t nth) { g_books = 0, g_fail_book = nth; }
 extern "C" void sim_fail_allocs(int64_t bytes) { g_fail_above = bytes; }
 extern "C" void sim_pool_limit(uint64_t bytes) { g_limit = bytes; }
@@ -207,6 +214,11 @@ void dense_plan(DenseCtl*, SrdDyn* d, uint32_t, const uint64_t* key_work, uint64
                 uint64_t*, uint32_t*, uint32_t grain, uint32_t least, hipStream_t) {
   ++g_plans;
   g_running = true;
+  if (g_hold.exchange(false)) {
+    std::lock_guard<std::mutex> g(g_dev->mu);
+    g_dev->paused = true;
+    g_queries = 0;
+  }
   // the third iteration is enqueued late: the device is already in the second
   if (g_split_tick && g_plans == g_split_tick + 1) wait_for([] { return g_half.load(); });
   enqueue([=] {

@@ -141,3 +141,17 @@ def test_a_run_after_a_failed_one_starts_clear(lib, engine, nth):
   e = ds.tc_edges(5, 40, 60)
   assert eng.run(e) == 0
   check(eng.path(), e)
+
+
+def test_a_failed_run_keeps_its_pinned_block_until_the_launches_ran(lib, engine):
+  """The third iteration cannot be launched; the first two are still to run
+  and report into the block."""
+  eng = engine()
+  lib.sim_hold()
+  lib.sim_fail_book(3)
+  assert eng.run(ds.tc_edges(4, 50, 200)) != 0
+  lib.sim_fail_book(0)
+  e = ds.tc_edges(5, 40, 60)
+  assert eng.run(e) == 0
+  check(eng.path(), e)
+  assert lib.sim_late_writes() == 0
