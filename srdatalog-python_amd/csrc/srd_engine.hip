@@ -2723,18 +2723,35 @@ struct DensePipeState {
   SrdDyn dyn_host;
   DlBind bind;
   uint64_t cap_keys = 0;
-  uint32_t grain = 0;
-  DevBuf<uint8_t> dyn;
+  uint32_t grain = 0, slots = 1;
   DevBuf<uint32_t> key_rng, key_aux, work_ctr;
   DevBuf<uint64_t> key_work, work_start, scan;
 };
 
-// Run the step's iterations on bitmaps; returns the iterations run (the host
-// loop continues from there unless *converged).
-static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint64_t max_iters,
-                               const DensePlan& plan, bool* converged) {
+// Memory of a loop on bitmaps beside its DELTA buffers, and of DELTA buffers
+// of `rows` rows: columns, and root arrays of as many entries as the rows
+// have column-0 values.
+static uint64_t dense_loop_bytes(const srd_engine& e, const DenseRelState& R, uint64_t words, uint64_t iters) {
+  return 2 * words * 4 + 3 * dense_sum_words(words) * 4 + R.d.nblocks * (8 + 64 * 8) +
+         iters * 8 * (1 + uint64_t(e.n_inst));
+}
+static uint64_t dense_roots(const DenseRelState& R, uint64_t rows) {
+  return R.d.k > 1 ? std::min(rows, uint64_t(1) << R.d.shift) : rows;
+}
+static uint64_t dense_delta_bytes(const DenseRelState& R, uint64_t rows) {
+  return (round_stride(rows) * R.d.k + 2 * dense_roots(R, round_stride(rows))) * 4;
+}
+
+// Run the step's iterations on bitmaps: *iters of them (the host loop
+// continues from there unless *converged).  False, with nothing run: there is
+// no room for the bitmaps and buffers within SRDATALOG_DEVLOOP_MAX_BYTES or
+// the device's memory.  Buffers that cannot grow within these end the loop
+// early and the host loop goes on.
+static bool run_step_dense(srd_engine& e, const Step& st, int step_no, uint64_t max_iters,
+                           const DensePlan& plan, uint64_t* iters_out, bool* converged) {
   hipStream_t s = e.s;
   *converged = false;
+  *iters_out = 0;
   const size_t nr = st.canonical_rels.size();
   std::vector<DenseRelState> rels(nr);
   bool weighs = false;
@@ -2785,7 +2802,7 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
   }
   // beyond devloop_max_rows a rule with nested levels is better off with the
   // host loop's cost-balanced slices
-  if (weighs && full_max > e.devloop_max_rows) return 0;
+  if (weighs && full_max > e.devloop_max_rows) return false;
 
   DenseBook book;
   std::memset(&book, 0, sizeof(book));
@@ -2795,43 +2812,116 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
   std::memset(&h, 0, sizeof(h));
   h.max_iter = max_iters;
   h.iter_cap = 1024;
-  auto alloc_delta = [&](DenseRelState& R, uint64_t rows) {
-    R.d.stride = round_stride(rows);
-    R.delta.alloc(R.d.k * R.d.stride, s);
-    R.root_v.alloc(R.d.stride, s);
-    R.root_o.alloc(R.d.stride + 1, s);
+  struct DeltaBufs {
+    DevBuf<uint32_t> cols, root_v, root_o;
+    uint64_t stride = 0;
+  };
+  auto new_delta = [&](const DenseRelState& R, uint64_t rows) {
+    DeltaBufs b;
+    b.stride = round_stride(rows);
+    b.cols.alloc(R.d.k * b.stride, s);
+    b.root_v.alloc(dense_roots(R, b.stride), s);
+    b.root_o.alloc(dense_roots(R, b.stride) + 1, s);
+    return b;
+  };
+  auto take_delta = [&](DenseRelState& R, DeltaBufs&& b) {
+    R.delta = std::move(b.cols);
+    R.root_v = std::move(b.root_v);
+    R.root_o = std::move(b.root_o);
+    R.d.stride = b.stride;
     R.d.delta = R.delta.p;
     R.d.root_v = R.root_v.p;
     R.d.root_o = R.root_o.p;
   };
+  // DELTA rows: 2^24, or the whole key space when that is smaller
+  auto first_rows = [&](size_t j) { return std::min<uint64_t>(e.dense_delta_rows, plan.words[j] * 32); };
+  uint64_t total = 0;
+  for (size_t j = 0; j < nr; ++j) {
+    DenseRelState& R = rels[j];
+    std::memset(&R.d, 0, sizeof(R.d));
+    R.d.k = e.rels[R.rel].arity;
+    R.d.shift = plan.shift[j];
+    R.d.nblocks = uint32_t(plan.words[j] / kDenseBlockWords);
+    total += dense_loop_bytes(e, R, plan.words[j], h.iter_cap) + dense_delta_bytes(R, first_rows(j));
+  }
+  for (auto& P : pipes) {
+    const SrdPipelineDesc* d = P.d;
+    SrdDyn& dh = P.dyn_host;
+    uint32_t drv = d->root_view[0];
+    P.cap_keys = ~uint64_t(0);
+    if (d->root_kind == SRD_ROOT_JOIN) {
+      for (uint32_t i = 0; i < d->n_root_src; ++i) {
+        const uint32_t v = d->root_view[i];
+        if (dh.views.v[v].r < dh.views.v[drv].r) drv = v;
+        // the driver has no more keys than any root source can have
+        const int j = P.bind.vrel[v];
+        P.cap_keys = std::min<uint64_t>(P.cap_keys, j < 0 ? dh.views.v[v].r : uint64_t(1) << rels[j].d.shift);
+      }
+      dh.n_root = dh.views.v[drv].r;
+    } else {
+      P.cap_keys = 1;
+      dh.n_root = dh.views.v[drv].n ? 1u : 0u;
+    }
+    P.cap_keys = std::max<uint64_t>(P.cap_keys, 1);
+    dh.drv_view = drv;
+    P.slots = std::max<uint32_t>(P.bind.n_root_src, 1);
+    total += P.cap_keys * (8 * P.slots + 4 + 8 + 8) +
+             (P.cap_keys > kDensePlanKeys ? scan_dev_words(P.cap_keys) * 8 : 0);
+  }
+  auto no_room = [&](const char* why) {
+    if (e.trace) {
+      std::fprintf(stderr, "[srd]   dense iterations: %llu bytes: %s\n", (unsigned long long)total, why);
+      std::fflush(stderr);
+    }
+    return false;
+  };
+  if (total > e.devloop_max_bytes) return no_room("above the memory budget");
+  try {
+    for (size_t j = 0; j < nr; ++j) {
+      DenseRelState& R = rels[j];
+      Relation& r = e.rels[R.rel];
+      const uint64_t words = plan.words[j], sum_words = dense_sum_words(words);
+      if (r.dense_bits.n < words) new_bitmap(e, r.dense_bits, r.dense_sum, words, s);
+      R.fl.alloc(words, s);
+      R.fsum.alloc(sum_words, s);
+      R.live.alloc(sum_words, s);
+      R.blk.alloc(uint64_t(R.d.nblocks) + 1, s);
+      R.chunk.alloc(uint64_t(R.d.nblocks) * 64, s);
+      R.rec.alloc(h.iter_cap, s);
+      if (e.n_inst) R.inst.alloc(h.iter_cap * e.n_inst, s);
+      take_delta(R, new_delta(R, first_rows(j)));
+    }
+    for (auto& P : pipes) {
+      P.key_rng.alloc(P.cap_keys * 2 * P.slots, s);
+      P.key_aux.alloc(P.cap_keys, s);
+      P.key_work.alloc(P.cap_keys, s);
+      P.work_start.alloc(P.cap_keys + 1, s);
+      if (P.cap_keys > kDensePlanKeys) P.scan.alloc(scan_dev_words(P.cap_keys), s);
+      P.work_ctr.alloc(SRD_XCDS * SRD_CTR_STRIDE, s);
+    }
+  } catch (const std::exception& ex) {
+    // the loop that runs instead gets the room of the clear bitmaps too
+    for (int ri : st.canonical_rels) {
+      Relation& r = e.rels[ri];
+      e.dense_bytes -= r.dense_bits.n * 4;
+      r.dense_bits.release();
+      r.dense_sum.release();
+    }
+    return no_room(ex.what());
+  }
   for (size_t j = 0; j < nr; ++j) {
     DenseRelState& R = rels[j];
     Relation& r = e.rels[R.rel];
-    const uint64_t words = plan.words[j], sum_words = dense_sum_words(words);
-    std::memset(&R.d, 0, sizeof(R.d));
-    R.d.k = r.arity;
-    R.d.shift = plan.shift[j];
-    R.d.nblocks = uint32_t(words / kDenseBlockWords);
-    if (r.dense_bits.n < words) new_bitmap(e, r.dense_bits, r.dense_sum, words, s);
-    R.fl.alloc(words, s);
-    fill_u32(R.fl.p, 0, words, s);
-    R.fsum.alloc(sum_words, s);
-    fill_u32(R.fsum.p, 0, sum_words, s);
-    R.live.alloc(sum_words, s);
-    R.blk.alloc(uint64_t(R.d.nblocks) + 1, s);
-    R.chunk.alloc(uint64_t(R.d.nblocks) * 64, s);
+    fill_u32(R.fl.p, 0, R.fl.n, s);
+    fill_u32(R.fsum.p, 0, R.fsum.n, s);
     R.d.live = reinterpret_cast<uint8_t*>(R.live.p);
     R.d.chunk = R.chunk.p;
-    R.rec.alloc(h.iter_cap, s);
-    if (e.n_inst) R.inst.alloc(h.iter_cap * e.n_inst, s);
     R.d.nw = reinterpret_cast<uint64_t*>(r.dense_bits.p);
     R.d.fl = reinterpret_cast<uint64_t*>(R.fl.p);
     R.d.nsum = reinterpret_cast<uint8_t*>(r.dense_sum.p);
     R.d.fsum = reinterpret_cast<uint8_t*>(R.fsum.p);
     R.d.blk = R.blk.p;
     R.d.rec = R.rec.p;
-    // DELTA rows: 2^24, or the whole key space when that is smaller
-    alloc_delta(R, std::min<uint64_t>(e.dense_delta_rows, words * 32));
     const Index& f = *R.full0;
     dense_set_rows(f.cols.p, f.stride, f.n, R.d.k, R.d.shift, R.d.fl, R.d.fsum, s);
     h.full_n[j] = h.delta_n[j] = f.n;
@@ -2865,31 +2955,7 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
     DensePipeState& P = pipes[p];
     const SrdPipelineDesc* d = P.d;
     SrdDyn& dh = P.dyn_host;
-    uint32_t drv = d->root_view[0];
-    P.cap_keys = ~uint64_t(0);
-    if (d->root_kind == SRD_ROOT_JOIN) {
-      for (uint32_t i = 0; i < d->n_root_src; ++i) {
-        const uint32_t v = d->root_view[i];
-        if (dh.views.v[v].r < dh.views.v[drv].r) drv = v;
-        // the driver has no more keys than any root source can have
-        const int j = P.bind.vrel[v];
-        P.cap_keys = std::min<uint64_t>(P.cap_keys, j < 0 ? dh.views.v[v].r : uint64_t(1) << rels[j].d.shift);
-      }
-      dh.n_root = dh.views.v[drv].r;
-    } else {
-      P.cap_keys = 1;
-      dh.n_root = dh.views.v[drv].n ? 1u : 0u;
-    }
-    P.cap_keys = std::max<uint64_t>(P.cap_keys, 1);
-    dh.drv_view = drv;
     h.keys[p] = dh.n_root;
-    const uint32_t slots = std::max<uint32_t>(P.bind.n_root_src, 1);
-    P.key_rng.alloc(P.cap_keys * 2 * slots, s);
-    P.key_aux.alloc(P.cap_keys, s);
-    P.key_work.alloc(P.cap_keys, s);
-    P.work_start.alloc(P.cap_keys + 1, s);
-    if (P.cap_keys > kDensePlanKeys) P.scan.alloc(scan_dev_words(P.cap_keys), s);
-    P.work_ctr.alloc(SRD_XCDS * SRD_CTR_STRIDE, s);
     P.grain = e.grain_override ? e.grain_override : d->default_grain;
     std::memset(&P.a, 0, sizeof(P.a));
     P.a.grid_blocks = SRD_GRID_WAVES / 4;
@@ -2989,27 +3055,55 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
         break;
       }
       // NEW holds the abandoned iteration's marks: only its emission runs
-      // again, with room for it
-      if (h.overflow & kOvfIters) {
-        const uint64_t cap = 2 * h.iter_cap;
-        for (auto& R : rels) {
-          DevBuf<uint64_t> nrec(cap, s);
-          SRD_CHECK(hipMemcpyAsync(nrec.p, R.rec.p, h.iter * 8, hipMemcpyDeviceToDevice, s));
-          R.rec = std::move(nrec);
-          R.d.rec = R.rec.p;
-          if (e.n_inst) {
-            DevBuf<uint64_t> ninst(cap * e.n_inst, s);
-            SRD_CHECK(hipMemcpyAsync(ninst.p, R.inst.p, h.iter * e.n_inst * 8, hipMemcpyDeviceToDevice, s));
-            R.inst = std::move(ninst);
+      // again, with room for it.  Every buffer is there before the first is
+      // exchanged: without room the state stays as the last iteration left it.
+      const uint64_t iter_cap = h.overflow & kOvfIters ? 2 * h.iter_cap : h.iter_cap;
+      std::vector<uint64_t> rows(nr);
+      uint64_t grown = 0;  // with the FULL index that the loop ends with
+      for (size_t j = 0; j < nr; ++j) {
+        const DenseRelState& R = rels[j];
+        rows[j] = R.d.stride;
+        if ((h.overflow & kOvfNew) && need > R.d.stride)
+          rows[j] = std::min<uint64_t>(std::max(2 * R.d.stride, need + need / 4), plan.words[j] * 32);
+        grown += dense_loop_bytes(e, R, plan.words[j], iter_cap) + dense_delta_bytes(R, rows[j]) +
+                 dense_delta_bytes(R, h.full_n[j] + std::min(need, rows[j]));
+      }
+      for (const auto& P : pipes) grown += P.cap_keys * (8 * P.slots + 4 + 8 + 8);
+      total = grown;
+      if (grown > e.devloop_max_bytes) {
+        no_room("above the memory budget");
+        handed = true;
+        break;
+      }
+      std::vector<DeltaBufs> nd(nr);
+      std::vector<DevBuf<uint64_t>> nrec(nr), ninst(nr);
+      try {
+        for (size_t j = 0; j < nr; ++j) {
+          if (rows[j] > rels[j].d.stride) nd[j] = new_delta(rels[j], rows[j]);
+          if (iter_cap > h.iter_cap) {
+            nrec[j].alloc(iter_cap, s);
+            if (e.n_inst) ninst[j].alloc(iter_cap * e.n_inst, s);
           }
         }
-        h.iter_cap = cap;
+      } catch (const std::exception& ex) {
+        no_room(ex.what());
+        handed = true;
+        break;
       }
-      if (h.overflow & kOvfNew)
-        for (size_t j = 0; j < nr; ++j)
-          if (need > rels[j].d.stride)
-            alloc_delta(rels[j], std::min<uint64_t>(std::max(2 * rels[j].d.stride, need + need / 4),
-                                                    plan.words[j] * 32));
+      for (size_t j = 0; j < nr; ++j) {
+        DenseRelState& R = rels[j];
+        if (rows[j] > R.d.stride) take_delta(R, std::move(nd[j]));
+        if (iter_cap > h.iter_cap) {
+          SRD_CHECK(hipMemcpyAsync(nrec[j].p, R.rec.p, h.iter * 8, hipMemcpyDeviceToDevice, s));
+          R.rec = std::move(nrec[j]);
+          R.d.rec = R.rec.p;
+          if (e.n_inst) {
+            SRD_CHECK(hipMemcpyAsync(ninst[j].p, R.inst.p, h.iter * e.n_inst * 8, hipMemcpyDeviceToDevice, s));
+            R.inst = std::move(ninst[j]);
+          }
+        }
+      }
+      h.iter_cap = iter_cap;
       for (size_t j = 0; j < nr; ++j) book.rel[j] = rels[j].d;
       h.overflow = h.skip = h.emit = 0;
       std::memcpy(pin + ctl_at, &h, sizeof(h));
@@ -3040,6 +3134,12 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
   std::memcpy(&h, pin + ctl_at, sizeof(h));
   const uint64_t iters = h.iter;
   const uint32_t bound = value_bound(e);
+  for (size_t j = 0; j < nr; ++j)
+    if (h.delta_n[j] == 0) {  // no rows to keep: room for the FULL indexes
+      rels[j].delta.release();
+      rels[j].root_v.release();
+      rels[j].root_o.release();
+    }
   for (size_t j = 0; j < nr; ++j) {
     DenseRelState& R = rels[j];
     Relation& r = e.rels[R.rel];
@@ -3120,7 +3220,8 @@ static uint64_t run_step_dense(srd_engine& e, const Step& st, int step_no, uint6
                  handed ? "host loop from here" : "done");
     std::fflush(stderr);
   }
-  return iters;
+  *iters_out = iters;
+  return true;
 }
 
 }  // namespace srd
@@ -3171,9 +3272,8 @@ static void run_program(srd_engine& e, uint64_t max_iters) {
       std::string why;
       if (e.devloop && !e.count_probes && devloop_eligible(e, st, why)) {
         DensePlan dense;
-        if (dense_eligible(e, st, dense))
-          it = run_step_dense(e, st, int(si), max_iters, dense, &converged);
-        else
+        if (!dense_eligible(e, st, dense) ||
+            !run_step_dense(e, st, int(si), max_iters, dense, &it, &converged))
           it = run_step_device(e, st, int(si), max_iters, &converged);
         converged = converged || it >= max_iters;
       } else if (e.trace && e.devloop) {

@@ -68,7 +68,7 @@ std::atomic<bool> g_hold{false};         // iterations wait for the host to wait
 std::atomic<bool> g_tail{false};         // and has enqueued launches since
 std::atomic<uint64_t> g_plans{0}, g_books{0}, g_fail_book{0}, g_queries{0};
 std::atomic<uint64_t> g_limit{0}, g_used{0}, g_late_writes{0};
-std::atomic<int64_t> g_fail_above{-1};   // allocations of at least this many bytes fail once iterations run
+std::atomic<uint64_t> g_fail_alloc{0};   // the nth allocation once iterations run fails (0: none)
 std::atomic<bool> g_running{false};      // a run has enqueued its first iteration
 std::mutex g_pin_mu;
 std::map<const char*, uint64_t> g_pins;   // pinned blocks handed out
@@ -111,7 +111,7 @@ extern "C" void sim_reset() {
   g_dev = new Device();
   g_split_tick = g_plans = g_books = g_fail_book = g_queries = g_limit = g_late_writes = 0;
   g_half = g_drained = g_tail = g_running = g_hold = false;
-  g_fail_above = -1;
+  g_fail_alloc = 0;
 }
 extern "C" void sim_split_report(uint64_t tick) { g_split_tick = tick; }
 // The device starts on what is enqueued only when the host waits for it (or
@@ -121,7 +121,8 @@ extern "C" void sim_hold() {
   g_hold = true;
 }
 extern "C" void sim_fail_book(uint64_t nth) { g_books = 0, g_fail_book = nth; }
-extern "C" void sim_fail_allocs(int64_t bytes) { g_fail_above = bytes; }
+extern "C" void sim_fail_alloc(uint64_t nth) { g_fail_alloc = nth; }
+extern "C" uint64_t sim_allocs_to_failure() { return g_fail_alloc; }
 extern "C" void sim_pool_limit(uint64_t bytes) { g_limit = bytes; }
 extern "C" uint64_t sim_pool_used() { return g_used; }
 extern "C" uint64_t sim_late_writes() { return g_late_writes; }
@@ -141,7 +142,8 @@ extern "C" uint64_t sim_dense_iterations() { return g_plans; }
 namespace srd {
 
 void* pool_alloc(uint64_t bytes, hipStream_t) {
-  if ((g_limit && g_used + bytes > g_limit) || (g_running && g_fail_above >= 0 && int64_t(bytes) >= g_fail_above))
+  const bool chosen = g_running && g_fail_alloc && --g_fail_alloc == 0;
+  if (chosen || (g_limit && g_used + bytes > g_limit))
     fail("simulated pool: no memory for " + std::to_string(bytes) + " bytes");
   g_used += bytes;
   return std::calloc(1, bytes ? bytes : 1);

@@ -31,10 +31,10 @@ def lib():
                                          ctypes.POINTER(ctypes.c_ulonglong), ctypes.c_ulonglong]
   lib.srd_engine_destroy.argtypes = [ctypes.c_void_p]
   lib.srd_engine_set_quiet.argtypes = [ctypes.c_void_p, ctypes.c_int]
-  for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit"):
+  for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit", "sim_fail_alloc"):
     getattr(lib, f).argtypes = [ctypes.c_uint64]
-  lib.sim_fail_allocs.argtypes = [ctypes.c_int64]
-  for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations", "sim_size_after_failure"):
+  for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations", "sim_size_after_failure",
+            "sim_allocs_to_failure"):
     getattr(lib, f).restype = ctypes.c_uint64
   return lib
 
@@ -155,3 +155,58 @@ def test_a_failed_run_keeps_its_pinned_block_until_the_launches_ran(lib, engine)
   assert eng.run(e) == 0
   check(eng.path(), e)
   assert lib.sim_late_writes() == 0
+
+
+def test_no_iterations_on_bitmaps_above_the_memory_budget(lib, engine, monkeypatch):
+  monkeypatch.setenv("SRDATALOG_DEVLOOP_MAX_BYTES", str(1 << 20))
+  e = ds.tc_edges(6, 500, 900)
+  eng = engine()
+  assert eng.run(e) == 0
+  check(eng.path(), e)
+  assert lib.sim_dense_iterations() == 0
+
+
+def test_no_iterations_on_bitmaps_without_memory_for_them(lib, engine):
+  """The pool holds the relations but not the DELTA buffer of 2^20 keys."""
+  e = ds.tc_edges(6, 1000, 1500)
+  eng = engine()
+  lib.sim_pool_limit(lib.sim_pool_used() + (8 << 20))
+  assert eng.run(e) == 0
+  check(eng.path(), e)
+  assert lib.sim_dense_iterations() == 0
+  lib.sim_pool_limit(0)
+  assert eng.run(e) == 0
+  check(eng.path(), e)
+  assert lib.sim_dense_iterations() > 0
+
+
+def test_growth_above_the_memory_budget_hands_over(lib, engine, monkeypatch):
+  """DELTA of 90,000 rows and more does not fit a megabyte: the second
+  iteration and those after it run on the host loop."""
+  monkeypatch.setenv("SRDATALOG_DENSE_DELTA_ROWS", "1300")
+  monkeypatch.setenv("SRDATALOG_DEVLOOP_MAX_BYTES", str(1 << 20))
+  w, tail = 300, 12
+  s, t = np.arange(w), 300 + np.arange(w)
+  e = np.concatenate([np.stack([s, np.full(w, 900)], 1), [[900, 901]], np.stack([np.full(w, 901), t], 1),
+                      np.stack([t, np.full(w, 910)], 1),
+                      np.stack([910 + np.arange(tail), 911 + np.arange(tail)], 1)]).astype(np.uint32)
+  eng = engine()
+  assert eng.run(e) == 0
+  check(eng.path(), e)
+  assert 2 <= lib.sim_dense_iterations() <= 4    # what was sent ahead of the overflow
+
+
+@pytest.mark.parametrize("nth", [1, 2, 3])
+def test_growth_without_memory_hands_over(lib, engine, monkeypatch, nth):
+  """One buffer of the larger DELTA (columns, root values, root offsets) cannot
+  be had: the last whole DELTA goes to the host loop."""
+  monkeypatch.setenv("SRDATALOG_DENSE_DELTA_ROWS", "128")
+  e = fan(30, 20)
+  eng = engine()
+  lib.sim_fail_alloc(nth)
+  assert eng.run(e) == 0
+  assert lib.sim_allocs_to_failure() == 0
+  check(eng.path(), e)
+  assert lib.sim_dense_iterations() <= 4
+  assert eng.run(e) == 0                          # and with the memory back
+  check(eng.path(), e)
