@@ -1435,7 +1435,15 @@ static void pr_union(srd_engine& e, PipeRun& R, uint64_t iteration) {
   const uint64_t words = std::max<uint64_t>((uint64_t(1) << (2 * sh)) / 32, kDenseBlockWords);
   if (sc.uni_bits.n < words) {
     if (e.dense_bytes - sc.uni_bits.n * 4 + words * 4 > e.device_bytes / 8) return;
-    new_bitmap(e, sc.uni_bits, sc.uni_sum, words, R.s);
+    try {
+      new_bitmap(e, sc.uni_bits, sc.uni_sum, words, R.s);
+    } catch (const std::exception& ex) {
+      if (e.trace) {
+        std::fprintf(stderr, "[srd]   %s: no unions (%s)\n", R.d->rule, ex.what());
+        std::fflush(stderr);
+      }
+      return;
+    }
   }
   const uint32_t k = R.d->dest[0].arity;
   UnionProducts& u = R.uni;

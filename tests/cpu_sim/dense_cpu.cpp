@@ -68,7 +68,8 @@ std::atomic<bool> g_hold{false};         // iterations wait for the host to wait
 std::atomic<bool> g_tail{false};         // and has enqueued launches since
 std::atomic<uint64_t> g_plans{0}, g_books{0}, g_fail_book{0}, g_queries{0};
 std::atomic<uint64_t> g_limit{0}, g_used{0}, g_late_writes{0};
-std::atomic<uint64_t> g_fail_alloc{0};   // the nth allocation once iterations run fails (0: none)
+// the nth allocation fails (0: none) of those once iterations run, or of those of g_fail_bytes
+std::atomic<uint64_t> g_fail_alloc{0}, g_fail_bytes{0};
 std::atomic<bool> g_running{false};      // a run has enqueued its first iteration
 std::mutex g_pin_mu;
 std::map<const char*, uint64_t> g_pins;   // pinned blocks handed out
@@ -111,7 +112,7 @@ extern "C" void sim_reset() {
   g_dev = new Device();
   g_split_tick = g_plans = g_books = g_fail_book = g_queries = g_limit = g_late_writes = 0;
   g_half = g_drained = g_tail = g_running = g_hold = false;
-  g_fail_alloc = 0;
+  g_fail_alloc = g_fail_bytes = 0;
 }
 extern "C" void sim_split_report(uint64_t tick) { g_split_tick = tick; }
 // The device starts on what is enqueued only when the host waits for it (or
@@ -121,7 +122,7 @@ extern "C" void sim_hold() {
   g_hold = true;
 }
 extern "C" void sim_fail_book(uint64_t nth) { g_books = 0, g_fail_book = nth; }
-extern "C" void sim_fail_alloc(uint64_t nth) { g_fail_alloc = nth; }
+extern "C" void sim_fail_alloc(uint64_t nth, uint64_t bytes) { g_fail_alloc = nth, g_fail_bytes = bytes; }
 extern "C" uint64_t sim_allocs_to_failure() { return g_fail_alloc; }
 extern "C" void sim_pool_limit(uint64_t bytes) { g_limit = bytes; }
 extern "C" uint64_t sim_pool_used() { return g_used; }
@@ -142,7 +143,7 @@ extern "C" uint64_t sim_dense_iterations() { return g_plans; }
 namespace srd {
 
 void* pool_alloc(uint64_t bytes, hipStream_t) {
-  const bool chosen = g_running && g_fail_alloc && --g_fail_alloc == 0;
+  const bool chosen = (g_fail_bytes ? bytes == g_fail_bytes : g_running.load()) && g_fail_alloc && --g_fail_alloc == 0;
   if (chosen || (g_limit && g_used + bytes > g_limit))
     fail("simulated pool: no memory for " + std::to_string(bytes) + " bytes");
   g_used += bytes;
@@ -385,10 +386,11 @@ void queued(const SrdLaunchArgs* a, hipStream_t s) {
 }
 
 // TCRec_D0's device-sized launches in the bitmap loop are queued; the other
-// two rules run outside it.
+// two rules run outside it.  On the host loop it marks too.
 SrdPipelineDesc* dense_pipes() {
   static SrdPipelineDesc p[3] = {k_pipes[0], k_pipes[1], k_pipes[2]};
   p[2].root_dyn = &queued<&rec_root>;
+  p[2].mark = &rec_mark;
   return p;
 }
 
@@ -399,6 +401,14 @@ const SrdPipelineExt k_exts[] = {
 };
 
 }  // namespace
+
+// The recursive rule as one with a union pipeline.  That one is not simulated
+// (union_products fails); the rule itself marks.
+extern "C" srd_engine* cpu_union_engine(const char* program_text) {
+  static const SrdPipelineExt exts[] = {k_exts[0], k_exts[1],
+                                        {"TCRec_D0", 2, nullptr, &dense_pipes()[2], 1, 0, 0, -1, 0}};
+  return srd_engine_create_ext(program_text, dense_pipes(), 3, exts, 3);
+}
 
 extern "C" srd_engine* cpu_dense_engine(const char* program_text) {
   return srd_engine_create_ext(program_text, dense_pipes(), 3, k_exts, 3);

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 # 700 vertices: the bitmaps of 2^20 keys, the key buffers and the first DELTA
-# are 0.32 MB, above the first limit; the fourth iteration's 48,384 rows of DELTA above the second limit; the third holds everything
+# are 0.32 MB, above the first limit; the fourth iteration's 48,384 rows of
+# DELTA are above the second; the third holds everything
 @pytest.mark.parametrize("limit", [100_000, 1_000_000, 1 << 26])
 def test_closure_within_a_memory_budget(limit, monkeypatch):
   monkeypatch.setenv("SRDATALOG_DEVLOOP_MAX_BYTES", str(limit))

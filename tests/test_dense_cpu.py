@@ -19,8 +19,9 @@ _u32p = ctypes.POINTER(ctypes.c_uint32)
 @pytest.fixture(scope="module")
 def lib():
   lib = ctypes.CDLL(build_cpu_sim("libdense_cpu.so"))
-  lib.cpu_dense_engine.restype = ctypes.c_void_p
-  lib.cpu_dense_engine.argtypes = [ctypes.c_char_p]
+  for f in ("cpu_dense_engine", "cpu_union_engine"):
+    getattr(lib, f).restype = ctypes.c_void_p
+    getattr(lib, f).argtypes = [ctypes.c_char_p]
   lib.srd_engine_ok.argtypes = [ctypes.c_void_p]
   lib.srd_engine_load_rows.argtypes = [ctypes.c_void_p, ctypes.c_char_p, _u32p, ctypes.c_uint64,
                                        ctypes.c_uint32]
@@ -31,7 +32,8 @@ def lib():
                                          ctypes.POINTER(ctypes.c_ulonglong), ctypes.c_ulonglong]
   lib.srd_engine_destroy.argtypes = [ctypes.c_void_p]
   lib.srd_engine_set_quiet.argtypes = [ctypes.c_void_p, ctypes.c_int]
-  for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit", "sim_fail_alloc"):
+  lib.sim_fail_alloc.argtypes = [ctypes.c_uint64, ctypes.c_uint64]
+  for f in ("sim_split_report", "sim_fail_book", "sim_pool_limit"):
     getattr(lib, f).argtypes = [ctypes.c_uint64]
   for f in ("sim_pool_used", "sim_late_writes", "sim_dense_iterations", "sim_size_after_failure",
             "sim_allocs_to_failure"):
@@ -48,10 +50,10 @@ def plain_settings(monkeypatch, lib):
 
 
 class Engine:
-  def __init__(self, lib):
+  def __init__(self, lib, make):
     prog = programs.tc_program()
     text = codegen.program_text(compiler.relation_decls(prog), compiler.compile_to_mir(prog))
-    self.lib, self.e = lib, ctypes.c_void_p(lib.cpu_dense_engine(text.encode()))
+    self.lib, self.e = lib, ctypes.c_void_p(make(text.encode()))
     assert lib.srd_engine_ok(self.e) == 1
     lib.srd_engine_set_quiet(self.e, 1)
 
@@ -78,8 +80,8 @@ class Engine:
 def engine(lib):
   engines = []
 
-  def make():
-    engines.append(Engine(lib))
+  def make(kind=lib.cpu_dense_engine):
+    engines.append(Engine(lib, kind))
     return engines[-1]
   yield make
   for e in engines:
@@ -203,10 +205,23 @@ def test_growth_without_memory_hands_over(lib, engine, monkeypatch, nth):
   monkeypatch.setenv("SRDATALOG_DENSE_DELTA_ROWS", "128")
   e = fan(30, 20)
   eng = engine()
-  lib.sim_fail_alloc(nth)
+  lib.sim_fail_alloc(nth, 0)
   assert eng.run(e) == 0
   assert lib.sim_allocs_to_failure() == 0
   check(eng.path(), e)
   assert lib.sim_dense_iterations() <= 4
   assert eng.run(e) == 0                          # and with the memory back
   check(eng.path(), e)
+
+
+def test_a_union_without_memory_leaves_the_rule_to_mark(lib, engine, monkeypatch):
+  """Ids below 1,024: NEW's bitmap and the unions' are 128 KiB each, and the
+  second of them cannot be had in any iteration."""
+  monkeypatch.setenv("SRDATALOG_DEVLOOP", "0")
+  e = ds.tc_edges(7, 600, 900)
+  eng = engine(lib.cpu_union_engine)
+  lib.sim_fail_alloc(2, 1 << 17)
+  # one iteration: the next would find the memory
+  assert eng.run(e, 1) == 0
+  assert lib.sim_allocs_to_failure() == 0
+  check(eng.path(), e, 1)
