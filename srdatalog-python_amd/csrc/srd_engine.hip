@@ -3833,23 +3833,28 @@ int srd_engine_load_rows(srd_engine* e, const char* rel, const uint32_t* rows, u
   Relation& r = e->rels[it->second];
   if (arity != r.arity) return 2;
   return eguard(e, 3, [&] {
-    r.dev_input_valid = false;
-    r.host_n = n;
-    r.has_input = true;
-    if (n * arity >= kUploadDirect && arity <= 8) {
+    // the relation keeps the rows it has until the new ones are in hand
+    DevBuf<uint32_t> dev;
+    std::vector<uint32_t> host, maxima;
+    bool direct = n * arity >= kUploadDirect && arity <= 8;
+    if (direct) {
       // no device memory for them now: kept on the host, and the run reports it
       try {
-        r.dev_stride = round_stride(n);
-        upload_rows(rows, n, arity, r.dev_input, r.dev_stride, r.input_max, e->ws, e->s);
-        r.host_rows.clear();
-        r.host_rows.shrink_to_fit();
-        r.dev_input_valid = true;
-        return;
+        upload_rows(rows, n, arity, dev, round_stride(n), maxima, e->ws, e->s);
       } catch (const std::exception&) {
-        r.dev_input.release();
+        direct = false;
       }
     }
-    r.host_rows.assign(rows, rows + n * arity);
+    if (!direct) host.assign(rows, rows + n * arity);
+    r.host_rows.swap(host);
+    r.host_n = n;
+    r.has_input = true;
+    r.dev_input_valid = direct;
+    if (direct) {
+      r.dev_input = std::move(dev);
+      r.dev_stride = round_stride(n);
+      r.input_max.swap(maxima);
+    }
   });
 }
 

@@ -225,3 +225,15 @@ def test_a_union_without_memory_leaves_the_rule_to_mark(lib, engine, monkeypatch
   assert eng.run(e, 1) == 0
   assert lib.sim_allocs_to_failure() == 0
   check(eng.path(), e, 1)
+
+
+def test_rows_that_cannot_be_loaded_leave_the_ones_there(lib, engine):
+  """A load that neither the device nor the host has memory for."""
+  e = ds.tc_edges(8, 60, 100)
+  eng = engine()
+  assert eng.run(e) == 0
+  lib.sim_pool_limit(lib.sim_pool_used() + (1 << 20))
+  assert lib.srd_engine_load_rows(eng.e, b"ArcInput", e.ctypes.data_as(_u32p), 1 << 60, 2) != 0
+  lib.sim_pool_limit(0)
+  assert lib.srd_engine_run(eng.e, 0) == 0
+  check(eng.path(), e)
