@@ -901,14 +901,21 @@ void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>&
   if (k == 0 || k > 8) fail("upload_rows: arity must be in [1, 8]");
   maxima.assign(k, 0);
   if (n == 0) return;
+  // the rows pass through a buffer of at most 128 MiB, so that an input takes
+  // no more device memory than its columns and that
+  constexpr uint64_t kRawWords = uint64_t(32) << 20;
+  const uint64_t part = std::min<uint64_t>(n, kRawWords / k);
   out.alloc(stride * k, s);
-  DevBuf<uint32_t> raw(n * k, s), mx(8, s);
+  DevBuf<uint32_t> raw(part * k, s), mx(8, s);
   fill_u32(mx.p, 0, 8, s);
-  copy_in(reinterpret_cast<uint8_t*>(raw.p), reinterpret_cast<const uint8_t*>(rows), n * k * 4, ws, s);
-  const uint32_t g = grid_for(n, kBlock * 4, 4096);
-  if (k == 2) deinterleave_kernel<2><<<g, kBlock, 0, s>>>(raw.p, n, k, out.p, stride, mx.p);
-  else deinterleave_kernel<0><<<g, kBlock, 0, s>>>(raw.p, n, k, out.p, stride, mx.p);
-  SRD_CHECK(hipGetLastError());
+  for (uint64_t i = 0; i < n; i += part) {
+    const uint64_t m = std::min(part, n - i);
+    copy_in(reinterpret_cast<uint8_t*>(raw.p), reinterpret_cast<const uint8_t*>(rows + i * k), m * k * 4, ws, s);
+    const uint32_t g = grid_for(m, kBlock * 4, 4096);
+    if (k == 2) deinterleave_kernel<2><<<g, kBlock, 0, s>>>(raw.p, m, k, out.p + i, stride, mx.p);
+    else deinterleave_kernel<0><<<g, kBlock, 0, s>>>(raw.p, m, k, out.p + i, stride, mx.p);
+    SRD_CHECK(hipGetLastError());
+  }
   uint32_t* h = pinned_words(ws, 8);
   SRD_CHECK(hipMemcpyAsync(h, mx.p, 8 * 4, hipMemcpyDeviceToHost, s));
   SRD_CHECK(hipStreamSynchronize(s));
