@@ -556,9 +556,17 @@ static void upload_input(srd_engine& e, Relation& r) {
   const uint64_t n = r.host_n, k = r.arity;
   r.dev_stride = round_stride(n);
   if (n * k >= kUploadDirect && k <= 8) {
-    upload_rows(r.host_rows.data(), n, uint32_t(k), r.dev_input, r.dev_stride, r.input_max, e.ws, e.s);
-    r.dev_input_valid = true;
-    return;
+    try {
+      upload_rows(r.host_rows.data(), n, uint32_t(k), r.dev_input, r.dev_stride, r.input_max, e.ws, e.s);
+      r.dev_input_valid = true;
+      return;
+    } catch (const std::exception& ex) {
+      // no pinned memory, or no room for the rows on their way: split here
+      if (e.trace) {
+        std::fprintf(stderr, "[srd]   %s: columns split on the host (%s)\n", r.name.c_str(), ex.what());
+        std::fflush(stderr);
+      }
+    }
   }
   std::vector<uint32_t> t(r.dev_stride * k, 0);
   r.input_max.assign(k, 0);

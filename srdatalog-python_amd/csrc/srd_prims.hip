@@ -94,7 +94,9 @@ void* pinned_acquire(uint64_t bytes, uint64_t* got) {
   void* p = nullptr;
   {
     std::lock_guard<std::recursive_mutex> cg(capture_mutex());
-    SRD_CHECK(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+    const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipGetLastError();  // callers may do without: not the next launch's error
+    SRD_CHECK(e);
   }
   *got = bytes;
   return p;

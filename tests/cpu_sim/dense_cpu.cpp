@@ -71,6 +71,7 @@ std::atomic<uint64_t> g_limit{0}, g_used{0}, g_late_writes{0};
 // the nth allocation fails (0: none) of those once iterations run, or of those of g_fail_bytes
 std::atomic<uint64_t> g_fail_alloc{0}, g_fail_bytes{0};
 std::atomic<bool> g_running{false};      // a run has enqueued its first iteration
+std::atomic<int> g_upload_fails{0};
 std::mutex g_pin_mu;
 std::map<const char*, uint64_t> g_pins;   // pinned blocks handed out
 
@@ -113,7 +114,10 @@ extern "C" void sim_reset() {
   g_split_tick = g_plans = g_books = g_fail_book = g_queries = g_limit = g_late_writes = 0;
   g_half = g_drained = g_tail = g_running = g_hold = false;
   g_fail_alloc = g_fail_bytes = 0;
+  g_upload_fails = 0;
 }
+extern "C" int sim_upload_fails() { return g_upload_fails; }
+extern "C" void sim_set_upload_fails(int on) { g_upload_fails = on; }
 extern "C" void sim_split_report(uint64_t tick) { g_split_tick = tick; }
 // The device starts on what is enqueued only when the host waits for it (or
 // asks three times).

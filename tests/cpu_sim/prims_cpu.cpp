@@ -59,6 +59,8 @@ uint32_t* pinned_words(Workspace& ws, uint64_t words) {
   return ws.pinned;
 }
 
+extern "C" __attribute__((weak)) int sim_upload_fails();
+
 using Row = std::vector<uint32_t>;
 
 static std::vector<Row> rows_of(const Index& x) {
@@ -198,6 +200,7 @@ void export_rows(const Index& x, uint32_t* host_out, const uint32_t* bounds, uin
 
 void upload_rows(const uint32_t* rows, uint64_t n, uint32_t k, DevBuf<uint32_t>& out, uint64_t stride,
                  std::vector<uint32_t>& maxima, Workspace&, hipStream_t s) {
+  if (sim_upload_fails && sim_upload_fails()) fail("simulated upload: no pinned memory");
   maxima.assign(k, 0);
   if (n == 0) return;
   out.alloc(stride * k, s);

@@ -237,3 +237,17 @@ def test_rows_that_cannot_be_loaded_leave_the_ones_there(lib, engine):
   lib.sim_pool_limit(0)
   assert lib.srd_engine_run(eng.e, 0) == 0
   check(eng.path(), e)
+
+
+def test_rows_the_device_cannot_split_are_split_on_the_host(lib, engine, monkeypatch):
+  """Neither at the load nor at the run is there pinned memory for rows on
+  their way to the device; the columns need none."""
+  monkeypatch.setenv("SRDATALOG_DEVLOOP", "0")
+  n = 1 << 16                                     # pairs: the smallest input sent as rows
+  e = np.stack([np.arange(n), n + np.arange(n)], 1).astype(np.uint32)
+  eng = engine()
+  lib.sim_set_upload_fails(1)
+  assert eng.run(e) == 0
+  got = eng.path()
+  np.testing.assert_array_equal(got[0], e)
+  assert got[1] == [0]
