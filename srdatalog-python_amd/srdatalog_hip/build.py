@@ -69,7 +69,10 @@ def compile_jit_project(project: dict, out_path: str | None = None) -> BuildResu
   rpaths = [f"-Wl,-rpath,{lib_dir}"]
   rel = os.path.relpath(lib_dir, os.path.dirname(os.path.abspath(so)))
   rpaths.insert(0, "-Wl,-rpath,$ORIGIN/" + rel)
-  cmd = [native.hipcc(), *native.hip_flags(), "-shared", "-x", "hip", main, "-o", tmp,
+  # -Bsymbolic: a program uses its own launchers and kernels.  Programs are
+  # loaded with global symbols, and two whose rules have the same name at the
+  # same place share every generated name.
+  cmd = [native.hipcc(), *native.hip_flags(), "-shared", "-Wl,-Bsymbolic", "-x", "hip", main, "-o", tmp,
          f"-L{lib_dir}", "-lsrdatalog_hip", *rpaths]
   r = subprocess.run(cmd, capture_output=True, text=True)
   res = BuildResult(returncode=r.returncode, stderr=r.stderr, compile_results=[r])
