@@ -334,7 +334,7 @@ def split_nonrec_program() -> Program:
 def products_program() -> Program:
   """Rules that end in a product of two sources, in the forms that decide
   how the product is marked; written for this package's tests."""
-  l, r, x, y = (Var(n) for n in ("l", "r", "x", "y"))
+  l, r, x, y, z = (Var(n) for n in ("l", "r", "x", "y", "z"))
   a = Relation("A", 2, input_file="A.csv")
   b = Relation("B", 2, input_file="B.csv")
   c = Relation("C", 2, input_file="C.csv")
@@ -345,6 +345,9 @@ def products_program() -> Program:
   neg = Relation("RootNeg", 2, print_size=True)
   filt = Relation("RootFilter", 2, print_size=True)
   twice = Relation("RootTwice", 4, print_size=True)
+  key_u = Relation("KeyUnion", 3, print_size=True)
+  key_m = Relation("KeyUnionMinor", 3, print_size=True)
+  deep = Relation("Deep", 2, print_size=True)
   return Program(rules=[
     # one side does not depend on the root key
     (indep(x, y) <= a(r, x) & u(r) & s(y)).named("IndepPairs"),
@@ -354,6 +357,12 @@ def products_program() -> Program:
     (filt(x, y) <= a(r, x) & c(r, y) & Filter(("r",), "return r != 3u;")).named("RootFilter"),
     # the root variable in two columns of the head
     (twice(r, r, x, y) <= a(r, l) & b(l, x) & c(r, y)).named("RootTwice"),
+    # unions with the root variable in the head, their values in the row and
+    # in the last column
+    (key_u(r, x, y) <= a(r, l) & b(l, x) & c(r, y)).named("KeyUnion"),
+    (key_m(y, r, x) <= a(r, l) & b(l, x) & c(r, y)).named("KeyUnionMinor"),
+    # a product at the third level
+    (deep(x, y) <= a(r, l) & b(l, z) & b(z, x) & c(r, y)).named("Deep"),
   ])
 
 

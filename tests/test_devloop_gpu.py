@@ -10,7 +10,9 @@ loop abandon and re-run iterations while it grows its buffers), and
 SRDATALOG_DEVLOOP_BATCH sets how many iterations are launched between two
 reads of the control block, and SRDATALOG_DEVLOOP_MAX_BYTES and
 SRDATALOG_DEVLOOP_MAX_ROWS bound the loop's buffers and its FULL / NEW rows
-(beyond them, the loop hands its state to the host loop)."""
+(beyond them, the loop hands its state to the host loop).  These steps also
+iterate on bitmaps where nothing asks for rows: SRDATALOG_DEVLOOP_DENSE=0
+keeps the loop on rows, with its settings as they are."""
 
 import numpy as np
 import pytest
@@ -22,9 +24,10 @@ pytestmark = pytest.mark.gpu
 
 ENV_KEYS = ("SRDATALOG_DEVLOOP", "SRDATALOG_DEVLOOP_GRAPH", "SRDATALOG_DEVLOOP_CAPS",
             "SRDATALOG_DEVLOOP_BATCH", "SRDATALOG_DEVLOOP_MAX_BYTES", "SRDATALOG_DEVLOOP_MAX_ROWS",
-            "SRDATALOG_JOIN_MODE", "SRDATALOG_GRAIN")
+            "SRDATALOG_JOIN_MODE", "SRDATALOG_GRAIN", "SRDATALOG_DEVLOOP_DENSE")
 
 VARIANTS = [({}, "default"),
+            ({"SRDATALOG_DEVLOOP_DENSE": "0"}, "rows"),
             ({"SRDATALOG_DEVLOOP_GRAPH": "0"}, "eager"),
             ({"SRDATALOG_DEVLOOP_CAPS": "64"}, "tiny-caps"),
             ({"SRDATALOG_DEVLOOP_CAPS": "200", "SRDATALOG_DEVLOOP_GRAPH": "0"}, "tiny-caps-eager"),
@@ -81,10 +84,17 @@ def test_devloop_parity(env, label, monkeypatch):
       lib.shutdown()
 
 
-@pytest.mark.parametrize("max_iters", [1, 3])
-def test_devloop_max_iters(max_iters, monkeypatch):
+def bitmaps_or_rows(dense, monkeypatch):
   for k in ENV_KEYS:
     monkeypatch.delenv(k, raising=False)
+  if not dense:
+    monkeypatch.setenv("SRDATALOG_DEVLOOP_DENSE", "0")
+
+
+@pytest.mark.parametrize("dense", [True, False])
+@pytest.mark.parametrize("max_iters", [1, 3])
+def test_devloop_max_iters(max_iters, dense, monkeypatch):
+  bitmaps_or_rows(dense, monkeypatch)
   e = ds.tc_edges(0, 1000, 5000)
   orc = oracle.run("tc", {"ArcInput": e}, max_iters=max_iters)
   lib = run("tc", {"ArcInput": e}, max_iters=max_iters)
@@ -95,10 +105,10 @@ def test_devloop_max_iters(max_iters, monkeypatch):
     lib.shutdown()
 
 
-def test_devloop_repeat_runs(monkeypatch):
+@pytest.mark.parametrize("dense", [True, False])
+def test_devloop_repeat_runs(dense, monkeypatch):
   """Runs of one session reuse the resident inputs; every run starts over."""
-  for k in ENV_KEYS:
-    monkeypatch.delenv(k, raising=False)
+  bitmaps_or_rows(dense, monkeypatch)
   e = ds.tc_edges(2, 1000, 5000)
   orc = oracle.run("tc", {"ArcInput": e})
   lib = run("tc", {"ArcInput": e})

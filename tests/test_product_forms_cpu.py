@@ -33,3 +33,11 @@ def test_a_union_adds_the_root_variable_once():
   g = gens()["RootTwice"]
   assert g.union_gen() is None and g.prod_kind() == 2
   assert g.gen_ext().strip() == '{"RootTwice", 2, nullptr, nullptr, 0, 0, 0, -1, 0}'
+
+
+def test_unions_with_the_root_variable_in_the_head():
+  """uni_minor, uni_row_col, uni_root_col of SrdPipelineExt."""
+  g = gens()
+  for rule, minor, row, root in (("KeyUnion", 0, 1, 0), ("KeyUnionMinor", 1, 0, 1)):
+    assert g[rule].gen_ext().strip().endswith(f"_{rule}_union::k_desc, 1, {minor}, {row}, {root}, 0}}")
+  assert g["Deep"].prod_kind() == 3 and g["Deep"].union_gen() is None

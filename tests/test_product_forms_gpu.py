@@ -48,6 +48,12 @@ def model(i):
     "RootFilter": {(x, y) for r in a if r in c and r != 3 for x in a[r] for y in c[r]},
     "RootTwice": {(r, r, x, y) for r in a if r in c
                   for x in {v for m in a[r] for v in b.get(m, ())} for y in c[r]},
+    "KeyUnion": {(r, x, y) for r in a if r in c
+                 for x in {v for m in a[r] for v in b.get(m, ())} for y in c[r]},
+    "KeyUnionMinor": {(y, r, x) for r in a if r in c
+                      for x in {v for m in a[r] for v in b.get(m, ())} for y in c[r]},
+    "Deep": {(x, y) for r in a if r in c
+             for x in {v for m in a[r] for z in b.get(m, ()) for v in b.get(z, ())} for y in c[r]},
   }
 
 
