@@ -368,10 +368,13 @@ struct srd_engine {
   // SRDATALOG_DEVLOOP_MAX_BYTES: a loop that would reserve more hands its
   // state to the host loop (default: a quarter of the device memory)
   uint64_t devloop_max_bytes = 0;
-  // SRDATALOG_DEVLOOP_MAX_ROWS: a step whose FULL or NEW outgrows this many
-  // rows continues on the host loop.  Its iterations then run long enough
+  // SRDATALOG_DEVLOOP_MAX_ROWS: a step on rows whose FULL or NEW outgrows this
+  // many rows continues on the host loop.  Its iterations then run long enough
   // that the host loop's read-backs cost little, while growing the device
   // loop's capacities costs a re-run of the iteration and fresh buffers.
+  // Iterations on bitmaps re-run only the emission; of these, a step that
+  // begins with more rows or whose DELTA outgrows its buffer and this leaves
+  // for the host loop if one of its rules weighs nested levels.
   uint64_t devloop_max_rows = uint64_t(1) << 24;
 };
 
@@ -999,8 +1002,9 @@ static void pr_slices(srd_engine& e, PipeRun& R) {
 
 // Replace the uniform slices (grain items each) of a weighed rule by slices
 // of about equal cost: slice s is cut at the item where the cost prefix
-// crosses s/S of the total.  An item is never split, so one item's
-// candidates bound a slice's cost.
+// crosses s/S of the total.  An item is split only where its product is marked
+// row by row (mark_prod 2); elsewhere one item's candidates bound a slice's
+// cost.
 static void pr_weighed(srd_engine& e, PipeRun& R) {
   if (!R.weigh_items) return;
   PipeScratch& x = *R.x;
@@ -1472,10 +1476,6 @@ static void pr_union(srd_engine& e, PipeRun& R, uint64_t iteration) {
   R.a.mark_shift = sh;
 }
 
-// Run pipelines -- one, or the members of a parallel group -- phase by
-// phase.  A group's members each get a stream and scratch of their own (a
-// member counting probes or needing the chunked or overflow path finishes
-// on the engine's stream, after the others).
 // A rule that copies a relation column by column, in the column order of the
 // index it reads: that index, already sorted and without repeats, becomes a
 // part of NEW as it is (indexes share their columns).  Deriving the rows
@@ -1506,6 +1506,10 @@ static bool pr_copy(srd_engine& e, PipeRun& R) {
   return true;
 }
 
+// Run pipelines -- one, or the members of a parallel group -- phase by
+// phase.  A group's members each get a stream and scratch of their own (a
+// member counting probes or needing the chunked or overflow path finishes
+// on the engine's stream, after the others).
 static void run_pipelines(srd_engine& e, const std::vector<const SrdPipelineDesc*>& ds,
                           uint64_t iteration) {
   const size_t P = ds.size();
@@ -1934,8 +1938,9 @@ static void reset_state(srd_engine& e) {
 // without host read-backs: every buffer is reserved at a capacity, row
 // counts live in a device control block (DevCtl), each pipeline's launches
 // read their views and sizes from a device SrdDyn that a bind kernel fills,
-// NEW is sorted by the device-planned radix sort, and DELTA = NEW - FULL and
-// FULL u DELTA are merge-path kernels sized from device counts.  One
+// NEW is sorted by the device-planned sort (two launches up to 2^20 rows of
+// capacity, radix passes beyond), and DELTA = NEW - FULL and FULL u DELTA are
+// merge-path kernels sized from device counts.  One
 // iteration is captured into a HIP graph -- two, since FULL alternates
 // between two buffers -- and replayed; the host reads the control block
 // every few iterations.  The reference drives the same loop from the host

@@ -121,16 +121,16 @@ struct SrdLaunchArgs {
   uint8_t* mark_sum;
   uint32_t mark_shift;
   // rules whose last level is a product marked row by row (srdj::prod_mark):
-  // 1 = the root launch and the weigh mode price large products in row
-  // steps, and the mark mode walks them so
+  // SrdPipelineExt::mark_prod, the root launch and the weigh mode price large
+  // products in row steps and the mark mode walks them so (0: by tuples)
   uint32_t mark_prod;
-  // weighed mark launches of such rules: slice s covers the cost range
-  // [srd_cost_cut(s), srd_cost_cut(s+1)) of the items' cost prefix (nullptr:
-  // whole items), slice_start[s] being the item that holds its first unit; a
-  // large product is split by rows where a cut falls inside it
   // device-sized mark launches: tuples derived, summed into SRD_ROW_CTRS
   // counters SRD_ROW_CTR_STRIDE words apart (nullptr: not counted)
   unsigned long long* mark_rows;
+  // weighed mark launches of rules with mark_prod 2: slice s covers the cost
+  // range [srd_cost_cut(s), srd_cost_cut(s+1)) of the items' cost prefix
+  // (nullptr: whole items), slice_start[s] being the item that holds its first
+  // unit; a large product is split by rows where a cut falls inside it
   const uint64_t* item_pref;
   uint64_t n_items;
   uint64_t cost_q, cost_rem;
