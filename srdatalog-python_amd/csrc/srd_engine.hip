@@ -39,6 +39,7 @@
 #include <set>
 #include <memory>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "srd_devloop.h"
@@ -3027,7 +3028,7 @@ static bool run_step_dense(srd_engine& e, const Step& st, int step_no, uint64_t 
     enqueue_tail();
   };
   // The bookkeeping block of every iteration reports to pinned memory; the
-  // host stays a few iterations ahead of it and never waits for the stream.
+  // host stays a few iterations ahead of it and does not wait for the stream.
   constexpr uint64_t kAhead = 3;
   uint64_t sent = 0, tick = 0;
   bool handed = false;
@@ -3036,6 +3037,7 @@ static bool run_step_dense(srd_engine& e, const Step& st, int step_no, uint64_t 
       enqueue();
       ++sent;
     }
+    const auto asked = std::chrono::steady_clock::now();
     for (uint32_t spin = 1;; ++spin) {
       const uint64_t t = __atomic_load_n(const_cast<const uint64_t*>(&seen->tick), __ATOMIC_ACQUIRE);
       if (t != tick) {
@@ -3051,6 +3053,10 @@ static bool run_step_dense(srd_engine& e, const Step& st, int step_no, uint64_t 
           break;
         }
         if (q != hipErrorNotReady) SRD_CHECK(q);
+        // an iteration of more than a millisecond: with others already sent,
+        // the host may sleep through its end
+        if (std::chrono::steady_clock::now() - asked > std::chrono::milliseconds(1))
+          std::this_thread::sleep_for(std::chrono::microseconds(50));
       }
     }
     // The words beside the tick may already be a later block's, whose tick is
