@@ -207,7 +207,9 @@ struct SrdDyn {
 // same values again: sessions of the closure of 1,200 pairs over 400 vertices
 // run in 1.32 / 1.11 / 1.02 / 0.96 ms with 1024 / 512 / 256 / 128, of 5,000
 // pairs over 1,000 in 1.15 / 1.01 / 0.93 / 1.10, Andersen at 1/30 in 10.5 /
-// 10.4 / 10.2 / 10.6.
+// 10.4 / 10.2 / 10.6.  Long closures of sparse graphs go on gaining below it:
+// runs over 2,000 vertices and 4,000 pairs 2.42 / 1.97 / 1.71 / 1.61 ms, over
+// 6,000 and 6,300 6.85 / 5.45 / 4.53 / 4.02.
 #define SRD_PROD_GRAIN 256u
 __host__ __device__ inline uint32_t srd_grain(uint64_t total, uint32_t dflt, uint32_t least = 64u) {
   if (dflt <= least) return dflt;
